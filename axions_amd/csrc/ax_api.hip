@@ -843,7 +843,7 @@ bool use_diag_march_windings(const ax_params &p) {
 size_t diag_part_blocks(const ax_params &p) {
   const size_t V = (size_t)p.nx * p.ny * p.nz;
   const size_t site = (V + 255) / 256;
-  const size_t march = (size_t)((p.nz + 63) / 64) * p.ny * ((p.nx + kDiagXseg - 1) / kDiagXseg);
+  const size_t march = (size_t)make_tile_grid(p.nx, p.ny, p.nz, diag_xseg(p.nx, p.ny, p.nz)).work;
   return site > march ? site : march;
 }
 
@@ -861,9 +861,8 @@ int ensure_phase_buffer(ax_lattice *L) {
 hipError_t launch_march_diag(ax_lattice *L, bool phases) {
   const DiagConsts k = diag_consts(&L->p);
   float *ph = phases ? L->phase : nullptr;
-  return L->esize == 8
-             ? launch_diag_march<double>(k, levels_of<double>(L, L->timestep), kDiagXseg, ph, L->part, L->dres, L->stream)
-             : launch_diag_march<float>(k, levels_of<float>(L, L->timestep), kDiagXseg, ph, L->part, L->dres, L->stream);
+  return L->esize == 8 ? launch_diag_march<double>(k, levels_of<double>(L, L->timestep), ph, L->part, L->dres, L->stream)
+                       : launch_diag_march<float>(k, levels_of<float>(L, L->timestep), ph, L->part, L->dres, L->stream);
 }
 
 /* windings of the current level from the edge values launch_march_diag

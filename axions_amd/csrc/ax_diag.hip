@@ -772,7 +772,7 @@ hipError_t launch_diag(const DiagConsts &k, const Levels<T> &L, double *part, do
     hipLaunchKernelGGL((diag_kernel<T, AX_MODEL_AH>), dim3(nb), dim3(256), 0, st, k, L, V, part);
   } else if (getenv("AX_DIAG_SITE_KERNEL") == nullptr) {
     /* part holds 3 doubles per work item (diag_part_blocks) */
-    const TileGrid g = make_tile_grid(k.nx, k.ny, k.nz, kDiagXseg);
+    const TileGrid g = make_tile_grid(k.nx, k.ny, k.nz, diag_xseg(k.nx, k.ny, k.nz));
     hipLaunchKernelGGL((moore_diag_march_kernel<T>), dim3(g.work), dim3(64), 0, st, k, L, g, part);
     nb = g.work;
   } else {
@@ -826,7 +826,7 @@ template <typename T>
 hipError_t launch_edge_winding(int nx, int ny, int nz, const T *fr, const T *fi, const T *tx, const T *ty,
                                const T *tz, double q, float *E, int8_t *out, double *part, double *out3,
                                hipStream_t st) {
-  const TileGrid g = make_tile_grid(nx, ny, nz, kDiagXseg);
+  const TileGrid g = make_tile_grid(nx, ny, nz, diag_xseg(nx, ny, nz));
   hipLaunchKernelGGL((edge_march_kernel<T>), dim3(g.work), dim3(64), 0, st, nx, ny, nz, fr, fi, tx, ty, tz, q, g,
                      E);
   hipError_t e = hipGetLastError();
@@ -834,9 +834,9 @@ hipError_t launch_edge_winding(int nx, int ny, int nz, const T *fr, const T *fi,
 }
 
 template <typename T>
-hipError_t launch_diag_march(const DiagConsts &k, const Levels<T> &L, int xseg, float *phase, double *part,
-                             double *out3, hipStream_t st) {
-  const TileGrid g = make_tile_grid(k.nx, k.ny, k.nz, xseg);
+hipError_t launch_diag_march(const DiagConsts &k, const Levels<T> &L, float *phase, double *part, double *out3,
+                             hipStream_t st) {
+  const TileGrid g = make_tile_grid(k.nx, k.ny, k.nz, diag_xseg(k.nx, k.ny, k.nz));
   /* every divisor the P2 kernel multiplies by the reciprocal of must be a
    * power of two whose reciprocal is finite (then a*(1/d) == a/d exactly) */
   const double dx = k.dx, dy = k.dy, dz = k.dz, gg = k.g;
@@ -896,7 +896,7 @@ bool diag_pow2(double dx, double dy, double dz, double gg) {
 hipError_t launch_wind_phase(int nx, int ny, int nz, const float *E, int8_t *out, double *part, double *out3,
                              hipStream_t st) {
   /* part holds 3 doubles per work item (diag_part_blocks) */
-  const TileGrid g = make_tile_grid(nx, ny, nz, kDiagXseg);
+  const TileGrid g = make_tile_grid(nx, ny, nz, diag_xseg(nx, ny, nz));
   hipLaunchKernelGGL(wind_march_kernel, dim3(g.work), dim3(64), 0, st, nx, ny, nz, E, g, out, part);
   hipLaunchKernelGGL(sum3_kernel, dim3(1), dim3(1024), 0, st, part, g.work, out3);
   return hipGetLastError();
@@ -909,8 +909,8 @@ hipError_t launch_wind_phase(int nx, int ny, int nz, const float *E, int8_t *out
   template hipError_t launch_crossings<T>(int, int, int, double, double, double, const T *, const T *, int,   \
                                           int, int *, long long *, long long *, double *, long long,          \
                                           hipStream_t, bool);                                               \
-  template hipError_t launch_diag_march<T>(const DiagConsts &, const Levels<T> &, int, float *, double *,     \
-                                           double *, hipStream_t);                                          \
+  template hipError_t launch_diag_march<T>(const DiagConsts &, const Levels<T> &, float *, double *, double *, \
+                                           hipStream_t);                                          \
   template hipError_t launch_edge_winding<T>(int, int, int, const T *, const T *, const T *, const T *,      \
                                              const T *, double, float *, int8_t *, double *, double *,      \
                                              hipStream_t);

@@ -4,8 +4,8 @@
 #ifndef AXIONS_AX_INTERNAL_H
 #define AXIONS_AX_INTERNAL_H
 
+#include <cmath>
 #include <cstdarg>
-
 #include <cstdlib>
 
 #include "ax_device.h"
@@ -44,6 +44,24 @@ inline TileGrid make_tile_grid(int nx, int ny, int nz, int xseg) {
   g.per = (!natural && (g.nw * ny) % 8 == 0) ? g.nw * ny / 8 : 0;
   g.rows = !(o && o[0] == 'c') && ny % 8 == 0;
   return g;
+}
+
+/* x planes per wave of a march over the whole lattice, at most cap.  A wave
+ * pays a prologue worth about one plane, so long segments do the least work;
+ * but a lattice of few rows then fills few of the chip's 1024 SIMDs, and
+ * the launch ends with a tail that lasts as long as one segment.  With W
+ * (64-site rows) x (planes) per SIMD, work W (1 + c / xseg) plus a tail of
+ * xseg planes is least near xseg = sqrt(W), which is what the sweeps show
+ * (AH FP64 step, us per step with 32 planes / with this rule / best of 1 ...
+ * 32: 32^3 68 / 6.6 / 6.6, 64^3 64 / 12.6 / 12.6, 101^3 87 / 50 / 50, 128^3
+ * 74 / 66 / 63, 160^3 150 / 136 / 135, 192^3 223 / 202 / 201, 256^3 475 /
+ * 477 / 475).  The length is then evened out over the segments. */
+inline int tile_xseg(int nx, int ny, int nz, int cap) {
+  const double w = (double)((nz + 63) / 64) * ny * nx / 1024.0;
+  const double x = std::sqrt(w) + 0.5;
+  const int xs = x >= cap ? cap : x < 1 ? 1 : (int)x;
+  const int nseg = (nx + xs - 1) / xs;
+  return (nx + nseg - 1) / nseg;
 }
 
 /* (z chunk, y row, x segment) of work item w in the order make_tile_grid chose */
@@ -127,13 +145,18 @@ hipError_t launch_diag(const DiagConsts &k, const Levels<T> &L, double *part, do
  * FP32 edge values [3][V] (forward edge phase + link angle, ax_wind.h);
  * launch_wind_phase turns them into windings (the field into out when
  * out != NULL, the counts into out3) */
-constexpr int kDiagXseg = 32;
+/* x planes per wave of the diagnostics and winding marches (us per
+ * ax_diagnostics call without / with windings; this rule against the best of
+ * 1 ... 32 planes: 64^3 27.5 / 41.8 against 27.4 / 41.7, 101^3 56.7 / 99
+ * against 55.9 / 97, 160^3 125 / 244 against 125 / 244; with 32 planes at
+ * 101^3 the energy march alone took 84, with this rule 35) */
+inline int diag_xseg(int nx, int ny, int nz) { return tile_xseg(nx, ny, nz, 32); }
 bool use_diag_march(const ax_params &p);
 bool use_diag_march_windings(const ax_params &p);
 size_t diag_part_blocks(const ax_params &p);
 template <typename T>
-hipError_t launch_diag_march(const DiagConsts &k, const Levels<T> &L, int xseg, float *phase, double *part,
-                             double *out3, hipStream_t st);
+hipError_t launch_diag_march(const DiagConsts &k, const Levels<T> &L, float *phase, double *part, double *out3,
+                             hipStream_t st);
 hipError_t launch_wind_phase(int nx, int ny, int nz, const float *E, int8_t *out, double *part, double *out3,
                              hipStream_t st);
 /* periodic lattices: the FP32 edge values of field (fr, fi) of charge q into

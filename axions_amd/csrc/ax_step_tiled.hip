@@ -118,15 +118,20 @@ bool use_tiled_ah(const ax_params &p) {
          getenv("AX_FORCE_SITE_KERNEL") == nullptr;
 }
 
-/* x planes per wave (measured at 512^3 AH, 256^3 Moore, on one box each):
+/* x planes per wave: tile_xseg's rule, up to the length that is best on
+ * large lattices (measured at 512^3 AH, 256^3 Moore, on one box each):
  * Abelian-Higgs FP64 32 (3.875 ms; 8: 3.95, 16: 3.90, 24: 3.88), FP32 16
  * (1.816 ms; 8: 1.834, 12: 1.823, 32: 1.826); Moore FP64 16 (0.963 ms; 4:
- * 0.993, 8: 0.979, 32: 0.974), FP32 8 (0.422 ms; 32: 0.444) */
+ * 0.993, 8: 0.979, 32: 0.974), FP32 8 (0.422 ms; 32: 0.444).  Moore FP32 has
+ * the cheapest prologue against a plane and takes half the rule's length
+ * (128^3: 8 planes 72 us, 6 65, 3 60; 160^3: 8 135, 4 118). */
 int default_xseg(const ax_params &p) {
   const char *xe = getenv("AX_TILED_XSEG");
   if (xe) return atoi(xe);
-  if (p.model == AX_MODEL_MOORE) return p.precision == 32 ? 8 : 16;
-  return p.precision == 32 ? 16 : 32;
+  const bool f32 = p.precision == 32;
+  if (p.model != AX_MODEL_MOORE) return tile_xseg(p.nx, p.ny, p.nz, f32 ? 16 : 32);
+  const int xs = tile_xseg(p.nx, p.ny, p.nz, 16);
+  return f32 ? (xs + 1) / 2 : xs;
 }
 
 /* The LDS prefetch of the FP64 march applies: whole 64-site chunks, three
