@@ -762,7 +762,7 @@ int ax_winding_field(ax_lattice *L, int32_t field, int8_t *out, size_t n) {
 int ax_crossings(ax_lattice *L, double *xyz, size_t cap, size_t *count) {
   if (!L || !count || (cap && !xyz)) return fail(AX_EINVAL, "NULL argument");
   const ax_params &p = L->p;
-  const size_t nb = (L->V + 255) / 256;
+  const size_t nb = cross_groups(L->V);
   hipError_t e = hipSuccess;
   if (!L->bcount) {
     if (hipMalloc((void **)&L->bcount, nb * sizeof(int)) != hipSuccess ||

@@ -10,20 +10,23 @@
  *  winding_kernel   per-plaquette winding numbers (no reference
  *                   counterpart) and their absolute sum.
  *  crossing kernels the bilinear face-crossing test of
- *                   mpi_evolution.cpp:536-789, compacted in site order.
+ *                   mpi_evolution.cpp:536-789, in FP32 with an error bound
+ *                   first, in FP64 where it is needed, compacted in site
+ *                   order.
  *
  * The diagnostics must read the current level of every neighbour and the
  * previous level (the Gauss law needs the neighbours' previous level,
  * evolution.cpp:390-391), so they run as a separate pass before the in-place
  * update of the same TimeStep.
  */
+#include <algorithm>
+
 #include "ax_energy.h"
 #include "ax_internal.h"
 #include "ax_march.h"
 #include "ax_wind.h"
 
 namespace ax {
-
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -267,12 +270,103 @@ __global__ void __launch_bounds__(256) winding_kernel(int nx, int ny, int nz, co
 }
 
 
-/* ------------------------------ crossings ------------------------------- */
-/* Solve the face of mpi_evolution.cpp:552-623; returns the number of roots
- * inside the face (0..2) and writes them as (sol1, sol2) pairs. */
+/* ------------------------------ crossings -------------------------------
+ * The face equations of mpi_evolution.cpp:552-623 cost some 280 instructions
+ * with six divisions and a root in FP64, for three faces a site.  Most faces
+ * are settled without them: face_class solves the face in FP32 in its own
+ * coordinates, with a bound on how far that may lie from the FP64 solution,
+ * and tells how many roots FP64 finds or that it cannot tell.  A wave takes
+ * a group of consecutive sites; what needs FP64 (the count: the undecided
+ * faces; the points: every face with a root) goes through a queue in LDS, in
+ * site and face order, and is solved 64 at a time with every lane at work.
+ * The points of a round are put in order with two ballots and stored through
+ * LDS as one contiguous run.  Two launches (counts, then points at their
+ * offsets) with a scan in between.  512^3 FP64, 1.2 points a site: counts
+ * 2.67 -> 1.56 ms, scan 0.92 -> 0.15, points 6.96 -> 2.94 (3.9 GB written);
+ * FP32 2.63 -> 1.45, 0.92 -> 0.15, 6.29 -> 2.72.  Bound by instructions. */
+
+/* n / d for n < 2^31 and d >= 2 by a multiplication: m = floor(2^(31+s)/d) + 1
+ * with 2^(s-1) < d <= 2^s exceeds 2^(31+s)/d by less than 2^s/d <= 2, so the
+ * quotient's error stays below 1/d */
+struct FastDiv {
+  uint32_t d, m, s;
+};
+static FastDiv fast_div(uint32_t d) {
+  uint32_t s = 1;
+  while (((uint64_t)1 << s) < d) ++s;
+  return {d, (uint32_t)(((uint64_t)1 << (31 + s)) / d + 1), s - 1};
+}
+__device__ __forceinline__ uint32_t quotient(uint32_t n, const FastDiv &f) { return __umulhi(n, f.m) >> f.s; }
+
+struct CrossGeom {
+  int nx, ny, nz, ex, ez, x0, y0, z0;
+  uint32_t V, sites, groups, per;   /* sites; sites of a group (a multiple of 64); groups; groups per XCD */
+  FastDiv by_nz, by_ny;
+  double dx, dy, dz;
+  float k;                          /* face_class's relative error bound; >= 1: solve every face in FP64 */
+};
+
+/* How many roots face_roots finds on the face with corners v.. of Re phi
+ * and Im phi: 0, 1 or 2, or 3 if FP32 cannot tell.
+ *
+ * In coordinates p, q in [0, 1] of the face, phi_c = A + B p + C q + D p q;
+ * the roots have a q^2 + b q + c = 0 and p = -(A0 + C0 q)/(B0 + D0 q), which
+ * are face_roots' equations scaled and shifted.  With S the product of the
+ * two largest |phi_c| of the corners, FP32 leaves a, b and c off by at most
+ * about 2^-18 S.  face_roots works in lattice coordinates: with h the
+ * largest coordinate in spacings and e = 2^-53, its rounding acts like errors
+ * of up to some 2^8 e h^3 S in these coefficients.  The launcher takes k =
+ * max(2^-16, 2^10 e h^3), above both; k S is followed through the
+ * discriminant, q and p, and a value within its bound of a decision (or
+ * not finite, or out of FP32's middle range) is left undecided, some 1e-4
+ * of the faces.
+ *
+ * Re phi of one sign settles a face by itself: a point is kept only where
+ * p = -(A0 + C0 q)/(B0 + D0 q) lies on it, that is where Re phi, a mean of
+ * the corners there, vanishes within rounding. */
+__device__ __forceinline__ bool one_sign(float a, float b, float c, float d, float k) {
+  const float lo = fminf(fminf(a, b), fminf(c, d)), hi = fmaxf(fmaxf(a, b), fmaxf(c, d));
+  return (lo > 1e-6f && lo > k * hi && hi < 1e6f) || (hi < -1e-6f && hi < k * lo && lo > -1e6f);
+}
+__device__ __forceinline__ int face_class(float r00, float r10, float r01, float r11, float i00, float i10, float i01,
+                                          float i11, float k) {
+  const float m0 = fmaxf(fmaxf(fabsf(r00), fabsf(r10)), fmaxf(fabsf(r01), fabsf(r11)));
+  const float m1 = fmaxf(fmaxf(fabsf(i00), fabsf(i10)), fmaxf(fabsf(i01), fabsf(i11)));
+  const float B0 = r10 - r00, C0 = r01 - r00, D0 = (r11 - r10) - C0;
+  const float B1 = i10 - i00, C1 = i01 - i00, D1 = (i11 - i10) - C1;
+  const float a = D1 * C0 - D0 * C1;
+  const float b = (D1 * r00 - D0 * i00) + (B1 * C0 - B0 * C1);
+  const float c = B1 * r00 - B0 * i00;
+  const float E = k * (m0 * m1);
+  const float disc = b * b - 4 * (a * c);
+  const float F = E * (4 * fabsf(b) + 8 * (fabsf(a) + fabsf(c)) + 16 * E);
+  /* not finite makes disc + F NaN or infinite and the tests below fail */
+  const bool sane = m0 > 1e-6f && m1 > 1e-6f && m0 < 1e6f && m1 < 1e6f && fabsf(disc) < 1e30f && k < 1;
+  if (sane && disc < -F) return 0;
+  if (!(sane && disc > 2 * F && fabsf(a) > 16 * E)) return 3;
+  const float root = __builtin_amdgcn_sqrtf(disc), inv = __builtin_amdgcn_rcpf(2 * a);
+  const float eq = (3 * E + F * __builtin_amdgcn_rcpf(root)) * fabsf(2 * inv) * 1.01f + 1e-5f;
+  const float en = m0 * (2 * k + 2 * eq), ed = 2 * en;
+  int n = 0;
+  bool sure = true;
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const float q = ((s ? -root : root) - b) * inv;
+    const float num = -(r00 + C0 * q), den = B0 + D0 * q;
+    const float t0 = den < 0 ? -num : num, t1 = fabsf(den) - t0;
+    const bool in = q > eq && q < 1 - eq && t0 > en && t1 > en + ed;
+    const bool out = q < -eq || q > 1 + eq || (fabsf(den) > ed && (t0 < -en || t1 < -(en + ed)));
+    n += in ? 1 : 0;
+    sure = sure && (in || out);
+  }
+  return sure ? n : 3;
+}
+
+/* Solve the face of mpi_evolution.cpp:552-623: its roots inside the face
+ * (0..2), the + root before the - root. */
 __device__ __forceinline__ int face_roots(const double v00[2], const double v10[2], const double v01[2],
                                           const double v11[2], double u, double du, double w, double dw,
-                                          double r[4]) {
+                                          double &r1, double &r2, double &q1, double &q2) {
   double c1[2], c2[2], c3[2], c4[2];
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
@@ -281,132 +375,208 @@ __device__ __forceinline__ int face_roots(const double v00[2], const double v10[
     c3[c] = (u + du) * (v01[c] - v00[c]) + u * (v10[c] - v11[c]);
     c4[c] = (u + du) * ((w + dw) * v00[c] - w * v01[c]) - u * ((w + dw) * v10[c] - w * v11[c]);
   }
-  double a = c1[1] * c3[0] - c1[0] * c3[1];
-  double b = c1[1] * c4[0] + c2[1] * c3[0] - c1[0] * c4[1] - c2[0] * c3[1];
-  double c = c2[1] * c4[0] - c2[0] * c4[1];
-  double disc = b * b - 4 * a * c;
+  const double a = c1[1] * c3[0] - c1[0] * c3[1];
+  const double b = c1[1] * c4[0] + c2[1] * c3[0] - c1[0] * c4[1] - c2[0] * c3[1];
+  const double c = c2[1] * c4[0] - c2[0] * c4[1];
+  const double disc = b * b - 4 * a * c;
+  auto inside = [&](double s2, double &s1) {
+    s1 = 0;
+    if (!(s2 >= w && s2 <= w + dw)) return false;
+    s1 = -(c3[0] * s2 + c4[0]) / (c1[0] * s2 + c2[0]);
+    return s1 >= u && s1 <= u + du;
+  };
   int n = 0;
   if (a == 0) {
     if (b != 0) {
-      double s2 = -c / b;
-      if (s2 >= w && s2 <= w + dw) {
-        double s1 = -(c3[0] * s2 + c4[0]) / (c1[0] * s2 + c2[0]);
-        if (s1 >= u && s1 <= u + du) { r[0] = s1; r[1] = s2; n = 1; }
-      }
+      r2 = -c / b;
+      n = inside(r2, r1) ? 1 : 0;
     }
   } else if (disc >= 0) {
-    double s2 = (-b + sqrt(disc)) / (2 * a);
-    if (s2 >= w && s2 <= w + dw) {
-      double s1 = -(c3[0] * s2 + c4[0]) / (c1[0] * s2 + c2[0]);
-      if (s1 >= u && s1 <= u + du) { r[2 * n] = s1; r[2 * n + 1] = s2; ++n; }
+    const double root = sqrt(disc);
+    double s1, s2 = (-b + root) / (2 * a);
+    if (inside(s2, s1)) {
+      r1 = s1;
+      r2 = s2;
+      n = 1;
     }
-    s2 = (-b - sqrt(disc)) / (2 * a);
-    if (s2 >= w && s2 <= w + dw) {
-      double s1 = -(c3[0] * s2 + c4[0]) / (c1[0] * s2 + c2[0]);
-      if (s1 >= u && s1 <= u + du) { r[2 * n] = s1; r[2 * n + 1] = s2; ++n; }
+    s2 = (-b - root) / (2 * a);
+    if (inside(s2, s1)) {
+      if (n) {
+        q1 = s1;
+        q2 = s2;
+      } else {
+        r1 = s1;
+        r2 = s2;
+      }
+      ++n;
     }
   }
   return n;
 }
 
-/* All crossings of site s, in the reference's order; returns count (<= 6). */
-template <typename T>
-__device__ int site_crossings(int nx, int ny, int nz, double dx, double dy, double dz, const T *fr, const T *fi,
-                              int ex, int ez, int s, double pts[18]) {
-  const int kk = s % nz, r = s / nz, j = r % ny, i = r / ny;
-  /* only the sites the bulk update covers (evolution.cpp:731-743) */
-  if ((ex && (i == 0 || i == nx - 1 || j == 0 || j == ny - 1)) || (ez && (kk == 0 || kk == nz - 1))) return 0;
-  const int ip = wrapp(i, nx), jp = wrapp(j, ny), kp = wrapp(kk, nz);
-  auto id = [&](int a, int b, int c) { return (a * ny + b) * nz + c; };
-  const int sx = id(ip, j, kk), sy = id(i, jp, kk), sz = id(i, j, kp);
-  const int sxy = id(ip, jp, kk), sxz = id(ip, j, kp), syz = id(i, jp, kp);
-  const int x0 = int(0.5 * (nx - 1)), y0 = int(0.5 * (ny - 1)), z0 = int(0.5 * (nz - 1));
-  const double x = (i - x0) * dx, y = (j - y0) * dy, z = (kk - z0) * dz;
-  const double v[2] = {ld(fr, s), ld(fi, s)}, vx[2] = {ld(fr, sx), ld(fi, sx)};
-  const double vy[2] = {ld(fr, sy), ld(fi, sy)}, vz[2] = {ld(fr, sz), ld(fi, sz)};
-  const double vxy[2] = {ld(fr, sxy), ld(fi, sxy)}, vxz[2] = {ld(fr, sxz), ld(fi, sxz)};
-  const double vyz[2] = {ld(fr, syz), ld(fi, syz)};
-  double rr[4];
-  int n = 0;
-  int m = face_roots(v, vx, vy, vxy, x, dx, y, dy, rr);
-  for (int q = 0; q < m; ++q) { pts[3 * n] = rr[2 * q]; pts[3 * n + 1] = rr[2 * q + 1]; pts[3 * n + 2] = z; ++n; }
-  m = face_roots(v, vx, vz, vxz, x, dx, z, dz, rr);
-  for (int q = 0; q < m; ++q) { pts[3 * n] = rr[2 * q]; pts[3 * n + 1] = y; pts[3 * n + 2] = rr[2 * q + 1]; ++n; }
-  m = face_roots(v, vy, vz, vyz, y, dy, z, dz, rr);
-  for (int q = 0; q < m; ++q) { pts[3 * n] = x; pts[3 * n + 1] = rr[2 * q]; pts[3 * n + 2] = rr[2 * q + 1]; ++n; }
-  return n;
-}
+/* WRITE: the points of each group from its offset on; else its count. */
+template <typename T, bool WRITE>
+__global__ void __launch_bounds__(64) cross_kernel(CrossGeom g, const T *__restrict__ fr, const T *__restrict__ fi,
+                                                   int *__restrict__ count, const long long *__restrict__ offset,
+                                                   double *__restrict__ xyz, long long cap) {
+  /* consecutive groups on one XCD, so that rows y + 1 are read from its L2 */
+  const uint32_t grp = (blockIdx.x & 7) * g.per + (blockIdx.x >> 3);
+  if (grp >= g.groups) return;
+  /* queue: site in the group, face; at most 63 left over + 192 of a chunk */
+  __shared__ uint16_t queue[256];
+  __shared__ double stage[WRITE ? 384 : 1];
+  const int lane = (int)threadIdx.x;
+  const uint64_t below = ((uint64_t)1 << lane) - 1;
+  const uint32_t base = grp * g.sites;
+  const int nx = g.nx, ny = g.ny, nz = g.nz;
+  auto id = [&](int i, int j, int k) { return (uint32_t)((i * ny + j) * nz + k); };
+  uint32_t head = 0, tail = 0;   /* of the queue (mod 256) */
+  long long out = WRITE ? offset[grp] : 0;
+  int own = 0;                   /* roots counted by this lane */
 
-/* pass 1: per-block crossing counts */
-template <typename T>
-__global__ void __launch_bounds__(256) cross_count_kernel(int nx, int ny, int nz, double dx, double dy, double dz,
-                                                          const T *fr, const T *fi, int ex, int ez, int *bcount) {
-  __shared__ int sh[4];
-  const int V = nx * ny * nz;
-  const int s = blockIdx.x * 256 + threadIdx.x;
-  int n = 0;
-  if (s < V) {
-    double pts[18];
-    n = site_crossings<T>(nx, ny, nz, dx, dy, dz, fr, fi, ex, ez, s, pts);
-  }
+  auto solve = [&](uint32_t n) {
+    int m = 0;
+    double r1 = 0, r2 = 0, q1 = 0, q2 = 0, third = 0;
+    int face = 0;
+    if ((uint32_t)lane < n) {
+      const uint32_t e = queue[(head + lane) & 255];
+      face = (int)(e & 3);
+      const uint32_t s = base + (e >> 2);
+      const uint32_t r = quotient(s, g.by_nz), i = quotient(r, g.by_ny);
+      const int k = (int)(s - r * nz), j = (int)(r - i * ny);
+      const int ip = wrapp((int)i, nx), jp = wrapp(j, ny), kp = wrapp(k, nz);
+      /* the face spans axes a < b: xy, xz, yz */
+      const int ia = face == 2 ? (int)i : ip, ja = face == 2 ? jp : j;
+      const int jb = face == 0 ? jp : j, kb = face == 0 ? k : kp;
+      const uint32_t sa = id(ia, ja, k), sb = id((int)i, jb, kb), sab = id(ia, face == 1 ? j : jp, kb);
+      const double x = ((int)i - g.x0) * g.dx, y = (j - g.y0) * g.dy, z = (k - g.z0) * g.dz;
+      const double v[2] = {ld(fr, s), ld(fi, s)}, va[2] = {ld(fr, sa), ld(fi, sa)};
+      const double vb[2] = {ld(fr, sb), ld(fi, sb)}, vab[2] = {ld(fr, sab), ld(fi, sab)};
+      third = face == 0 ? z : face == 1 ? y : x;
+      m = face_roots(v, va, vb, vab, face == 2 ? y : x, face == 2 ? g.dy : g.dx, face == 0 ? y : z,
+                     face == 0 ? g.dy : g.dz, r1, r2, q1, q2);
+    }
+    const uint64_t one = __builtin_amdgcn_ballot_w64(m >= 1), two = __builtin_amdgcn_ballot_w64(m == 2);
+    const int tot = __popcll(one) + __popcll(two);
+    if (WRITE && tot) {
+      auto put = [&](int at, double s1, double s2) {
+        stage[3 * at] = face == 2 ? third : s1;
+        stage[3 * at + 1] = face == 0 ? s2 : face == 1 ? third : s1;
+        stage[3 * at + 2] = face == 0 ? third : s2;
+      };
+      const int at = __popcll(one & below) + __popcll(two & below);
+      if (m >= 1) put(at, r1, r2);
+      if (m == 2) put(at + 1, q1, q2);
+      __syncthreads();
+      /* beyond the caller's capacity only the count goes on */
+      const int fit = (int)min((long long)tot, max(cap - out, 0ll));
+      for (int d = lane; d < 3 * fit; d += 64) xyz[3 * out + d] = stage[d];
+      __syncthreads();
+    }
+    out += tot;
+    head += n;
+  };
+
+  for (uint32_t c = 0; c < g.sites; c += 64) {
+    if (base + c >= g.V) break;
+    const uint32_t s = min(base + c + lane, g.V - 1);
+    const uint32_t r = quotient(s, g.by_nz), i = quotient(r, g.by_ny);
+    const int k = (int)(s - r * nz), j = (int)(r - i * ny);
+    /* only the sites the bulk update covers (evolution.cpp:731-743) */
+    const bool bulk = base + c + lane < g.V &&
+                      !((g.ex && ((int)i == 0 || (int)i == nx - 1 || j == 0 || j == ny - 1)) ||
+                        (g.ez && (k == 0 || k == nz - 1)));
+    const int ip = wrapp((int)i, nx), jp = wrapp(j, ny), kp = wrapp(k, nz);
+    const uint32_t at7[7] = {s, id(ip, j, k), id((int)i, jp, k), id((int)i, j, kp), id(ip, jp, k), id(ip, j, kp),
+                             id((int)i, jp, kp)};
+    float re[7], im[7];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = n;
-  __syncthreads();
-  if (threadIdx.x == 0) bcount[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
-}
-
-/* pass 2: exclusive scan of the block counts (one block). */
-__global__ void __launch_bounds__(1024) scan_kernel(const int *in, long long *out, int n, long long *total) {
-  __shared__ long long sh[1024];
-  const int t = threadIdx.x;
-  const int per = (n + 1023) / 1024;
-  const int b0 = t * per, b1 = min(n, b0 + per);
-  long long loc = 0;
-  for (int i = b0; i < b1; ++i) loc += in[i];
-  sh[t] = loc;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    long long v = (t >= off) ? sh[t - off] : 0;
-    __syncthreads();
-    sh[t] += v;
-    __syncthreads();
-  }
-  long long run = sh[t] - loc;
-  for (int i = b0; i < b1; ++i) {
-    out[i] = run;
-    run += in[i];
-  }
-  if (t == 1023) *total = sh[1023];
-}
-
-/* pass 3: recompute and write points at their global offsets. */
-template <typename T>
-__global__ void __launch_bounds__(256) cross_write_kernel(int nx, int ny, int nz, double dx, double dy, double dz,
-                                                          const T *fr, const T *fi, int ex, int ez,
-                                                          const long long *boff, double *xyz, long long cap) {
-  __shared__ int sh[256];
-  const int V = nx * ny * nz;
-  const int s = blockIdx.x * 256 + threadIdx.x;
-  double pts[18];
-  int n = 0;
-  if (s < V) n = site_crossings<T>(nx, ny, nz, dx, dy, dz, fr, fi, ex, ez, s, pts);
-  sh[threadIdx.x] = n;
-  __syncthreads();
-  for (int off = 1; off < 256; off <<= 1) {
-    int v = ((int)threadIdx.x >= off) ? sh[threadIdx.x - off] : 0;
-    __syncthreads();
-    sh[threadIdx.x] += v;
-    __syncthreads();
-  }
-  long long o = boff[blockIdx.x] + sh[threadIdx.x] - n;
-  for (int q = 0; q < n; ++q, ++o) {
-    if (o < cap) {
-      xyz[3 * o] = pts[3 * q];
-      xyz[3 * o + 1] = pts[3 * q + 1];
-      xyz[3 * o + 2] = pts[3 * q + 2];
+    for (int q = 0; q < 7; ++q) re[q] = (float)fr[at7[q]];
+#pragma unroll
+    for (int q = 0; q < 7; ++q) im[q] = (float)fi[at7[q]];
+    uint64_t mask[3];   /* lanes whose xy, xz, yz face goes to the queue */
+#pragma unroll
+    for (int f = 0; f < 3; ++f) {
+      const int a = f == 2 ? 2 : 1, b = f == 0 ? 2 : 3, ab = 4 + f;
+      int n = 0;
+      const bool open = bulk && !one_sign(re[0], re[a], re[b], re[ab], g.k);
+      if (__builtin_amdgcn_ballot_w64(open) && open)
+        n = face_class(re[0], re[a], re[b], re[ab], im[0], im[a], im[b], im[ab], g.k);
+      if (!WRITE) own += n == 3 ? 0 : n;
+      mask[f] = __builtin_amdgcn_ballot_w64(WRITE ? n != 0 : n == 3);
     }
+    uint32_t at = tail;
+#pragma unroll
+    for (int f = 0; f < 3; ++f) at += __popcll(mask[f] & below);
+#pragma unroll
+    for (int f = 0; f < 3; ++f)
+      if ((mask[f] >> lane) & 1) queue[at++ & 255] = (uint16_t)((c + lane) << 2 | f);
+#pragma unroll
+    for (int f = 0; f < 3; ++f) tail += __popcll(mask[f]);
+    __syncthreads();
+    while (tail - head >= 64) solve(64);
   }
+  if (tail != head) solve(tail - head);
+  if (!WRITE) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) own += __shfl_xor(own, off, 64);
+    if (lane == 0) count[grp] = own + (int)out;
+  }
+}
+
+/* Exclusive scan of n counts by one workgroup, 8192 a round, the next
+ * round's counts loaded ahead (262 144 counts, 512^3: 0.15 ms; one count at a
+ * time per thread it was 0.92 ms). */
+__global__ void __launch_bounds__(1024) scan_kernel(const int *__restrict__ in, long long *__restrict__ out, int n,
+                                                    long long *total) {
+  __shared__ int sums[16];
+  const int t = (int)threadIdx.x, lane = t & 63, w = t >> 6;
+  auto load = [&](int b, int v[8]) {
+    const int i = b + 8 * t;
+    if (i + 8 <= n) {
+      const int4 lo = *(const int4 *)(in + i), hi = *(const int4 *)(in + i + 4);
+      v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w;
+      v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] = i + q < n ? in[i + q] : 0;
+    }
+  };
+  int v[8], next[8];
+  load(0, v);
+  long long carry = 0;
+  for (int b = 0; b < n; b += 8192) {
+    if (b + 8192 < n) load(b + 8192, next);
+    int own = 0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) own += v[q];
+    int inc = own;   /* a round's counts sum to below 2^25 */
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(inc, off, 64);
+      if (lane >= off) inc += o;
+    }
+    if (lane == 63) sums[w] = inc;
+    __syncthreads();
+    int before = 0, all = 0;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      if (q < w) before += sums[q];
+      all += sums[q];
+    }
+    long long run = carry + before + inc - own;
+    const int i = b + 8 * t;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      if (i + q < n) out[i + q] = run;
+      run += v[q];
+    }
+    carry += all;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = next[q];
+  }
+  if (t == 0) *total = carry;
 }
 
 /* ------------------- marching diagnostics (Abelian-Higgs) -----------------
@@ -798,14 +968,25 @@ template <typename T>
 hipError_t launch_crossings(int nx, int ny, int nz, double dx, double dy, double dz, const T *fr, const T *fi,
                             int ex, int ez, int *bcount, long long *boff, long long *total, double *xyz,
                             long long cap, hipStream_t st, bool write) {
-  const int V = nx * ny * nz;
-  const int nb = (V + 255) / 256;
-  hipLaunchKernelGGL((cross_count_kernel<T>), dim3(nb), dim3(256), 0, st, nx, ny, nz, dx, dy, dz, fr, fi, ex, ez,
-                     bcount);
-  hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, st, bcount, boff, nb, total);
-  if (write)
-    hipLaunchKernelGGL((cross_write_kernel<T>), dim3(nb), dim3(256), 0, st, nx, ny, nz, dx, dy, dz, fr, fi,
-                       ex, ez, boff, xyz, cap);
+  CrossGeom g;
+  g.nx = nx; g.ny = ny; g.nz = nz; g.ex = ex; g.ez = ez;
+  g.x0 = int(0.5 * (nx - 1)); g.y0 = int(0.5 * (ny - 1)); g.z0 = int(0.5 * (nz - 1));
+  g.V = (uint32_t)nx * ny * nz;
+  g.sites = cross_sites(g.V);
+  g.groups = (uint32_t)cross_groups(g.V);
+  g.per = (g.groups + 7) / 8;
+  g.by_nz = fast_div((uint32_t)nz);
+  g.by_ny = fast_div((uint32_t)ny);
+  g.dx = dx; g.dy = dy; g.dz = dz;
+  /* face_class's bound, h = n/2 + 2 spacings; where it would decide little,
+   * every face is solved */
+  const double h = 0.5 * std::max(nx, std::max(ny, nz)) + 2;
+  const double k = std::max(0x1p-16, 0x1p-43 * h * h * h);
+  g.k = k < 0x1p-8 ? (float)k : 2.0f;
+  const dim3 grid(8 * g.per), block(64);
+  hipLaunchKernelGGL((cross_kernel<T, false>), grid, block, 0, st, g, fr, fi, bcount, boff, xyz, cap);
+  hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, st, bcount, boff, (int)g.groups, total);
+  if (write) hipLaunchKernelGGL((cross_kernel<T, true>), grid, block, 0, st, g, fr, fi, bcount, boff, xyz, cap);
   return hipGetLastError();
 }
 

@@ -168,6 +168,16 @@ hipError_t launch_edge_winding(int nx, int ny, int nz, const T *fr, const T *fi,
 template <typename T>
 hipError_t launch_winding(int nx, int ny, int nz, const T *fr, const T *fi, const T *tx, const T *ty, const T *tz,
                           double q, int ex, int ez, int8_t *out, double *part, double *out3, hipStream_t st);
+/* Crossings: sites of one wave's group (a multiple of 64), and the groups of
+ * a lattice, which is how many counts (bcount) and offsets (boff)
+ * launch_crossings uses.  512 sites a group, fewer where that would leave
+ * the chip short of waves (8192 resident); at most max(2^14, V / 512 + 1)
+ * groups. */
+inline uint32_t cross_sites(size_t V) {
+  const size_t s = V / 8192 / 64 * 64;
+  return (uint32_t)(s < 64 ? 64 : s > 512 ? 512 : s);
+}
+inline size_t cross_groups(size_t V) { return (V + cross_sites(V) - 1) / cross_sites(V); }
 template <typename T>
 hipError_t launch_crossings(int nx, int ny, int nz, double dx, double dy, double dz, const T *fr, const T *fi,
                             int ex, int ez, int *bcount, long long *boff, long long *total, double *xyz,

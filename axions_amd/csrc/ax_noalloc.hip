@@ -3,7 +3,7 @@
  * ax_crossings (mpi_evolution.cpp:536-789) for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops).
  *
- * ax_crossings allocates its per-block counts and offsets and its point
+ * ax_crossings allocates its per-group counts and offsets and its point
  * buffer on first use (and the point buffer again whenever the capacity
  * grows).  Here the points go straight into a device buffer the caller owns,
  * and the counts and offsets live in `scratch`, a fixed array in the
@@ -15,7 +15,7 @@
  *
  * The array is shared by every call on a GPU: calls that overlap on one GPU
  * (different streams or host threads) race on it.  Nothing in it needs
- * clearing: each call's count pass writes every block count it later reads,
+ * clearing: each call's count pass writes every group count it later reads,
  * and the scan writes every offset.
  */
 #include <climits>
@@ -25,8 +25,9 @@
 
 namespace ax {
 
-/* block counts (int) + block offsets (long long) of up to kNoallocBlocks
- * 256-site blocks: 2^19 blocks = 2^27 sites (512^3), 6 MiB */
+/* group counts (int) + group offsets (long long) of up to kNoallocBlocks
+ * groups, 6 MiB; the lattices accepted, up to kNoallocBlocks * 256 = 2^27
+ * sites (512^3), have at most 2^18 groups (cross_groups) */
 constexpr size_t kNoallocBlocks = (size_t)1 << 19;
 constexpr size_t kNoallocCountBytes = kNoallocBlocks * sizeof(int);
 constexpr size_t kNoallocBytes = kNoallocCountBytes + kNoallocBlocks * sizeof(long long);
@@ -62,8 +63,7 @@ extern "C" int ax_crossings_noalloc(ax_lattice *L, double *xyz, size_t cap, int6
   if (!L || !count || (cap && !xyz)) return fail(AX_EINVAL, "NULL argument");
   const ax_params &p = lattice_params(L);
   const size_t V = lattice_sites(L);
-  const size_t nb = (V + 255) / 256;
-  if (nb > kNoallocBlocks)
+  if (V > kNoallocBlocks * 256 || cross_groups(V) > kNoallocBlocks)
     return fail(AX_EINVAL, "lattice of %zu sites exceeds the %zu sites ax_crossings_noalloc supports", V,
                 kNoallocBlocks * 256);
   if (cap > (size_t)LLONG_MAX / 3) return fail(AX_EINVAL, "capacity %zu", cap);
