@@ -844,7 +844,8 @@ size_t diag_part_blocks(const ax_params &p) {
   const size_t V = (size_t)p.nx * p.ny * p.nz;
   const size_t site = (V + 255) / 256;
   const size_t march = (size_t)make_tile_grid(p.nx, p.ny, p.nz, diag_xseg(p.nx, p.ny, p.nz)).work;
-  return site > march ? site : march;
+  const size_t glob = p.model == AX_MODEL_GLOBAL ? global_energy_blocks(p) : 0;
+  return std::max(site, std::max(march, glob));
 }
 
 int ensure_phase_buffer(ax_lattice *L) {

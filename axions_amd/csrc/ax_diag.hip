@@ -219,6 +219,7 @@ __global__ void __launch_bounds__(256) diag_kernel(DiagConsts k, Levels<T> L, in
 __global__ void __launch_bounds__(1024) sum3_kernel(const double *part, int nb, double *out) {
   __shared__ double sh[3][16];
   double v[3] = {0, 0, 0};
+#pragma unroll 4
   for (int i = threadIdx.x; i < nb; i += 1024)
     for (int c = 0; c < 3; ++c) v[c] += part[3 * i + c];
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -284,19 +285,6 @@ __global__ void __launch_bounds__(256) winding_kernel(int nx, int ny, int nz, co
  * offsets) with a scan in between.  512^3 FP64, 1.2 points a site: counts
  * 2.67 -> 1.56 ms, scan 0.92 -> 0.15, points 6.96 -> 2.94 (3.9 GB written);
  * FP32 2.63 -> 1.45, 0.92 -> 0.15, 6.29 -> 2.72.  Bound by instructions. */
-
-/* n / d for n < 2^31 and d >= 2 by a multiplication: m = floor(2^(31+s)/d) + 1
- * with 2^(s-1) < d <= 2^s exceeds 2^(31+s)/d by less than 2^s/d <= 2, so the
- * quotient's error stays below 1/d */
-struct FastDiv {
-  uint32_t d, m, s;
-};
-static FastDiv fast_div(uint32_t d) {
-  uint32_t s = 1;
-  while (((uint64_t)1 << s) < d) ++s;
-  return {d, (uint32_t)(((uint64_t)1 << (31 + s)) / d + 1), s - 1};
-}
-__device__ __forceinline__ uint32_t quotient(uint32_t n, const FastDiv &f) { return __umulhi(n, f.m) >> f.s; }
 
 struct CrossGeom {
   int nx, ny, nz, ex, ez, x0, y0, z0;

@@ -21,9 +21,21 @@
  *                        dt/2 and central differences of the field as a
  *                        one-thread run holds it mid-loop -- neighbours
  *                        earlier in loop order already updated, later ones
- *                        not -- accumulated in FP64 per block.
+ *                        not -- accumulated in FP64 per wave.
+ *
+ * The last two take one thread per site, or per two z neighbours where nz is
+ * even, blocks of consecutive sites on one XCD.  With spacings that are
+ * powers of two (POW2) the divisions by dx^2 and 2 dx are multiplications by
+ * the exact reciprocals, the same bits.  200^3 FP64, Neumann faces: step 132
+ * -> 103 us (64 bytes a site: 5.0 TB/s, a copy reaches 4.8), energy 192 ->
+ * 121 us; before, every index was divided out for each neighbour, the twelve
+ * quotients were divisions and every lane loaded 8 bytes at a time.  A march
+ * along x with the planes in registers was slower (156 and 125 us).
  */
+#include <algorithm>
+
 #include "ax_internal.h"
+#include "ax_march.h"
 
 namespace ax {
 
@@ -31,25 +43,24 @@ struct GlobalGeom {
   int nx, ny, nz;
   int periodic;          /* 1: all sites updated, periodic wrap; 0: Neumann x/y faces */
   double dx, dy, dz, dt;
+  uint32_t V, per, eper;   /* sites; blocks of the step and of the energy per XCD */
+  bool wide;               /* two sites a thread */
+  FastDiv by_nz, by_ny;
 };
 
 template <typename R>
-__device__ __forceinline__ R glap(const R *f, size_t s, size_t xp, size_t xm, size_t yp, size_t ym, size_t zp,
-                                  size_t zm, R dx2, R dy2, R dz2, R mag) {
-  R xx = (f[xp] - 2 * f[s] + f[xm]) / dx2;
-  R yy = (f[yp] - 2 * f[s] + f[ym]) / dy2;
-  R zz = (f[zp] - 2 * f[s] + f[zm]) / dz2;
-  return xx + yy + zz - (mag - 1) * f[s];
-}
+struct GlobalConsts {
+  R dx2, dy2, dz2, ix2, iy2, iz2;   /* dx*dx ... and their reciprocals */
+  R tx, ty, tz, itx, ity, itz;      /* 2 dx ... */
+  R dt;
+};
 
-/* site s = (i,j,k) is updated by the step: interior x/y for Neumann faces */
-__device__ __forceinline__ bool g_site(const GlobalGeom &g, int s, int &i, int &j, int &k) {
-  k = s % g.nz;
-  const int r = s / g.nz;
-  j = r % g.ny;
-  i = r / g.ny;
-  if (g.periodic) return true;
-  return i > 0 && i < g.nx - 1 && j > 0 && j < g.ny - 1;
+template <typename R, bool POW2>
+__device__ __forceinline__ R glap(const GlobalConsts<R> &k, R f, R xp, R xm, R yp, R ym, R zp, R zm, R mag) {
+  R xx = mdiv<R, POW2>(xp - 2 * f + xm, k.dx2, k.ix2);
+  R yy = mdiv<R, POW2>(yp - 2 * f + ym, k.dy2, k.iy2);
+  R zz = mdiv<R, POW2>(zp - 2 * f + zm, k.dz2, k.iz2);
+  return xx + yy + zz - (mag - 1) * f;
 }
 
 template <typename R>
@@ -87,80 +98,185 @@ __global__ void __launch_bounds__(256) global_bc_kernel(GlobalGeom g, R *pr, R *
   qi[d] = vi;
 }
 
+/* W sites of a thread: one, or two neighbours along z (nz even, so that both
+ * lie in one row and their 16 (FP64) or 8 bytes are aligned).  A request
+ * takes the addresser the same time whatever a lane's width, and both kernels
+ * were bound by it (busy 78 % of the launch): with two sites a lane issues 9
+ * instead of 20 requests per site (step), 11 instead of 26 (energy). */
+template <typename R, int W>
+struct Sites {
+  typedef R vec __attribute__((ext_vector_type(W)));
+  R v[W];
+  __device__ static Sites load(const R *p, uint32_t s) {
+    Sites o;
+    const vec t = *(const vec *)(p + s);
+#pragma unroll
+    for (int q = 0; q < W; ++q) o.v[q] = t[q];
+    return o;
+  }
+  __device__ void store(R *p, uint32_t s) const {
+    vec t;
+#pragma unroll
+    for (int q = 0; q < W; ++q) t[q] = v[q];
+    *(vec *)(p + s) = t;
+  }
+};
 template <typename R>
-__global__ void __launch_bounds__(256) global_step_kernel(GlobalGeom g, const R *ar, const R *ai, R *br, R *bi,
-                                                          R *mr, R *mi) {
-  const int V = g.nx * g.ny * g.nz;
-  const int s = blockIdx.x * 256 + threadIdx.x;
+struct Sites<R, 1> {
+  R v[1];
+  __device__ static Sites load(const R *p, uint32_t s) { return {{p[s]}}; }
+  __device__ void store(R *p, uint32_t s) const { p[s] = v[0]; }
+};
+
+/* The first of this thread's W sites in run `run` of 256 threads, its
+ * coordinates and its neighbours; on: the step updates them (they are within
+ * the lattice and no Neumann face). */
+template <int W>
+struct GlobalSite {
+  uint32_t s, xp, xm, yp, ym, zp, zm;   /* zp: after the last of the W sites */
   int i, j, k;
-  if (s >= V || !g_site(g, s, i, j, k)) return;
-  const int ny = g.ny, nz = g.nz;
-  auto id = [&](int a, int b, int c) { return ((size_t)a * ny + b) * nz + c; };
-  const int ip = wrapp(i, g.nx), im = wrapm(i, g.nx), jp = wrapp(j, ny), jm = wrapm(j, ny);
-  const int kp = wrapp(k, nz), km = wrapm(k, nz);
-  const size_t xp = id(ip, j, k), xm = id(im, j, k), yp = id(i, jp, k), ym = id(i, jm, k);
-  const size_t zp = id(i, j, kp), zm = id(i, j, km);
-  const R dx2 = (R)(g.dx * g.dx), dy2 = (R)(g.dy * g.dy), dz2 = (R)(g.dz * g.dz), dt = (R)g.dt;
-  const R mag = ar[s] * ar[s] + ai[s] * ai[s];
-  const R t0 = glap(ar, s, xp, xm, yp, ym, zp, zm, dx2, dy2, dz2, mag);
-  const R t1 = glap(ai, s, xp, xm, yp, ym, zp, zm, dx2, dy2, dz2, mag);
-  const R p0 = mr[s] + t0 * dt, p1 = mi[s] + t1 * dt;
-  mr[s] = p0;
-  mi[s] = p1;
-  br[s] = ar[s] + p0 * dt;
-  bi[s] = ai[s] + p1 * dt;
+  bool on;
+  __device__ GlobalSite(const GlobalGeom &g, uint32_t run) {
+    const uint32_t at = (run * 256 + threadIdx.x) * W;
+    s = min(at, g.V - W);               /* every lane holds loadable sites */
+    const uint32_t r = quotient(s, g.by_nz);
+    i = (int)quotient(r, g.by_ny);
+    k = (int)(s - r * g.nz);
+    j = (int)(r - i * g.ny);
+    on = at < g.V && (g.periodic || (i > 0 && i < g.nx - 1 && j > 0 && j < g.ny - 1));
+    const int nz = g.nz, nyz = g.ny * nz;
+    xp = i == g.nx - 1 ? s - (g.nx - 1) * nyz : s + nyz;
+    xm = i == 0 ? s + (g.nx - 1) * nyz : s - nyz;
+    yp = j == g.ny - 1 ? s - (nyz - nz) : s + nz;
+    ym = j == 0 ? s + (nyz - nz) : s - nz;
+    zp = k + W == nz ? s - k : s + W;
+    zm = k == 0 ? s + (nz - 1) : s - 1;
+  }
+  /* f at z - 1 and z + 1 of the W sites from f there: between lanes by a
+   * shift, at the ends of the wave and of the row by a load */
+  template <typename R>
+  __device__ Sites<R, W> below(const GlobalGeom &g, const R *f, const Sites<R, W> &c) const {
+    Sites<R, W> o;
+    o.v[0] = lane_prev(c.v[W - 1], c.v[0]);
+    if ((threadIdx.x & 63) == 0 || k == 0) o.v[0] = f[zm];
+    if (W == 2) o.v[W - 1] = c.v[0];
+    return o;
+  }
+  template <typename R>
+  __device__ Sites<R, W> above(const GlobalGeom &g, const R *f, const Sites<R, W> &c) const {
+    Sites<R, W> o;
+    const R next = lane_next(c.v[0], c.v[0]);
+    o.v[W - 1] = next;
+    if ((threadIdx.x & 63) == 63 || k + W == g.nz) o.v[W - 1] = f[zp];
+    if (W == 2) o.v[0] = c.v[W - 1];
+    return o;
+  }
+};
+
+template <typename R, bool POW2, int W>
+__global__ void __launch_bounds__(256) global_step_kernel(GlobalGeom g, GlobalConsts<R> c, const R *__restrict__ ar,
+                                                          const R *__restrict__ ai, R *__restrict__ br,
+                                                          R *__restrict__ bi, R *__restrict__ mr, R *__restrict__ mi) {
+  typedef Sites<R, W> S;
+  const GlobalSite<W> q(g, (blockIdx.x & 7) * g.per + (blockIdx.x >> 3));
+  const R *f[2] = {ar, ai};
+  R *n[2] = {br, bi}, *m[2] = {mr, mi};
+  S here[2], xp[2], xm[2], yp[2], ym[2], mom[2];
+#pragma unroll
+  for (int v = 0; v < 2; ++v) {
+    here[v] = S::load(f[v], q.s);
+    xp[v] = S::load(f[v], q.xp);
+    xm[v] = S::load(f[v], q.xm);
+    yp[v] = S::load(f[v], q.yp);
+    ym[v] = S::load(f[v], q.ym);
+    mom[v] = S::load(m[v], q.s);
+  }
+#pragma unroll
+  for (int v = 0; v < 2; ++v) {
+    const S zm = q.below(g, f[v], here[v]), zp = q.above(g, f[v], here[v]);
+    S p, o;
+#pragma unroll
+    for (int e = 0; e < W; ++e) {
+      const R mag = here[0].v[e] * here[0].v[e] + here[1].v[e] * here[1].v[e];
+      const R t = glap<R, POW2>(c, here[v].v[e], xp[v].v[e], xm[v].v[e], yp[v].v[e], ym[v].v[e], zp.v[e], zm.v[e], mag);
+      p.v[e] = mom[v].v[e] + t * c.dt;
+      o.v[e] = here[v].v[e] + p.v[e] * c.dt;
+    }
+    if (q.on) {
+      p.store(m[v], q.s);
+      o.store(n[v], q.s);
+    }
+  }
 }
 
-template <typename R>
-__global__ void __launch_bounds__(256) global_energy_kernel(GlobalGeom g, const R *ar, const R *ai, const R *br,
-                                                            const R *bi, const R *mr, const R *mi, double *part) {
+/* o: the pre-step field, n: the step's result, m: its momentum.  A block
+ * takes kEnergyRuns consecutive runs of 256 threads' sites. */
+constexpr int kEnergyRuns = 4;
+template <typename R, bool POW2, int W>
+__global__ void __launch_bounds__(256) global_energy_kernel(GlobalGeom g, GlobalConsts<R> c, const R *__restrict__ ar,
+                                                            const R *__restrict__ ai, const R *__restrict__ br,
+                                                            const R *__restrict__ bi, const R *__restrict__ mr,
+                                                            const R *__restrict__ mi, double *__restrict__ part) {
+  typedef Sites<R, W> S;
   __shared__ double sh[2][4];
-  const int V = g.nx * g.ny * g.nz;
-  const int s = blockIdx.x * 256 + threadIdx.x;
   double rho = 0, bad = 0;
-  int i, j, k;
-  if (s < V && g_site(g, s, i, j, k)) {
-    const int ny = g.ny, nz = g.nz;
-    auto id = [&](int a, int b, int c) { return ((size_t)a * ny + b) * nz + c; };
-    const int ip = wrapp(i, g.nx), im = wrapm(i, g.nx), jp = wrapp(j, ny), jm = wrapm(j, ny);
-    const int kp = wrapp(k, nz), km = wrapm(k, nz);
-    const size_t xp = id(ip, j, k), xm = id(im, j, k), yp = id(i, jp, k), ym = id(i, jm, k);
-    const size_t zp = id(i, j, kp), zm = id(i, j, km);
-    const R dx2 = (R)(g.dx * g.dx), dy2 = (R)(g.dy * g.dy), dz2 = (R)(g.dz * g.dz);
-    const R dx = (R)g.dx, dy = (R)g.dy, dz = (R)g.dz;
-    const R mag = ar[s] * ar[s] + ai[s] * ai[s];
-    const R t[2] = {glap(ar, s, xp, xm, yp, ym, zp, zm, dx2, dy2, dz2, mag),
-                    glap(ai, s, xp, xm, yp, ym, zp, zm, dx2, dy2, dz2, mag)};
-    /* the value a one-thread loop sees at neighbour n: updated already
-     * (new field) iff n is an updated site earlier in loop order */
-    auto seen = [&](const R *o, const R *nw, size_t n) -> R {
-      int a, b, c;
-      const bool upd = g_site(g, (int)n, a, b, c);
-      return (upd && n < (size_t)s) ? nw[n] : o[n];
-    };
-    double gx[2], gy[2], gz[2];
-    const R *O[2] = {ar, ai}, *N[2] = {br, bi};
+  const uint32_t blk = (blockIdx.x & 7) * g.eper + (blockIdx.x >> 3);
+  const R *o[2] = {ar, ai}, *n[2] = {br, bi}, *m[2] = {mr, mi};
+#pragma unroll 1
+  for (int run = 0; run < kEnergyRuns; ++run) {
+    const GlobalSite<W> q(g, blk * kEnergyRuns + run);
+    /* a neighbour holds its new value when it is an updated site earlier in
+     * loop order (x, then y, then z): x - 1 and y - 1 unless they wrap or are
+     * faces, z - 1 unless it wraps; x + 1, y + 1, z + 1 only where they wrap */
+    const int first = g.periodic ? 0 : 1;
+    S here[2], now[2], mom[2];
+    R t[2][W], gx[2][W], gy[2][W], gz[2][W];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      gx[c] = (double)((seen(O[c], N[c], xp) - seen(O[c], N[c], xm)) / (2 * dx));
-      gy[c] = (double)((seen(O[c], N[c], yp) - seen(O[c], N[c], ym)) / (2 * dy));
-      gz[c] = (double)((seen(O[c], N[c], zp) - seen(O[c], N[c], zm)) / (2 * dz));
+    for (int v = 0; v < 2; ++v) {
+      here[v] = S::load(o[v], q.s);
+      now[v] = S::load(n[v], q.s);
+      mom[v] = S::load(m[v], q.s);
     }
-    const double r0 = (double)mr[s] - 0.5 * (double)t[0] * g.dt;
-    const double r1 = (double)mi[s] - 0.5 * (double)t[1] * g.dt;
-    const double dm = (double)mag - 1;
-    rho = r0 * r0 + r1 * r1 + gx[0] * gx[0] + gx[1] * gx[1] + gy[0] * gy[0] + gy[1] * gy[1] + gz[0] * gz[0] +
-          gz[1] * gz[1] + 0.5 * (dm * dm);
-    rho = g.dx * g.dy * g.dz * rho;
-    bad = (isfinite((double)br[s]) && isfinite((double)bi[s]) && isfinite((double)mr[s]) && isfinite((double)mi[s]))
-              ? 0.0 : 1.0;
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      const S xp = S::load(o[v], q.xp), xm = S::load(o[v], q.xm), yp = S::load(o[v], q.yp), ym = S::load(o[v], q.ym);
+      const S zp = q.above(g, o[v], here[v]), zm = q.below(g, o[v], here[v]);
+      S xps = xp, yps = yp, zps = zp;
+      S xms = S::load(n[v], q.xm), yms = S::load(n[v], q.ym), zms = q.below(g, n[v], now[v]);
+      if (q.i <= first) xms = xm;
+      if (q.j <= first) yms = ym;
+      if (q.k == 0) zms.v[0] = zm.v[0];
+      if (q.i == g.nx - 1) xps = S::load(n[v], q.xp);
+      if (q.j == g.ny - 1) yps = S::load(n[v], q.yp);
+      if (q.k + W == g.nz) zps.v[W - 1] = n[v][q.zp];
+#pragma unroll
+      for (int e = 0; e < W; ++e) {
+        const R mag = here[0].v[e] * here[0].v[e] + here[1].v[e] * here[1].v[e];
+        t[v][e] = glap<R, POW2>(c, here[v].v[e], xp.v[e], xm.v[e], yp.v[e], ym.v[e], zp.v[e], zm.v[e], mag);
+        gx[v][e] = mdiv<R, POW2>(xps.v[e] - xms.v[e], c.tx, c.itx);
+        gy[v][e] = mdiv<R, POW2>(yps.v[e] - yms.v[e], c.ty, c.ity);
+        gz[v][e] = mdiv<R, POW2>(zps.v[e] - zms.v[e], c.tz, c.itz);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < W; ++e) {
+      const R mag = here[0].v[e] * here[0].v[e] + here[1].v[e] * here[1].v[e];
+      const double r0 = (double)mom[0].v[e] - 0.5 * (double)t[0][e] * g.dt;
+      const double r1 = (double)mom[1].v[e] - 0.5 * (double)t[1][e] * g.dt;
+      const double dm = (double)mag - 1;
+      const double gx0 = gx[0][e], gx1 = gx[1][e], gy0 = gy[0][e], gy1 = gy[1][e], gz0 = gz[0][e], gz1 = gz[1][e];
+      const double r = r0 * r0 + r1 * r1 + gx0 * gx0 + gx1 * gx1 + gy0 * gy0 + gy1 * gy1 + gz0 * gz0 + gz1 * gz1 +
+                       0.5 * (dm * dm);
+      if (q.on) {
+        rho += g.dx * g.dy * g.dz * r;
+        bad += (isfinite((double)now[0].v[e]) && isfinite((double)now[1].v[e]) && isfinite((double)mom[0].v[e]) &&
+                isfinite((double)mom[1].v[e])) ? 0.0 : 1.0;
+      }
+    }
   }
   /* fixed-order block sums */
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    rho += __shfl_xor(rho, off, 64);
-    bad += __shfl_xor(bad, off, 64);
-  }
+  rho = march_wave_sum(rho);
+  bad = march_wave_sum(bad);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   if (l == 0) {
     sh[0][w] = rho;
@@ -168,28 +284,9 @@ __global__ void __launch_bounds__(256) global_energy_kernel(GlobalGeom g, const 
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    part[3 * blockIdx.x] = (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]);
-    part[3 * blockIdx.x + 1] = 0;
-    part[3 * blockIdx.x + 2] = (sh[1][0] + sh[1][1]) + (sh[1][2] + sh[1][3]);
-  }
-}
-
-__global__ void __launch_bounds__(1024) global_sum3_kernel(const double *part, int nb, double *out) {
-  __shared__ double sh[3][16];
-  double a[3] = {0, 0, 0};
-  for (int b = threadIdx.x; b < nb; b += 1024)
-    for (int c = 0; c < 3; ++c) a[c] += part[3 * b + c];
-  for (int c = 0; c < 3; ++c) {
-    double v = a[c];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if ((threadIdx.x & 63) == 0) sh[c][threadIdx.x >> 6] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < 3) {
-    double v = 0;
-    for (int w = 0; w < 16; ++w) v += sh[threadIdx.x][w];
-    out[threadIdx.x] = v;
+    part[3 * (size_t)blockIdx.x] = (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]);
+    part[3 * (size_t)blockIdx.x + 1] = 0;
+    part[3 * (size_t)blockIdx.x + 2] = (sh[1][0] + sh[1][1]) + (sh[1][2] + sh[1][3]);
   }
 }
 
@@ -198,7 +295,36 @@ static GlobalGeom geom_of(const ax_params &p) {
   g.nx = p.nx; g.ny = p.ny; g.nz = p.nz;
   g.periodic = p.boundary == AX_BC_PERIODIC;
   g.dx = p.dx; g.dy = p.dy; g.dz = p.dz; g.dt = p.dt;
+  g.V = (uint32_t)p.nx * p.ny * p.nz;
+  g.wide = p.nz % 2 == 0;
+  const uint32_t runs = (g.V + 255) / 256 / (g.wide ? 2 : 1) + 1;   /* of 256 threads */
+  g.per = (runs + 7) / 8;
+  g.eper = ((runs + kEnergyRuns - 1) / kEnergyRuns + 7) / 8;
+  g.by_nz = fast_div((uint32_t)p.nz);
+  g.by_ny = fast_div((uint32_t)p.ny);
   return g;
+}
+
+size_t global_energy_blocks(const ax_params &p) { return (size_t)8 * geom_of(p).eper; }
+
+template <typename R>
+static GlobalConsts<R> consts_of(const ax_params &p) {
+  GlobalConsts<R> k;
+  k.dx2 = (R)(p.dx * p.dx); k.dy2 = (R)(p.dy * p.dy); k.dz2 = (R)(p.dz * p.dz);
+  k.tx = 2 * (R)p.dx; k.ty = 2 * (R)p.dy; k.tz = 2 * (R)p.dz;
+  k.ix2 = 1 / k.dx2; k.iy2 = 1 / k.dy2; k.iz2 = 1 / k.dz2;
+  k.itx = 1 / k.tx; k.ity = 1 / k.ty; k.itz = 1 / k.tz;
+  k.dt = (R)p.dt;
+  return k;
+}
+
+/* every divisor a power of two with a normal reciprocal */
+template <typename R>
+static bool pow2_of(const GlobalConsts<R> &k) {
+  const R d[6] = {k.dx2, k.dy2, k.dz2, k.tx, k.ty, k.tz};
+  for (R v : d)
+    if (!is_pow2(v) || !std::isnormal(v) || !std::isnormal(1 / v)) return false;
+  return true;
 }
 
 template <typename R>
@@ -213,8 +339,16 @@ hipError_t launch_global_step(const ax_params &p, void *state, size_t pitch, int
     const int nbs = 2 * p.ny * p.nz + 2 * (p.nx - 2) * p.nz;
     hipLaunchKernelGGL((global_bc_kernel<R>), dim3((nbs + 255) / 256), dim3(256), 0, st, g, ar, ai, br, bi);
   }
-  const int V = p.nx * p.ny * p.nz;
-  hipLaunchKernelGGL((global_step_kernel<R>), dim3((V + 255) / 256), dim3(256), 0, st, g, ar, ai, br, bi, mr, mi);
+  const GlobalConsts<R> k = consts_of<R>(p);
+  const dim3 grid(8 * g.per), block(256);
+#define AX_GS(P2, W) \
+  hipLaunchKernelGGL((global_step_kernel<R, P2, W>), grid, block, 0, st, g, k, ar, ai, br, bi, mr, mi)
+  const bool p2 = pow2_of(k);
+  if (p2 && g.wide) AX_GS(true, 2);
+  else if (p2) AX_GS(true, 1);
+  else if (g.wide) AX_GS(false, 2);
+  else AX_GS(false, 1);
+#undef AX_GS
   return hipGetLastError();
 }
 
@@ -224,13 +358,20 @@ hipError_t launch_global_energy(const ax_params &p, const void *state, size_t pi
   const R *b = (const R *)state;
   const int cur = n % 2, nw = 1 - cur;   /* the pre-step field of TimeStep n and its result */
   const GlobalGeom g = geom_of(p);
-  const int V = p.nx * p.ny * p.nz;
-  const int nb = (V + 255) / 256;
-  hipLaunchKernelGGL((global_energy_kernel<R>), dim3(nb), dim3(256), 0, st, g, b + (size_t)cur * pitch,
-                     b + (size_t)(2 + cur) * pitch, b + (size_t)nw * pitch, b + (size_t)(2 + nw) * pitch,
-                     b + 4 * pitch, b + 5 * pitch, part);
-  hipLaunchKernelGGL(global_sum3_kernel, dim3(1), dim3(1024), 0, st, part, nb, out3);
-  return hipGetLastError();
+  const GlobalConsts<R> k = consts_of<R>(p);
+  const dim3 grid(8 * g.eper), block(256);   /* part holds 3 doubles each (diag_part_blocks) */
+#define AX_GE(P2, W)                                                                                              \
+  hipLaunchKernelGGL((global_energy_kernel<R, P2, W>), grid, block, 0, st, g, k, b + (size_t)cur * pitch,          \
+                     b + (size_t)(2 + cur) * pitch, b + (size_t)nw * pitch, b + (size_t)(2 + nw) * pitch, b + 4 * pitch, \
+                     b + 5 * pitch, part)
+  const bool p2 = pow2_of(k);
+  if (p2 && g.wide) AX_GE(true, 2);
+  else if (p2) AX_GE(true, 1);
+  else if (g.wide) AX_GE(false, 2);
+  else AX_GE(false, 1);
+#undef AX_GE
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? launch_sum3(part, 8 * g.eper, out3, st) : e;
 }
 
 template hipError_t launch_global_step<double>(const ax_params &, void *, size_t, int, hipStream_t);

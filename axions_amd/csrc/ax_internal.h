@@ -46,6 +46,19 @@ inline TileGrid make_tile_grid(int nx, int ny, int nz, int xseg) {
   return g;
 }
 
+/* n / d for n < 2^31 and d >= 2 by a multiplication: m = floor(2^(31+s)/d) + 1
+ * with 2^(s-1) < d <= 2^s exceeds 2^(31+s)/d by less than 2^s/d <= 2, so the
+ * quotient's error stays below 1/d */
+struct FastDiv {
+  uint32_t d, m, s;
+};
+inline FastDiv fast_div(uint32_t d) {
+  uint32_t s = 1;
+  while (((uint64_t)1 << s) < d) ++s;
+  return {d, (uint32_t)(((uint64_t)1 << (31 + s)) / d + 1), s - 1};
+}
+__device__ __forceinline__ uint32_t quotient(uint32_t n, const FastDiv &f) { return __umulhi(n, f.m) >> f.s; }
+
 /* x planes per wave of a march over the whole lattice, at most cap.  A wave
  * pays a prologue worth about one plane, so long segments do the least work;
  * but a lattice of few rows then fills few of the chip's 1024 SIMDs, and
@@ -135,6 +148,7 @@ hipError_t launch_step_tiled_moore(const StepConsts &k, const Levels<R> &L, int 
 
 template <typename R>
 hipError_t launch_global_step(const ax_params &p, void *state, size_t pitch, int n, hipStream_t st);
+size_t global_energy_blocks(const ax_params &p);   /* partial-sum blocks of launch_global_energy */
 template <typename R>
 hipError_t launch_global_energy(const ax_params &p, const void *state, size_t pitch, int n, double *part,
                                 double *out3, hipStream_t st);

@@ -101,3 +101,29 @@ def test_global_winding_and_crossings():
     assert np.array_equal(w, orc.winding(pa, sa, 0, 0))
     po, co = orc.crossings(pa, sa, 0)
     assert cnt == co and np.array_equal(pts, po)
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("boundary", [AX_BC_PERIODIC, ax.AX_BC_NEUMANN_XY])
+@pytest.mark.parametrize("shape", [(3, 3, 3), (3, 4, 4), (6, 5, 130), (9, 7, 63), (5, 6, 128), (17, 33, 34)])
+def test_global_sites_per_thread(shape, boundary, precision):
+    """One and two sites per thread (nz odd, even), rows shorter and longer
+    than a wave, exact reciprocals (dx = 0.25) and divisions (0.3)."""
+    nx, ny, nz = shape
+    for dx in (0.25, 0.3):
+        p = ax.global_params(nx, ny=ny, nz=nz, dx=dx, dt=0.05, boundary=boundary, precision=precision)
+        say(f"[global] {shape} dx={dx} boundary={boundary} FP{precision}")
+        st = orc.init_random_phase(p, 5)
+        V = nx * ny * nz
+        st[2 * V:] = np.random.default_rng(3).uniform(-0.2, 0.2, 2 * V)
+        if precision == 32:
+            st = st.astype(np.float32)
+        with ax.Lattice(p) as lat:
+            lat.set_state(st.astype(np.float64))
+            for n in range(6):
+                lat.step(1)
+                e = orc.global_step(p, st, 1)[0]
+                d = lat.diagnostics(winding=False)
+                assert d["finite"] == 1 and rel(d["energy"], e) < 1e-12, (n, d["energy"], e)
+            g = lat.get_state()
+            assert np.array_equal(g.view(np.uint64), st.astype(np.float64).view(np.uint64))
