@@ -551,9 +551,9 @@ int ax_diagnostics(ax_lattice *L, int32_t want_winding, ax_diag *out) {
     int rc = prepare_faces(L);
     if (rc) return rc;
     march = use_diag_march(p);
-    /* the windings come from the march's edge values (periodic), else from
+    /* the windings come from the march's edge values, else from
      * launch_winding_field */
-    mwind = want_winding && march && use_diag_march_windings(p) && ensure_phase_buffer(L) == AX_OK;
+    mwind = want_winding && march && ensure_phase_buffer(L) == AX_OK;
     if (march)
       e = launch_march_diag(L, mwind);
     else if (L->esize == 8)
@@ -568,8 +568,7 @@ int ax_diagnostics(ax_lattice *L, int32_t want_winding, ax_diag *out) {
       e = launch_phase_winding(L, nullptr, L->dres + 4);
       if (e != hipSuccess) return hip_fail(e, "winding launch");
     } else {
-      int rc = ensure_winding_buffer(L);
-      if (!rc) rc = launch_winding_field(L, 0, L->wind, L->part, L->dres + 4);
+      int rc = launch_winding_field(L, 0, nullptr, L->part, L->dres + 4);
       if (rc) return rc;
     }
   }
@@ -745,15 +744,9 @@ int ax_winding_field(ax_lattice *L, int32_t field, int8_t *out, size_t n) {
   if (n != 3 * L->V) return fail(AX_EINVAL, "winding length %zu != %zu", n, 3 * L->V);
   if (field < 0 || field > (L->p.model == AX_MODEL_MOORE ? 1 : 0)) return fail(AX_EINVAL, "field %d", field);
   int rc = ensure_winding_buffer(L);
+  if (!rc) rc = prepare_faces(L);
+  if (!rc) rc = launch_winding_field(L, field, L->wind, L->part, L->dres + 4);
   if (rc) return rc;
-  if (use_diag_march_windings(L->p) && ensure_phase_buffer(L) == AX_OK) {
-    hipError_t e = launch_march_diag(L, true);
-    if (e == hipSuccess) e = launch_phase_winding(L, L->wind, L->dres + 4);
-    if (e != hipSuccess) return hip_fail(e, "winding launch");
-  } else {
-    rc = launch_winding_field(L, field, L->wind, L->part, L->dres + 4);
-    if (rc) return rc;
-  }
   hipError_t e = hipMemcpyAsync(out, L->wind, n, hipMemcpyDeviceToHost, L->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(L->stream);
   return e == hipSuccess ? AX_OK : hip_fail(e, "winding readback");
@@ -834,11 +827,6 @@ bool use_diag_march(const ax_params &p) {
   return p.model == AX_MODEL_AH && getenv("AX_DIAG_SITE_KERNEL") == nullptr;
 }
 
-/* ... and the windings from the edge values it stores (periodic lattices) */
-bool use_diag_march_windings(const ax_params &p) {
-  return use_diag_march(p) && p.boundary == AX_BC_PERIODIC && p.boundary_z == AX_BC_PERIODIC;
-}
-
 /* partial-sum blocks any diagnostic pass of this lattice writes */
 size_t diag_part_blocks(const ax_params &p) {
   const size_t V = (size_t)p.nx * p.ny * p.nz;
@@ -869,7 +857,9 @@ hipError_t launch_march_diag(ax_lattice *L, bool phases) {
 /* windings of the current level from the edge values launch_march_diag
  * stored */
 hipError_t launch_phase_winding(ax_lattice *L, int8_t *out, double *res3) {
-  return launch_wind_phase(L->p.nx, L->p.ny, L->p.nz, L->phase, out, L->part, res3, L->stream);
+  const ax_params &p = L->p;
+  return launch_wind_phase(p.nx, p.ny, p.nz, p.boundary != AX_BC_PERIODIC, p.boundary_z != AX_BC_PERIODIC, L->phase, out,
+                           L->part, res3, L->stream);
 }
 
 int ensure_winding_buffer(ax_lattice *L) {
@@ -893,21 +883,26 @@ int launch_winding_field(ax_lattice *L, int field, int8_t *out, double *part, do
   hipError_t e;
   auto P = [&](int c) { return glob && c >= 2 ? (size_t)4 * L->pitch : (size_t)(c * 2 + tN) * L->pitch; };
   const int ex = !glob && p.boundary != AX_BC_PERIODIC, ez = !glob && p.boundary_z != AX_BC_PERIODIC;
-  int rc = prepare_faces(L);
-  if (rc) return rc;
-  /* periodic Abelian-Higgs and Moore: the marching edge-value passes
-   * (ax_wind.h; the same integers as the site kernel) */
-  if (!glob && !ex && !ez && getenv("AX_DIAG_SITE_KERNEL") == nullptr && ensure_phase_buffer(L) == AX_OK) {
+  /* the marching edge-value passes (ax_wind.h; three edge phases a site and
+   * the same integers as the site kernel, which evaluates nine: 256^3 FP64
+   * with absorbing faces 0.78 ms against 0.20 within the energy march), while
+   * memory holds the edge values */
+  if (getenv("AX_DIAG_SITE_KERNEL") == nullptr && ensure_phase_buffer(L) == AX_OK) {
     if (L->esize == 8) {
       const double *b = (const double *)L->state;
-      e = launch_edge_winding<double>(p.nx, p.ny, p.nz, b + P(c0), b + P(c0 + 1), b + P(t0), b + P(t0 + 1),
+      e = launch_edge_winding<double>(p.nx, p.ny, p.nz, ex, ez, b + P(c0), b + P(c0 + 1), b + P(t0), b + P(t0 + 1),
                                       b + P(t0 + 2), q, L->phase, out, part, res3, L->stream);
     } else {
       const float *b = (const float *)L->state;
-      e = launch_edge_winding<float>(p.nx, p.ny, p.nz, b + P(c0), b + P(c0 + 1), b + P(t0), b + P(t0 + 1),
+      e = launch_edge_winding<float>(p.nx, p.ny, p.nz, ex, ez, b + P(c0), b + P(c0 + 1), b + P(t0), b + P(t0 + 1),
                                      b + P(t0 + 2), q, L->phase, out, part, res3, L->stream);
     }
     return e == hipSuccess ? AX_OK : hip_fail(e, "winding launch");
+  }
+  if (!out) {   /* the site kernel stores the field whether wanted or not */
+    int rc = ensure_winding_buffer(L);
+    if (rc) return rc;
+    out = L->wind;
   }
   if (L->esize == 8) {
     const double *b = (const double *)L->state;

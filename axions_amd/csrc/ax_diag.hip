@@ -574,7 +574,7 @@ __global__ void __launch_bounds__(1024) scan_kernel(const int *__restrict__ in, 
  * with x/y or z not periodic only the bulk region's terms are summed, as
  * diag_kernel does),
  * carrying the x-backward field, link and link trig from the previous
- * plane, and, with PH (periodic lattices), the three forward edge phases
+ * plane, and, with PH, the three forward edge phases
  *   delta_a(s) = arg( conj(phi(s)) exp(-i theta_a(s)) phi(s+a) )
  * from the same link sincos, stored as the FP32 edge values
  * e_a(s) = delta_a(s) + theta_a(s) that wind_march_kernel combines
@@ -770,19 +770,24 @@ __global__ void __launch_bounds__(64, sizeof(T) == 8 ? 3 : 1) diag_march_kernel(
  * diagnostics stored (wind_march, ax_wind.h): one wave per work item of
  * the tile grid, carrying plane x+1's values.  out (the winding field
  * [3][V]) may be null when only the counts are wanted. */
-__global__ void __launch_bounds__(64) wind_march_kernel(int nx, int ny, int nz, const float *E, TileGrid g, int8_t *out,
-                                                        double *part) {
+__global__ void __launch_bounds__(64) wind_march_kernel(int nx, int ny, int nz, const float *E, TileGrid g, int ex,
+                                                        int ez, int8_t *out, double *part) {
   const int item = (int)blockIdx.x;
   int zc, y, seg;
   tile_item(g, ny, item, zc, y, seg);
   const int x0 = seg * g.xseg, x1 = min(nx, x0 + g.xseg);
   const WindRow w(nx, ny, nz, y, zc);
   double tot[3] = {0, 0, 0};
-  wind_march(w, E, x0, x1, [&](size_t s, const int *wn) {
+  /* plaquettes that would wrap across a non-periodic axis do not exist */
+  const bool ye = ex && y == ny - 1, ze = ez && w.z == nz - 1;
+  wind_march(w, E, x0, x1, [&](int x, size_t s, const int *wn) {
+    const bool xe = ex && x == nx - 1;
+    const bool none[3] = {xe || ye, xe || ze, ye || ze};
 #pragma unroll
     for (int pl = 0; pl < 3; ++pl) {
-      if (out) out[(size_t)pl * w.V + s] = (int8_t)wn[pl];
-      tot[pl] += (double)(wn[pl] < 0 ? -wn[pl] : wn[pl]);
+      const int v = none[pl] ? 0 : wn[pl];
+      if (out) out[(size_t)pl * w.V + s] = (int8_t)v;
+      tot[pl] += (double)(v < 0 ? -v : v);
     }
   });
   const double a = wave_sum(tot[0]), b = wave_sum(tot[1]), c = wave_sum(tot[2]);
@@ -979,8 +984,8 @@ hipError_t launch_crossings(int nx, int ny, int nz, double dx, double dy, double
 }
 
 /* The FP32 edge values of field (fr, fi) of charge q over the work items of
- * the tile grid (phase_march, ax_wind.h), for periodic lattices whose
- * energy and Gauss law take the site kernel (Moore). */
+ * the tile grid (phase_march, ax_wind.h), where no energy pass stores them
+ * along the way. */
 template <typename T>
 __global__ void __launch_bounds__(64) edge_march_kernel(int nx, int ny, int nz, const T *fr, const T *fi, const T *tx,
                                                         const T *ty, const T *tz, double q, TileGrid g, float *E) {
@@ -992,27 +997,23 @@ __global__ void __launch_bounds__(64) edge_march_kernel(int nx, int ny, int nz, 
 }
 
 template <typename T>
-hipError_t launch_edge_winding(int nx, int ny, int nz, const T *fr, const T *fi, const T *tx, const T *ty,
-                               const T *tz, double q, float *E, int8_t *out, double *part, double *out3,
+hipError_t launch_edge_winding(int nx, int ny, int nz, int ex, int ez, const T *fr, const T *fi, const T *tx,
+                               const T *ty, const T *tz, double q, float *E, int8_t *out, double *part, double *out3,
                                hipStream_t st) {
   const TileGrid g = make_tile_grid(nx, ny, nz, diag_xseg(nx, ny, nz));
   hipLaunchKernelGGL((edge_march_kernel<T>), dim3(g.work), dim3(64), 0, st, nx, ny, nz, fr, fi, tx, ty, tz, q, g,
                      E);
   hipError_t e = hipGetLastError();
-  return e == hipSuccess ? launch_wind_phase(nx, ny, nz, E, out, part, out3, st) : e;
+  return e == hipSuccess ? launch_wind_phase(nx, ny, nz, ex, ez, E, out, part, out3, st) : e;
 }
 
 template <typename T>
 hipError_t launch_diag_march(const DiagConsts &k, const Levels<T> &L, float *phase, double *part, double *out3,
                              hipStream_t st) {
   const TileGrid g = make_tile_grid(k.nx, k.ny, k.nz, diag_xseg(k.nx, k.ny, k.nz));
-  /* every divisor the P2 kernel multiplies by the reciprocal of must be a
-   * power of two whose reciprocal is finite (then a*(1/d) == a/d exactly) */
-  const double dx = k.dx, dy = k.dy, dz = k.dz, gg = k.g;
-  const double dvs[10] = {dx, dy, dz, dx * dx, dy * dy, dz * dz, gg, (gg * dx * dy) * (gg * dx * dy),
-                          (gg * dx * dz) * (gg * dx * dz), (gg * dy * dz) * (gg * dy * dz)};
-  bool p2 = gg != 0;
-  for (double d : dvs) p2 = p2 && is_pow2(fabs(d)) && std::isfinite(1 / d);
+  /* without a gauge coupling the pass divides by dx, dy, dz alone
+   * (energy_form 0 leaves out the gauge terms) */
+  const bool p2 = diag_pow2(k.dx, k.dy, k.dz, k.g == 0 && k.energy_form == 0 ? 1.0 : k.g);
 #define AX_DM(PH, P2) \
   hipLaunchKernelGGL((diag_march_kernel<T, PH, P2>), dim3(g.work), dim3(64), 0, st, k, L, g, phase, part)
   if (phase && p2) AX_DM(true, true);
@@ -1062,11 +1063,11 @@ bool diag_pow2(double dx, double dy, double dz, double gg) {
   return p2;
 }
 
-hipError_t launch_wind_phase(int nx, int ny, int nz, const float *E, int8_t *out, double *part, double *out3,
-                             hipStream_t st) {
+hipError_t launch_wind_phase(int nx, int ny, int nz, int ex, int ez, const float *E, int8_t *out, double *part,
+                             double *out3, hipStream_t st) {
   /* part holds 3 doubles per work item (diag_part_blocks) */
   const TileGrid g = make_tile_grid(nx, ny, nz, diag_xseg(nx, ny, nz));
-  hipLaunchKernelGGL(wind_march_kernel, dim3(g.work), dim3(64), 0, st, nx, ny, nz, E, g, out, part);
+  hipLaunchKernelGGL(wind_march_kernel, dim3(g.work), dim3(64), 0, st, nx, ny, nz, E, g, ex, ez, out, part);
   hipLaunchKernelGGL(sum3_kernel, dim3(1), dim3(1024), 0, st, part, g.work, out3);
   return hipGetLastError();
 }
@@ -1080,7 +1081,7 @@ hipError_t launch_wind_phase(int nx, int ny, int nz, const float *E, int8_t *out
                                           hipStream_t, bool);                                               \
   template hipError_t launch_diag_march<T>(const DiagConsts &, const Levels<T> &, float *, double *, double *, \
                                            hipStream_t);                                          \
-  template hipError_t launch_edge_winding<T>(int, int, int, const T *, const T *, const T *, const T *,      \
+  template hipError_t launch_edge_winding<T>(int, int, int, int, int, const T *, const T *, const T *, const T *,      \
                                              const T *, double, float *, int8_t *, double *, double *,      \
                                              hipStream_t);
 AX_INST(double)

@@ -131,6 +131,7 @@ int ensure_phase_buffer(ax_lattice *L);
 hipError_t launch_march_diag(ax_lattice *L, bool phases);
 hipError_t launch_phase_winding(ax_lattice *L, int8_t *out, double *res3);
 int prepare_faces(ax_lattice *L);
+/* the Neumann faces prepared (prepare_faces); out may be null */
 int launch_winding_field(ax_lattice *L, int field, int8_t *out, double *part, double *res3);
 
 template <typename R>
@@ -155,10 +156,9 @@ hipError_t launch_global_energy(const ax_params &p, const void *state, size_t pi
 
 template <typename T>
 hipError_t launch_diag(const DiagConsts &k, const Levels<T> &L, double *part, double *out3, hipStream_t st);
-/* periodic Abelian-Higgs: energy/Gauss march, with phase != NULL also the
- * FP32 edge values [3][V] (forward edge phase + link angle, ax_wind.h);
- * launch_wind_phase turns them into windings (the field into out when
- * out != NULL, the counts into out3) */
+/* Abelian-Higgs: energy/Gauss march, with phase != NULL also the FP32 edge
+ * values [3][V] (forward edge phase + link angle, ax_wind.h); launch_wind_phase turns them into windings (the field into out when
+ * out != NULL, the counts into out3; ex, ez: x and y, z not periodic) */
 /* x planes per wave of the diagnostics and winding marches (us per
  * ax_diagnostics call without / with windings; this rule against the best of
  * 1 ... 32 planes: 64^3 27.5 / 41.8 against 27.4 / 41.7, 101^3 56.7 / 99
@@ -166,18 +166,17 @@ hipError_t launch_diag(const DiagConsts &k, const Levels<T> &L, double *part, do
  * 101^3 the energy march alone took 84, with this rule 35) */
 inline int diag_xseg(int nx, int ny, int nz) { return tile_xseg(nx, ny, nz, 32); }
 bool use_diag_march(const ax_params &p);
-bool use_diag_march_windings(const ax_params &p);
 size_t diag_part_blocks(const ax_params &p);
 template <typename T>
 hipError_t launch_diag_march(const DiagConsts &k, const Levels<T> &L, float *phase, double *part, double *out3,
                              hipStream_t st);
-hipError_t launch_wind_phase(int nx, int ny, int nz, const float *E, int8_t *out, double *part, double *out3,
-                             hipStream_t st);
-/* periodic lattices: the FP32 edge values of field (fr, fi) of charge q into
- * E, then the windings from them, as launch_wind_phase */
+hipError_t launch_wind_phase(int nx, int ny, int nz, int ex, int ez, const float *E, int8_t *out, double *part,
+                             double *out3, hipStream_t st);
+/* the FP32 edge values of field (fr, fi) of charge q into E, then the
+ * windings from them, as launch_wind_phase */
 template <typename T>
-hipError_t launch_edge_winding(int nx, int ny, int nz, const T *fr, const T *fi, const T *tx, const T *ty,
-                               const T *tz, double q, float *E, int8_t *out, double *part, double *out3,
+hipError_t launch_edge_winding(int nx, int ny, int nz, int ex, int ez, const T *fr, const T *fi, const T *tx,
+                               const T *ty, const T *tz, double q, float *E, int8_t *out, double *part, double *out3,
                                hipStream_t st);
 template <typename T>
 hipError_t launch_winding(int nx, int ny, int nz, const T *fr, const T *fi, const T *tx, const T *ty, const T *tz,

@@ -193,7 +193,7 @@ __global__ void __launch_bounds__(64) pool_wind_pass_kernel(const BatchHeader *_
     const Levels<T> L = entry_levels<T>(E, E.t0 + (which == 0 ? 0 : E.steps));   /* state after t TimeSteps */
     const WindRow row(E.n, E.n, E.n, y, zc);
     if (WIND) {
-      wind_march(row, (const float *)E.phase, x0, x1, [&](size_t, const int *wn) {
+      wind_march(row, (const float *)E.phase, x0, x1, [&](int, size_t, const int *wn) {
 #pragma unroll
                       for (int c = 0; c < 3; ++c) v[c] += abs(wn[c]);
                     });

@@ -161,7 +161,7 @@ __device__ __forceinline__ int phase_march(const WindRow &w, const T *fr, const 
 }
 
 /* Windings of the xy, xz, yz plaquettes of one wave's march from the stored
- * edge values E[a V + s] = e_a(s) of the same level (above).  emit(s, w) is
+ * edge values E[a V + s] = e_a(s) of the same level (above).  emit(x, s, w) is
  * called for each of the lane's sites. */
 template <typename Emit>
 __device__ __forceinline__ void wind_march(const WindRow &w, const float *E, int x0, int x1, Emit emit) {
@@ -177,7 +177,7 @@ __device__ __forceinline__ void wind_march(const WindRow &w, const float *E, int
     wn[0] = (int)rint((cX + nY - yX - cY) * 0.15915494309189535);   /* (a, b) = (x, y) */
     wn[1] = (int)rint((cX + nZ - zX - cZ) * 0.15915494309189535);   /* (x, z) */
     wn[2] = (int)rint((cY + yZ - zY - cZ) * 0.15915494309189535);   /* (y, z) */
-    if (w.act) emit(w.site(x), wn);
+    if (w.act) emit(x, w.site(x), wn);
     cX = nX; cY = nY; cZ = nZ;
   }
 }
