@@ -11,21 +11,22 @@
  * in-place array races at chunk edges, so only the one-thread order is a
  * defined result): each point uses the new values at j-1 and the previous
  * sweep's values at j and j+1.  Sweep k at point j therefore depends only
- * on sweep k at j-1 and sweep k-1 at j, j+1.  Here lane L of a workgroup
+ * on sweep k at j-1 and sweep k-1 at j, j+1.  Here lane L of a wave
  * runs sweep k0 + L, two points behind lane L-1: at time s lane L updates
  * j = s - 2L, and the two values of sweep k-1 it needs are what lane L-1
- * produced at times s-1 (point j+1) and s-2 (point j).  They move between
- * lanes of a wave by a DPP row-crossing shift and between waves through an
- * LDS ring; the whole workgroup advances in phases of PT time steps, wave w
- * working PT*w steps behind wave 0, with one barrier per phase.  Every
- * sweep sees exactly the operands it sees in the reference loop, so the
- * profile, the sweep count and the stopping residual are the reference's
- * bits.
+ * produced at times s-1 (point j+1) and s-2 (point j), moved by a DPP
+ * row-crossing shift.  The last lane's sweep goes through device memory to
+ * the next wave, a workgroup on another CU some 150 time steps behind, so a
+ * launch keeps up to 512 waves x 64 sweeps in flight.  Every sweep sees
+ * exactly the operands it sees in the reference loop, so the profile, the
+ * sweep count and the stopping residual are the reference's bits.
  *
  * The loop stops after the first sweep whose largest |F| is not above tol
- * (or at max_iter).  A launch runs up to SOR_LANES sweeps; the host reads
- * their residuals, and when sweep k0 + L (L < last) is the stopping one it
- * re-runs that launch from its input with L + 1 lanes.
+ * (or at max_iter).  A wave holding such a sweep ends the waves behind it;
+ * the host finds the sweep in the residuals and runs that wave again up to
+ * it.  A time step is a chain of some 250 dependent instructions, 16 waves
+ * on one CU shared its issue slots: 5001 points x 6000 sweeps 51 -> 8.8 ms,
+ * 30001 points x 23278 sweeps 1.04 s -> 51 ms.
  */
 #include <math.h>
 #include <string.h>
@@ -37,11 +38,10 @@
 
 namespace ax {
 
-constexpr int SOR_WAVES = 16;                /* four waves per SIMD hide the divide latency
-                                                (30001 points: 1.37 s with 4 waves, 1.04 s with 16) */
-constexpr int SOR_LANES = 64 * SOR_WAVES;    /* sweeps in flight per launch */
-constexpr int SOR_PT = 64;                   /* time steps per phase */
-constexpr int SOR_RING = 3 * SOR_PT;         /* slots: the phase written, and the two read */
+constexpr int SOR_MAX_WAVES = 512;           /* one per SIMD on half the chip */
+constexpr size_t SOR_ROWS_BYTES = (size_t)1 << 30;   /* device memory the rows between waves may take */
+constexpr int SOR_CHUNK = 32;                /* points a wave takes from the row before it at a time */
+constexpr unsigned SOR_SPINS = 1u << 24;     /* polls (some 20 s) before a wave gives the launch up */
 
 struct SorConsts {
   int nx;
@@ -86,81 +86,140 @@ __device__ inline double from_prev_lane(double v, double first) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-/* nb sweeps (nb <= SOR_LANES) from (ip, ia) -> (op, oa); res[L] = the
- * largest |F| of sweep L.  One workgroup of SOR_LANES threads. */
-__global__ void __launch_bounds__(SOR_LANES) sor_kernel(SorConsts k, const double *__restrict__ ip,
-                                                        const double *__restrict__ ia, double *__restrict__ op,
-                                                        double *__restrict__ oa, double *__restrict__ res, int nb) {
-  /* ring[0]: the input sweep, slot s holds point s+2 (a virtual lane -1);
-   * ring[w+1]: lane 63 of wave w, slot s holds its output at time s */
-  __shared__ double2 ring[SOR_WAVES + 1][SOR_RING];
-  const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
-  const int L = (int)threadIdx.x;
-  const int nx = k.nx;
-  const int last = nb - 1;
-  const int s_end = nx - 2 + 2 * last;                  /* last time any sweep works */
-  const int nchunk = (s_end + SOR_PT - 1) / SOR_PT;     /* chunk c: times c*PT+1 .. c*PT+PT */
-  auto mod = [](int s) { return ((s % SOR_RING) + SOR_RING) % SOR_RING; };
+/* What the waves of a launch share besides the rows. */
+struct SorControl {
+  int ticket;     /* waves started */
+  int stop;       /* lowest wave holding a sweep that meets the tolerance */
+  int failed;     /* a wave waited longer than SOR_SPINS polls */
+};
 
-  /* input slots for times -1 .. PT (points 1 .. PT+2) */
-  if (w == 0) {
-    for (int s = lane - 1; s <= SOR_PT; s += 64) {
-      const int j = s + 2;
-      if (j <= nx - 1) ring[0][mod(s)] = make_double2(ip[j], ia[j]);
-    }
-  }
-  if (L == 0) {
+/* "Not written yet" in a row: a signalling NaN, which no arithmetic returns. */
+constexpr unsigned long long kSorUnset = 0x7ff40a5eab5e17edull;
+
+__global__ void __launch_bounds__(256) sor_clear_kernel(unsigned long long *rows, size_t n, SorControl *ctl) {
+  const size_t step = (size_t)gridDim.x * 256;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += step) rows[i] = kSorUnset;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *ctl = {0, 1 << 30, 0};
+}
+
+__device__ __forceinline__ unsigned long long sor_peek(const double *p) {
+  return __hip_atomic_load((const unsigned long long *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int sor_flag(const int *p) {
+  return __builtin_amdgcn_readfirstlane(__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+__device__ __forceinline__ void sor_post(double *p, double v) {
+  __hip_atomic_store((unsigned long long *)p, (unsigned long long)__double_as_longlong(v), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+
+/* nb sweeps from (ip, ia) -> (op, oa); res[L] = the largest |F| of sweep L
+ * (not of the sweeps in waves after one that stops).  Wave w = sweeps 64 w
+ * ... 64 w + 63, in a workgroup of its own; rows[w] takes the last of them,
+ * phi then A, and is what wave w + 1 starts from.  A value is handed over by
+ * itself: the row holds kSorUnset until the producer's relaxed store, and the
+ * consumer polls for it, so no order between two stores matters.  A wave
+ * waits only for the one numbered before it, and numbers are handed out in
+ * the order the waves start, so the lowest waiting wave always has a running
+ * predecessor; the wait is bounded all the same. */
+__global__ void __launch_bounds__(64) sor_kernel(SorConsts k, double tol, const double *__restrict__ ip,
+                                                 const double *__restrict__ ia, double *rows, double *__restrict__ op,
+                                                 double *__restrict__ oa, double *__restrict__ res, int nb,
+                                                 SorControl *ctl) {
+  __shared__ double2 in[SOR_CHUNK];          /* in[t]: the previous sweep at point s0 + 2 + t */
+  const int lane = (int)threadIdx.x;
+  int ticket = 0;
+  if (lane == 0) ticket = atomicAdd(&ctl->ticket, 1);
+  const int w = __builtin_amdgcn_readfirstlane(ticket);
+  const int nx = k.nx, L = 64 * w + lane;
+  const int last = min(63, nb - 1 - 64 * w);             /* this wave's last sweep */
+  const bool final = 64 * w + last == nb - 1;
+  const double *bp = w ? rows + (size_t)2 * (w - 1) * nx : ip, *ba = w ? bp + nx : ia;
+  double *rp = rows + (size_t)2 * w * nx, *ra = rp + nx;
+  if (final && lane == last) {
     op[0] = 0;
     oa[0] = 0;
   }
-  __syncthreads();
-
-  double o1p = 0, o1a = 0, o2p = 0, o2a = 0;            /* own outputs at s-1, s-2 */
+  const bool live = lane <= last;
+  const int s_end = nx - 2 + 2 * last;                   /* last time any sweep works */
+  double o1p = 0, o1a = 0;                               /* own outputs at s-1 */
+  double u1p = 0, u1a = 0;                               /* the previous sweep at point j + 1, j */
   double r = 0;
-  const bool live = L < nb;
-  for (int P = 0; P < nchunk + SOR_WAVES - 1; ++P) {
-    const int c = P - w;
-    if (c >= 0 && c < nchunk) {
-      for (int t = 1; t <= SOR_PT; ++t) {
-        const int s = c * SOR_PT + t;
-        const double2 f1 = ring[w][mod(s - 1)], f2 = ring[w][mod(s - 2)];
-        const double u1p = from_prev_lane(o1p, f1.x), u1a = from_prev_lane(o1a, f1.y);
-        const double u2p = from_prev_lane(o2p, f2.x), u2a = from_prev_lane(o2a, f2.y);
-        const int j = s - 2 * L;
-        double np = o1p, na = o1a;
-        if (live && j >= 1 && j <= nx - 2) {
-          const bool edge = j == nx - 2;              /* phi(nx-1) = phi(nx-2) of the previous sweep */
-          const SorPoint q = sor_point(k, j, j == 1 ? 0.0 : o1p, u2p, edge ? u2p : u1p, j == 1 ? 0.0 : o1a, u2a,
-                                       edge ? u2a : u1a);
-          np = q.phi;
-          na = q.A;
-          if (q.rphi > r) r = q.rphi;
-          if (q.rA > r) r = q.rA;
-          if (L == last) {
-            op[j] = np;
-            oa[j] = na;
+  /* point j of the row before, as raw bits; what is not needed reads as 0 */
+  auto need = [&](int j) { return lane < SOR_CHUNK && j <= nx - 2; };
+  unsigned long long np = 0, na = 0;
+  auto fetch = [&](int j) {
+    np = na = 0;
+    if (need(j)) {
+      np = sor_peek(bp + j);
+      na = sor_peek(ba + j);
+    }
+  };
+  /* true when every needed value has arrived */
+  auto settle = [&](int j) {
+    for (unsigned n = 0;; ++n) {
+      const bool wait = need(j) && w && (np == kSorUnset || na == kSorUnset);
+      if (__builtin_amdgcn_ballot_w64(wait) == 0) return true;
+      if ((n & 63) == 63) {
+        const bool over = n > SOR_SPINS;
+        if (over && lane == 0) __hip_atomic_store(&ctl->failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (over || sor_flag(&ctl->failed) || sor_flag(&ctl->stop) < w) return false;
+      }
+      __builtin_amdgcn_s_sleep(2);
+      fetch(j);
+    }
+  };
+  /* point 1: u1 at time 0 */
+  fetch(1 + lane);
+  if (!settle(1 + lane)) return;
+  u1p = __longlong_as_double((long long)__shfl((long long)np, 0, 64));
+  u1a = __longlong_as_double((long long)__shfl((long long)na, 0, 64));
+  if (lane) u1p = u1a = 0;
+  fetch(2 + lane);
+  for (int s0 = 0; s0 < s_end; s0 += SOR_CHUNK) {
+    if (!settle(s0 + 2 + lane)) return;
+    if (lane < SOR_CHUNK)
+      in[lane] = make_double2(__longlong_as_double((long long)np), __longlong_as_double((long long)na));
+    __syncthreads();
+    /* the next chunk's values, and whether a wave before this one stops */
+    fetch(s0 + SOR_CHUNK + 2 + lane);
+    const bool stopped = sor_flag(&ctl->stop) < w;
+    for (int t = 0; t < SOR_CHUNK; ++t) {
+      const int s = s0 + 1 + t, j = s - 2 * lane;
+      const double2 f = in[t];
+      /* at point j + 1 the previous lane's output of the last time step; at
+       * point j the one before, which is the last time's u1 */
+      const double u2p = u1p, u2a = u1a;
+      u1p = from_prev_lane(o1p, f.x);
+      u1a = from_prev_lane(o1a, f.y);
+      if (live && j >= 1 && j <= nx - 2) {
+        const bool edge = j == nx - 2;              /* phi(nx-1) = phi(nx-2) of the previous sweep */
+        const SorPoint q = sor_point(k, j, j == 1 ? 0.0 : o1p, u2p, edge ? u2p : u1p, j == 1 ? 0.0 : o1a, u2a,
+                                     edge ? u2a : u1a);
+        o1p = q.phi;
+        o1a = q.A;
+        if (q.rphi > r) r = q.rphi;
+        if (q.rA > r) r = q.rA;
+        if (lane == last) {
+          if (final) {
+            op[j] = o1p;
+            oa[j] = o1a;
             if (edge) {
               op[nx - 1] = u2p;
               oa[nx - 1] = u2a;
             }
+          } else {
+            sor_post(rp + j, o1p);
+            sor_post(ra + j, o1a);
           }
         }
-        o2p = o1p;
-        o2a = o1a;
-        o1p = np;
-        o1a = na;
-        if (lane == 63) ring[w + 1][mod(s)] = make_double2(np, na);
       }
     }
-    /* wave 0 stages the input for its next chunk (slots of chunk c-2) */
-    if (w == 0 && P + 1 < nchunk) {
-      const int s = (P + 1) * SOR_PT + 1 + lane;
-      const int j = s + 2;
-      if (j <= nx - 1) ring[0][mod(s)] = make_double2(ip[j], ia[j]);
-    }
+    if (stopped) return;
     __syncthreads();
   }
   if (live) res[L] = r;
+  if (__builtin_amdgcn_ballot_w64(live && !(r > tol)) && lane == 0) atomicMin(&ctl->stop, w);
 }
 
 /* straight_ic.cpp:63-134 at one (x, y): phi and the gauge field A */
@@ -319,11 +378,21 @@ int ax_sor_profile(const ax_sor_params *p, const double *init, double *out, int3
     k.half_lam = 0.5 * p->lambda;
     k.eta2 = p->eta * p->eta;
 
-    DevBuf buf, dres;
+    /* waves per launch, as many as the sweeps and the rows' memory allow (at
+     * least 4, as fast as one workgroup of 16 waves would be) */
+    int waves = (int)std::min<long long>(SOR_MAX_WAVES, ((long long)p->max_iter + 63) / 64);
+    waves = (int)std::min<size_t>(waves, std::max<size_t>(4, SOR_ROWS_BYTES / ((size_t)16 * nx)));
+    DevBuf buf, rows, dres;
     hipError_t e = hipMalloc(&buf.p, (size_t)4 * nx * sizeof(double));
     if (e != hipSuccess) return hip_fail(e, "hipMalloc profile");
-    e = hipMalloc(&dres.p, SOR_LANES * sizeof(double));
+    while ((e = hipMalloc(&rows.p, (size_t)2 * waves * nx * sizeof(double))) != hipSuccess && waves > 1) {
+      (void)hipGetLastError();   /* clear the sticky error of the failed call */
+      waves /= 2;
+    }
+    if (e != hipSuccess) return hip_fail(e, "hipMalloc sweep rows");
+    e = hipMalloc(&dres.p, (size_t)64 * waves * sizeof(double) + sizeof(SorControl));
     if (e != hipSuccess) return hip_fail(e, "hipMalloc residuals");
+    SorControl *ctl = (SorControl *)(dres.p + (size_t)64 * waves);
     double *inp = buf.p, *ina = buf.p + nx, *outp = buf.p + 2 * (size_t)nx, *outa = buf.p + 3 * (size_t)nx;
     hipStream_t st;
     e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
@@ -335,14 +404,25 @@ int ax_sor_profile(const ax_sor_params *p, const double *init, double *out, int3
     e = hipMemcpyAsync(inp, hp.data(), nx * sizeof(double), hipMemcpyHostToDevice, st);
     if (e == hipSuccess) e = hipMemcpyAsync(ina, ha.data(), nx * sizeof(double), hipMemcpyHostToDevice, st);
     if (e != hipSuccess) return hip_fail(e, "upload profile");
-    std::vector<double> hres(SOR_LANES);
+    std::vector<double> hres((size_t)64 * waves);
+    /* n sweeps from (fp, fa) into (outp, outa), their residuals into hres */
+    auto sweep = [&](const double *fp, const double *fa, double *between, int n) -> int {
+      const int nw = (n + 63) / 64;
+      const size_t cells = (size_t)2 * (nw - 1) * nx;
+      const unsigned cb = (unsigned)std::min<size_t>(2048, cells / 256 + 1);
+      hipLaunchKernelGGL(sor_clear_kernel, dim3(cb), dim3(256), 0, st, (unsigned long long *)between, cells, ctl);
+      hipLaunchKernelGGL(sor_kernel, dim3(nw), dim3(64), 0, st, k, p->tol, fp, fa, between, outp, outa, dres.p, n, ctl);
+      SorControl done;
+      hipError_t er = hipGetLastError();
+      if (er == hipSuccess) er = hipMemcpyAsync(hres.data(), dres.p, n * sizeof(double), hipMemcpyDeviceToHost, st);
+      if (er == hipSuccess) er = hipMemcpyAsync(&done, ctl, sizeof done, hipMemcpyDeviceToHost, st);
+      if (er == hipSuccess) er = hipStreamSynchronize(st);
+      if (er != hipSuccess) return hip_fail(er, "SOR sweeps");
+      return done.failed ? fail(AX_EHIP, "SOR sweeps: a wave waited too long for the one before it") : AX_OK;
+    };
     while (iters < p->max_iter) {
-      const int nb = std::min(SOR_LANES, p->max_iter - iters);
-      hipLaunchKernelGGL(sor_kernel, dim3(1), dim3(SOR_LANES), 0, st, k, inp, ina, outp, outa, dres.p, nb);
-      e = hipGetLastError();
-      if (e == hipSuccess) e = hipMemcpyAsync(hres.data(), dres.p, nb * sizeof(double), hipMemcpyDeviceToHost, st);
-      if (e == hipSuccess) e = hipStreamSynchronize(st);
-      if (e != hipSuccess) return hip_fail(e, "SOR sweeps");
+      const int nb = std::min(64 * waves, p->max_iter - iters);
+      if ((rc = sweep(inp, ina, rows.p, nb)) != AX_OK) return rc;
       int stop = -1;
       for (int l = 0; l < nb; ++l)
         if (!(hres[l] > p->tol)) {
@@ -350,14 +430,15 @@ int ax_sor_profile(const ax_sor_params *p, const double *init, double *out, int3
           break;
         }
       if (stop >= 0) {
+        tol_test = hres[stop];
         if (stop < nb - 1) {
-          hipLaunchKernelGGL(sor_kernel, dim3(1), dim3(SOR_LANES), 0, st, k, inp, ina, outp, outa, dres.p, stop + 1);
-          e = hipGetLastError();
-          if (e == hipSuccess) e = hipStreamSynchronize(st);
-          if (e != hipSuccess) return hip_fail(e, "SOR sweeps");
+          /* the stopping sweep's own wave again, from the row before it; the
+           * row it was in the launch's last place for is free */
+          const int w = stop / 64;
+          const double *fp = w ? rows.p + (size_t)2 * (w - 1) * nx : inp, *fa = w ? fp + nx : ina;
+          if ((rc = sweep(fp, fa, rows.p + (size_t)2 * w * nx, stop % 64 + 1)) != AX_OK) return rc;
         }
         iters += stop + 1;
-        tol_test = hres[stop];
         std::swap(inp, outp);
         std::swap(ina, outa);
         break;

@@ -174,3 +174,22 @@ def test_straight_string_rejects_moore_and_bad_profiles():
             lat.init_straight_string(prof[:1], 0.1)
         with pytest.raises(ax.AxError):
             lat.init_straight_string(prof, 0.0)
+
+
+@pytest.mark.parametrize("sweeps", [1, 63, 64, 65, 128, 700])
+@pytest.mark.parametrize("nx", [3, 4, 32, 35, 66, 200])
+def test_sor_wave_edges(nx, sweeps):
+    """Sweeps around whole waves of 64, grids shorter and longer than a chunk
+    and than a wave's span: against the oracle, stopping at the cap and at a
+    tolerance that a sweep in the middle of the launch meets."""
+    say(f"[sor-waves] nx={nx} sweeps={sweeps}")
+    args = (0.08, 1.4)
+    ref, it, res = orc.sor_profile(nx, *args, 0.0, 1.0, 1.3, 0.9, 0.5, sweeps)
+    prof, gi, gr = ax.sor_profile(nx=nx, h=args[0], w=args[1], tol=0.0, n=1.0, lam=1.3, eta=0.9, g=0.5, max_iter=sweeps)
+    assert (gi, gr) == (it, res)
+    assert np.array_equal(prof.view(np.uint64), ref.view(np.uint64))
+    _, _, tol = orc.sor_profile(nx, *args, 0.0, 1.0, 1.3, 0.9, 0.5, max(1, sweeps // 2))
+    ref, it, res = orc.sor_profile(nx, *args, tol, 1.0, 1.3, 0.9, 0.5, sweeps)
+    prof, gi, gr = ax.sor_profile(nx=nx, h=args[0], w=args[1], tol=tol, n=1.0, lam=1.3, eta=0.9, g=0.5, max_iter=sweeps)
+    assert (gi, gr) == (it, res) and it <= sweeps
+    assert np.array_equal(prof.view(np.uint64), ref.view(np.uint64))
