@@ -106,9 +106,11 @@ struct ax_lattice {
   int device = 0;
   hipStream_t stream = nullptr;
   void *state = nullptr;
-  double *part = nullptr;   /* 3 doubles per reduction block (diag_part_blocks) */
-  double *dres = nullptr;   /* small device results */
-  double *hres = nullptr;   /* pinned host copy */
+  /* 3 doubles per reduction block, twice (diag_part_blocks each): the energy
+   * and Gauss sums' and the windings' */
+  double *part = nullptr;
+  size_t part_n = 0;
+  double *hres = nullptr;   /* pinned host memory the reductions write their results to */
   int8_t *wind = nullptr;
   float *phase = nullptr;   /* FP32 edge values [3][V] of the marching diagnostics (ax_wind.h) */
   int *bcount = nullptr;
@@ -121,7 +123,7 @@ struct ax_lattice {
   int div_for = -1;         /* the TimeStep whose diagnostics divb serves (-1: none) */
   double *fpart = nullptr;  /* fused diagnostics: partial sums per step work item */
   size_t fpart_n = 0;
-  double *fres = nullptr;   /* fused diagnostics: 8 doubles per diagnostic point */
+  double *fres = nullptr;   /* fused diagnostics: 8 doubles per diagnostic point, pinned host memory as hres */
   size_t fres_n = 0;
   int band_steps = 0;       /* marching steps since the state or TimeStep was last set from the host */
   bool timing = false;                         /* ax_kernel_timer */
@@ -235,9 +237,8 @@ int ax_create(const ax_params *p, ax_lattice **out) {
     return hip_fail(e, "hipStreamCreate");
   }
   const size_t bytes = (size_t)L->ncomp * 2 * L->pitch * L->esize;
-  const size_t nb = diag_part_blocks(*p);
-  if (hipMalloc(&L->state, bytes) != hipSuccess || hipMalloc((void **)&L->part, 3 * nb * sizeof(double)) != hipSuccess ||
-      hipMalloc((void **)&L->dres, 16 * sizeof(double)) != hipSuccess ||
+  const size_t nb = L->part_n = diag_part_blocks(*p);
+  if (hipMalloc(&L->state, bytes) != hipSuccess || hipMalloc((void **)&L->part, 6 * nb * sizeof(double)) != hipSuccess ||
       (p->model == AX_MODEL_MOORE && hipMalloc((void **)&L->band, 3 * sizeof(int)) != hipSuccess) ||
       hipHostMalloc((void **)&L->hres, 16 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();   /* clear the sticky error of the failed call */
@@ -262,11 +263,10 @@ void ax_destroy(ax_lattice *L) {
   }
   if (L->state) (void)hipFree(L->state);
   if (L->part) (void)hipFree(L->part);
-  if (L->dres) (void)hipFree(L->dres);
   if (L->band) (void)hipFree(L->band);
   if (L->divb) (void)hipFree(L->divb);
   if (L->fpart) (void)hipFree(L->fpart);
-  if (L->fres) (void)hipFree(L->fres);
+  if (L->fres) (void)hipHostFree(L->fres);
   if (L->hres) (void)hipHostFree(L->hres);
   if (L->wind) (void)hipFree(L->wind);
   if (L->phase) (void)hipFree(L->phase);
@@ -536,43 +536,43 @@ int ax_diagnostics(ax_lattice *L, int32_t want_winding, ax_diag *out) {
   if (!L || !out) return fail(AX_EINVAL, "NULL argument");
   const ax_params &p = L->p;
   const bool glob = p.model == AX_MODEL_GLOBAL;
-  hipError_t e;
-  bool march = false, mwind = false;
+  hipError_t e = hipSuccess;
+  Partials sums = {L->part, 0}, winds = {L->part + 3 * L->part_n, 0};
+  bool mwind = false;
   if (glob) {
     /* the energy leapfrog.cpp prints for the last TimeStep (its pre-step
      * field is still in the other buffer); none before the first step */
     if (L->timestep > 0)
-      e = L->esize == 8 ? launch_global_energy<double>(p, L->state, L->pitch, L->timestep - 1, L->part, L->dres, L->stream)
-                        : launch_global_energy<float>(p, L->state, L->pitch, L->timestep - 1, L->part, L->dres, L->stream);
-    else
-      e = hipMemsetAsync(L->dres, 0, 3 * sizeof(double), L->stream);
+      e = L->esize == 8 ? launch_global_energy<double>(p, L->state, L->pitch, L->timestep - 1, sums, L->stream)
+                        : launch_global_energy<float>(p, L->state, L->pitch, L->timestep - 1, sums, L->stream);
   } else {
     DiagConsts k = diag_consts(&p);
     int rc = prepare_faces(L);
     if (rc) return rc;
-    march = use_diag_march(p);
+    const bool march = use_diag_march(p);
     /* the windings come from the march's edge values, else from
      * launch_winding_field */
     mwind = want_winding && march && ensure_phase_buffer(L) == AX_OK;
     if (march)
-      e = launch_march_diag(L, mwind);
+      e = launch_march_diag(L, mwind, sums);
     else if (L->esize == 8)
-      e = launch_diag<double>(k, levels_of<double>(L, L->timestep), L->part, L->dres, L->stream);
+      e = launch_diag<double>(k, levels_of<double>(L, L->timestep), sums, L->stream);
     else
-      e = launch_diag<float>(k, levels_of<float>(L, L->timestep), L->part, L->dres, L->stream);
+      e = launch_diag<float>(k, levels_of<float>(L, L->timestep), sums, L->stream);
   }
   if (e != hipSuccess) return hip_fail(e, "diag launch");
   if (want_winding) {
     /* only the count is returned: the march stores no winding field */
     if (mwind) {
-      e = launch_phase_winding(L, nullptr, L->dres + 4);
+      e = launch_phase_winding(L, nullptr, winds);
       if (e != hipSuccess) return hip_fail(e, "winding launch");
     } else {
-      int rc = launch_winding_field(L, 0, nullptr, L->part, L->dres + 4);
+      int rc = launch_winding_field(L, 0, nullptr, winds);
       if (rc) return rc;
     }
   }
-  e = hipMemcpyAsync(L->hres, L->dres, 8 * sizeof(double), hipMemcpyDeviceToHost, L->stream);
+  if (sums.n || winds.n) e = launch_sums(sums, L->hres, winds, L->hres + 4, L->stream);
+  else L->hres[0] = L->hres[1] = L->hres[2] = 0;   /* a global lattice before its first step */
   if (e == hipSuccess) e = hipStreamSynchronize(L->stream);
   if (e != hipSuccess) return hip_fail(e, "diag readback");
   fill_diag(L, L->hres, L->timestep, want_winding != 0, out);
@@ -611,7 +611,16 @@ static int ensure_fused(ax_lattice *L, size_t npoints) {
   size_t have_div = L->divb ? L->V : 0;
   int rc = grow(&L->divb, &have_div, L->V, "divergence buffer");
   if (!rc) rc = grow(&L->fpart, &L->fpart_n, 3 * items, "partial sums");
-  if (!rc) rc = grow(&L->fres, &L->fres_n, 8 * (npoints ? npoints : 1), "diagnostic results");
+  if (!rc && L->fres_n < 8 * npoints) {
+    if (L->fres) (void)hipHostFree(L->fres);   /* the last call waited for its results */
+    L->fres = nullptr;
+    L->fres_n = 0;
+    if (hipHostMalloc((void **)&L->fres, 8 * npoints * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      return fail(AX_ENOMEM, "diagnostic results of %zu points", npoints);
+    }
+    L->fres_n = 8 * npoints;
+  }
   if (!rc) rc = ensure_phase_buffer(L);
   return rc;
 }
@@ -639,9 +648,11 @@ static int launch_fused(ax_lattice *L, int mode, size_t k, bool winding) {
     e = launch_step_fused(sk, lv, L->xseg, L->stream, mode, diag_pow2(p.dx, p.dy, p.dz, p.g), fd);
   if (e == hipSuccess && mode == 2) {
     double *res = L->fres + 8 * k;
-    e = launch_sum3(L->fpart, fused_work_items(p.nx, p.ny, p.nz, L->xseg), res, L->stream);
+    const Partials sums = {L->fpart, fused_work_items(p.nx, p.ny, p.nz, L->xseg)};
+    Partials winds = {L->part + 3 * L->part_n, 0};
     /* windings of level n: its links are intact until the next step */
-    if (e == hipSuccess && winding) e = launch_phase_winding(L, nullptr, res + 4);
+    if (winding) e = launch_phase_winding(L, nullptr, winds);
+    if (e == hipSuccess) e = launch_sums(sums, res, winds, res + 4, L->stream);
   }
   if (e != hipSuccess) return hip_fail(e, "fused step launch");
   L->div_for = mode == 1 ? n + 1 : -1;
@@ -722,17 +733,9 @@ int ax_step_diag(ax_lattice *L, int32_t nsteps, int32_t every, int32_t want_wind
     L->timestep++;
   }
   rc = plain_steps(L, run);
+  if (!rc) rc = ax_sync(L);   /* the results, and the steps after the last output too */
   if (rc) return rc;
-  if (k) {
-    std::vector<double> h(8 * k);
-    hipError_t e = hipMemcpyAsync(h.data(), L->fres, 8 * k * sizeof(double), hipMemcpyDeviceToHost, L->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(L->stream);
-    if (e != hipSuccess) return hip_fail(e, "diagnostic readback");
-    for (size_t j = 0; j < k; ++j) fill_diag(L, &h[8 * j], at[j], want_winding != 0, &out[j]);
-  } else {
-    rc = ax_sync(L);
-    if (rc) return rc;
-  }
+  for (size_t j = 0; j < k; ++j) fill_diag(L, L->fres + 8 * j, at[j], want_winding != 0, &out[j]);
   *count = k;
   return AX_OK;
 }
@@ -745,7 +748,8 @@ int ax_winding_field(ax_lattice *L, int32_t field, int8_t *out, size_t n) {
   if (field < 0 || field > (L->p.model == AX_MODEL_MOORE ? 1 : 0)) return fail(AX_EINVAL, "field %d", field);
   int rc = ensure_winding_buffer(L);
   if (!rc) rc = prepare_faces(L);
-  if (!rc) rc = launch_winding_field(L, field, L->wind, L->part, L->dres + 4);
+  Partials winds = {L->part + 3 * L->part_n, 0};
+  if (!rc) rc = launch_winding_field(L, field, L->wind, winds);
   if (rc) return rc;
   hipError_t e = hipMemcpyAsync(out, L->wind, n, hipMemcpyDeviceToHost, L->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(L->stream);
@@ -847,19 +851,19 @@ int ensure_phase_buffer(ax_lattice *L) {
 }
 
 /* energy/Gauss (and, with phases, the edge phases) of the current level */
-hipError_t launch_march_diag(ax_lattice *L, bool phases) {
+hipError_t launch_march_diag(ax_lattice *L, bool phases, Partials &part) {
   const DiagConsts k = diag_consts(&L->p);
   float *ph = phases ? L->phase : nullptr;
-  return L->esize == 8 ? launch_diag_march<double>(k, levels_of<double>(L, L->timestep), ph, L->part, L->dres, L->stream)
-                       : launch_diag_march<float>(k, levels_of<float>(L, L->timestep), ph, L->part, L->dres, L->stream);
+  return L->esize == 8 ? launch_diag_march<double>(k, levels_of<double>(L, L->timestep), ph, part, L->stream)
+                       : launch_diag_march<float>(k, levels_of<float>(L, L->timestep), ph, part, L->stream);
 }
 
 /* windings of the current level from the edge values launch_march_diag
  * stored */
-hipError_t launch_phase_winding(ax_lattice *L, int8_t *out, double *res3) {
+hipError_t launch_phase_winding(ax_lattice *L, int8_t *out, Partials &part) {
   const ax_params &p = L->p;
   return launch_wind_phase(p.nx, p.ny, p.nz, p.boundary != AX_BC_PERIODIC, p.boundary_z != AX_BC_PERIODIC, L->phase, out,
-                           L->part, res3, L->stream);
+                           part, L->stream);
 }
 
 int ensure_winding_buffer(ax_lattice *L) {
@@ -871,7 +875,7 @@ int ensure_winding_buffer(ax_lattice *L) {
   return AX_OK;
 }
 
-int launch_winding_field(ax_lattice *L, int field, int8_t *out, double *part, double *res3) {
+int launch_winding_field(ax_lattice *L, int field, int8_t *out, Partials &part) {
   const ax_params &p = L->p;
   const bool glob = p.model == AX_MODEL_GLOBAL;
   const int tN = glob ? L->timestep % 2 : (L->timestep + 1) % 2;
@@ -891,11 +895,11 @@ int launch_winding_field(ax_lattice *L, int field, int8_t *out, double *part, do
     if (L->esize == 8) {
       const double *b = (const double *)L->state;
       e = launch_edge_winding<double>(p.nx, p.ny, p.nz, ex, ez, b + P(c0), b + P(c0 + 1), b + P(t0), b + P(t0 + 1),
-                                      b + P(t0 + 2), q, L->phase, out, part, res3, L->stream);
+                                      b + P(t0 + 2), q, L->phase, out, part, L->stream);
     } else {
       const float *b = (const float *)L->state;
       e = launch_edge_winding<float>(p.nx, p.ny, p.nz, ex, ez, b + P(c0), b + P(c0 + 1), b + P(t0), b + P(t0 + 1),
-                                     b + P(t0 + 2), q, L->phase, out, part, res3, L->stream);
+                                     b + P(t0 + 2), q, L->phase, out, part, L->stream);
     }
     return e == hipSuccess ? AX_OK : hip_fail(e, "winding launch");
   }
@@ -907,11 +911,11 @@ int launch_winding_field(ax_lattice *L, int field, int8_t *out, double *part, do
   if (L->esize == 8) {
     const double *b = (const double *)L->state;
     e = launch_winding<double>(p.nx, p.ny, p.nz, b + P(c0), b + P(c0 + 1), b + P(t0), b + P(t0 + 1), b + P(t0 + 2), q,
-                               ex, ez, out, part, res3, L->stream);
+                               ex, ez, out, part, L->stream);
   } else {
     const float *b = (const float *)L->state;
     e = launch_winding<float>(p.nx, p.ny, p.nz, b + P(c0), b + P(c0 + 1), b + P(t0), b + P(t0 + 1), b + P(t0 + 2), q,
-                              ex, ez, out, part, res3, L->stream);
+                              ex, ez, out, part, L->stream);
   }
   return e == hipSuccess ? AX_OK : hip_fail(e, "winding launch");
 }

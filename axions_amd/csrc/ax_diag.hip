@@ -214,14 +214,20 @@ __global__ void __launch_bounds__(256) diag_kernel(DiagConsts k, Levels<T> L, in
   }
 }
 
-/* One block sums nb triples: thread t adds blocks t, t+1024, ... in order,
- * then a fixed tree; deterministic for a given nb. */
-__global__ void __launch_bounds__(1024) sum3_kernel(const double *part, int nb, double *out) {
+/* One block sums the na triples of a, and a second block the nb of b where
+ * there are any: thread t adds triples t, t+1024, ... in order, then a fixed
+ * tree; deterministic for a given number.  The results may go straight to
+ * pinned host memory. */
+__global__ void __launch_bounds__(1024) sum3_kernel(const double *a, int na, double *outa, const double *b, int nb,
+                                                    double *outb) {
   __shared__ double sh[3][16];
+  const double *part = blockIdx.x ? b : a;
+  double *out = blockIdx.x ? outb : outa;
+  const int n = blockIdx.x ? nb : na;
   double v[3] = {0, 0, 0};
 #pragma unroll 4
-  for (int i = threadIdx.x; i < nb; i += 1024)
-    for (int c = 0; c < 3; ++c) v[c] += part[3 * i + c];
+  for (int i = threadIdx.x; i < n; i += 1024)
+    for (int c = 0; c < 3; ++c) v[c] += part[3 * (size_t)i + c];
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   for (int c = 0; c < 3; ++c) {
     double x = wave_sum(v[c]);
@@ -928,32 +934,31 @@ __global__ void __launch_bounds__(64, sizeof(T) == 8 ? 3 : 1) moore_diag_march_k
 
 /* ------------------------------ launchers ------------------------------- */
 template <typename T>
-hipError_t launch_diag(const DiagConsts &k, const Levels<T> &L, double *part, double *out3, hipStream_t st) {
+hipError_t launch_diag(const DiagConsts &k, const Levels<T> &L, Partials &part, hipStream_t st) {
   const int V = k.nx * k.ny * k.nz;
   int nb = (V + kDiagSitesPerBlock - 1) / kDiagSitesPerBlock;
   if (k.model == AX_MODEL_AH) {
-    hipLaunchKernelGGL((diag_kernel<T, AX_MODEL_AH>), dim3(nb), dim3(256), 0, st, k, L, V, part);
+    hipLaunchKernelGGL((diag_kernel<T, AX_MODEL_AH>), dim3(nb), dim3(256), 0, st, k, L, V, part.p);
   } else if (getenv("AX_DIAG_SITE_KERNEL") == nullptr) {
     /* part holds 3 doubles per work item (diag_part_blocks) */
     const TileGrid g = make_tile_grid(k.nx, k.ny, k.nz, diag_xseg(k.nx, k.ny, k.nz));
-    hipLaunchKernelGGL((moore_diag_march_kernel<T>), dim3(g.work), dim3(64), 0, st, k, L, g, part);
+    hipLaunchKernelGGL((moore_diag_march_kernel<T>), dim3(g.work), dim3(64), 0, st, k, L, g, part.p);
     nb = g.work;
   } else {
-    hipLaunchKernelGGL((diag_kernel<T, AX_MODEL_MOORE>), dim3(nb), dim3(256), 0, st, k, L, V, part);
+    hipLaunchKernelGGL((diag_kernel<T, AX_MODEL_MOORE>), dim3(nb), dim3(256), 0, st, k, L, V, part.p);
   }
-  hipLaunchKernelGGL(sum3_kernel, dim3(1), dim3(1024), 0, st, part, nb, out3);
+  part.n = nb;
   return hipGetLastError();
 }
 
 template <typename T>
 hipError_t launch_winding(int nx, int ny, int nz, const T *fr, const T *fi, const T *tx, const T *ty,
-                          const T *tz, double q, int ex, int ez, int8_t *out, double *part, double *out1,
-                          hipStream_t st) {
+                          const T *tz, double q, int ex, int ez, int8_t *out, Partials &part, hipStream_t st) {
   const int V = nx * ny * nz;
   const int nb = (V + kSitesPerBlock - 1) / kSitesPerBlock;
   hipLaunchKernelGGL((winding_kernel<T>), dim3(nb), dim3(256), 0, st, nx, ny, nz, fr, fi, tx, ty, tz, q, ex, ez,
-                     out, part);
-  hipLaunchKernelGGL(sum3_kernel, dim3(1), dim3(1024), 0, st, part, nb, out1);
+                     out, part.p);
+  part.n = nb;
   return hipGetLastError();
 }
 
@@ -998,35 +1003,33 @@ __global__ void __launch_bounds__(64) edge_march_kernel(int nx, int ny, int nz, 
 
 template <typename T>
 hipError_t launch_edge_winding(int nx, int ny, int nz, int ex, int ez, const T *fr, const T *fi, const T *tx,
-                               const T *ty, const T *tz, double q, float *E, int8_t *out, double *part, double *out3,
-                               hipStream_t st) {
+                               const T *ty, const T *tz, double q, float *E, int8_t *out, Partials &part, hipStream_t st) {
   const TileGrid g = make_tile_grid(nx, ny, nz, diag_xseg(nx, ny, nz));
   hipLaunchKernelGGL((edge_march_kernel<T>), dim3(g.work), dim3(64), 0, st, nx, ny, nz, fr, fi, tx, ty, tz, q, g,
                      E);
   hipError_t e = hipGetLastError();
-  return e == hipSuccess ? launch_wind_phase(nx, ny, nz, ex, ez, E, out, part, out3, st) : e;
+  return e == hipSuccess ? launch_wind_phase(nx, ny, nz, ex, ez, E, out, part, st) : e;
 }
 
 template <typename T>
-hipError_t launch_diag_march(const DiagConsts &k, const Levels<T> &L, float *phase, double *part, double *out3,
-                             hipStream_t st) {
+hipError_t launch_diag_march(const DiagConsts &k, const Levels<T> &L, float *phase, Partials &part, hipStream_t st) {
   const TileGrid g = make_tile_grid(k.nx, k.ny, k.nz, diag_xseg(k.nx, k.ny, k.nz));
   /* without a gauge coupling the pass divides by dx, dy, dz alone
    * (energy_form 0 leaves out the gauge terms) */
   const bool p2 = diag_pow2(k.dx, k.dy, k.dz, k.g == 0 && k.energy_form == 0 ? 1.0 : k.g);
 #define AX_DM(PH, P2) \
-  hipLaunchKernelGGL((diag_march_kernel<T, PH, P2>), dim3(g.work), dim3(64), 0, st, k, L, g, phase, part)
+  hipLaunchKernelGGL((diag_march_kernel<T, PH, P2>), dim3(g.work), dim3(64), 0, st, k, L, g, phase, part.p)
   if (phase && p2) AX_DM(true, true);
   else if (phase) AX_DM(true, false);
   else if (p2) AX_DM(false, true);
   else AX_DM(false, false);
 #undef AX_DM
-  hipLaunchKernelGGL(sum3_kernel, dim3(1), dim3(1024), 0, st, part, g.work, out3);
+  part.n = g.work;
   return hipGetLastError();
 }
 
-hipError_t launch_sum3(const double *part, int nb, double *out3, hipStream_t st) {
-  hipLaunchKernelGGL(sum3_kernel, dim3(1), dim3(1024), 0, st, part, nb, out3);
+hipError_t launch_sums(const Partials &a, double *out3, const Partials &b, double *outb3, hipStream_t st) {
+  hipLaunchKernelGGL(sum3_kernel, dim3(b.n ? 2 : 1), dim3(1024), 0, st, a.p, a.n, out3, b.p, b.n, outb3);
   return hipGetLastError();
 }
 
@@ -1063,26 +1066,26 @@ bool diag_pow2(double dx, double dy, double dz, double gg) {
   return p2;
 }
 
-hipError_t launch_wind_phase(int nx, int ny, int nz, int ex, int ez, const float *E, int8_t *out, double *part,
-                             double *out3, hipStream_t st) {
+hipError_t launch_wind_phase(int nx, int ny, int nz, int ex, int ez, const float *E, int8_t *out, Partials &part,
+                             hipStream_t st) {
   /* part holds 3 doubles per work item (diag_part_blocks) */
   const TileGrid g = make_tile_grid(nx, ny, nz, diag_xseg(nx, ny, nz));
-  hipLaunchKernelGGL(wind_march_kernel, dim3(g.work), dim3(64), 0, st, nx, ny, nz, E, g, ex, ez, out, part);
-  hipLaunchKernelGGL(sum3_kernel, dim3(1), dim3(1024), 0, st, part, g.work, out3);
+  hipLaunchKernelGGL(wind_march_kernel, dim3(g.work), dim3(64), 0, st, nx, ny, nz, E, g, ex, ez, out, part.p);
+  part.n = g.work;
   return hipGetLastError();
 }
 
-#define AX_INST(T)                                                                                          \
-  template hipError_t launch_diag<T>(const DiagConsts &, const Levels<T> &, double *, double *, hipStream_t); \
-  template hipError_t launch_winding<T>(int, int, int, const T *, const T *, const T *, const T *, const T *,  \
-                                        double, int, int, int8_t *, double *, double *, hipStream_t);        \
-  template hipError_t launch_crossings<T>(int, int, int, double, double, double, const T *, const T *, int,   \
-                                          int, int *, long long *, long long *, double *, long long,          \
-                                          hipStream_t, bool);                                               \
-  template hipError_t launch_diag_march<T>(const DiagConsts &, const Levels<T> &, float *, double *, double *, \
-                                           hipStream_t);                                          \
-  template hipError_t launch_edge_winding<T>(int, int, int, int, int, const T *, const T *, const T *, const T *,      \
-                                             const T *, double, float *, int8_t *, double *, double *,      \
+#define AX_INST(T)                                                                                             \
+  template hipError_t launch_diag<T>(const DiagConsts &, const Levels<T> &, Partials &, hipStream_t);           \
+  template hipError_t launch_winding<T>(int, int, int, const T *, const T *, const T *, const T *, const T *,   \
+                                        double, int, int, int8_t *, Partials &, hipStream_t);                   \
+  template hipError_t launch_crossings<T>(int, int, int, double, double, double, const T *, const T *, int,     \
+                                          int, int *, long long *, long long *, double *, long long,            \
+                                          hipStream_t, bool);                                                   \
+  template hipError_t launch_diag_march<T>(const DiagConsts &, const Levels<T> &, float *, Partials &,          \
+                                           hipStream_t);                                                        \
+  template hipError_t launch_edge_winding<T>(int, int, int, int, int, const T *, const T *, const T *,          \
+                                             const T *, const T *, double, float *, int8_t *, Partials &,       \
                                              hipStream_t);
 AX_INST(double)
 AX_INST(float)

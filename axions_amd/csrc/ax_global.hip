@@ -353,8 +353,8 @@ hipError_t launch_global_step(const ax_params &p, void *state, size_t pitch, int
 }
 
 template <typename R>
-hipError_t launch_global_energy(const ax_params &p, const void *state, size_t pitch, int n, double *part,
-                                double *out3, hipStream_t st) {
+hipError_t launch_global_energy(const ax_params &p, const void *state, size_t pitch, int n, Partials &part,
+                                hipStream_t st) {
   const R *b = (const R *)state;
   const int cur = n % 2, nw = 1 - cur;   /* the pre-step field of TimeStep n and its result */
   const GlobalGeom g = geom_of(p);
@@ -363,22 +363,21 @@ hipError_t launch_global_energy(const ax_params &p, const void *state, size_t pi
 #define AX_GE(P2, W)                                                                                              \
   hipLaunchKernelGGL((global_energy_kernel<R, P2, W>), grid, block, 0, st, g, k, b + (size_t)cur * pitch,          \
                      b + (size_t)(2 + cur) * pitch, b + (size_t)nw * pitch, b + (size_t)(2 + nw) * pitch, b + 4 * pitch, \
-                     b + 5 * pitch, part)
+                     b + 5 * pitch, part.p)
   const bool p2 = pow2_of(k);
   if (p2 && g.wide) AX_GE(true, 2);
   else if (p2) AX_GE(true, 1);
   else if (g.wide) AX_GE(false, 2);
   else AX_GE(false, 1);
 #undef AX_GE
-  const hipError_t e = hipGetLastError();
-  return e == hipSuccess ? launch_sum3(part, 8 * g.eper, out3, st) : e;
+  part.n = (int)(8 * g.eper);
+  return hipGetLastError();
 }
 
 template hipError_t launch_global_step<double>(const ax_params &, void *, size_t, int, hipStream_t);
 template hipError_t launch_global_step<float>(const ax_params &, void *, size_t, int, hipStream_t);
-template hipError_t launch_global_energy<double>(const ax_params &, const void *, size_t, int, double *, double *,
+template hipError_t launch_global_energy<double>(const ax_params &, const void *, size_t, int, Partials &,
                                                  hipStream_t);
-template hipError_t launch_global_energy<float>(const ax_params &, const void *, size_t, int, double *, double *,
-                                                hipStream_t);
+template hipError_t launch_global_energy<float>(const ax_params &, const void *, size_t, int, Partials &, hipStream_t);
 
 }  // namespace ax

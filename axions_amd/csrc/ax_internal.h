@@ -125,14 +125,22 @@ int lattice_device(const ax_lattice *L);
 int lattice_timestep(const ax_lattice *L);
 void lattice_reset_timestep(ax_lattice *L);
 
+/* Partial sums of a diagnostic pass: triples at p (room for
+ * diag_part_blocks), n of them once the pass is launched; launch_sums adds
+ * them up. */
+struct Partials {
+  double *p;
+  int n;
+};
+
 int launch_step(ax_lattice *L, int n);
 int ensure_winding_buffer(ax_lattice *L);
 int ensure_phase_buffer(ax_lattice *L);
-hipError_t launch_march_diag(ax_lattice *L, bool phases);
-hipError_t launch_phase_winding(ax_lattice *L, int8_t *out, double *res3);
+hipError_t launch_march_diag(ax_lattice *L, bool phases, Partials &part);
+hipError_t launch_phase_winding(ax_lattice *L, int8_t *out, Partials &part);
 int prepare_faces(ax_lattice *L);
 /* the Neumann faces prepared (prepare_faces); out may be null */
-int launch_winding_field(ax_lattice *L, int field, int8_t *out, double *part, double *res3);
+int launch_winding_field(ax_lattice *L, int field, int8_t *out, Partials &part);
 
 template <typename R>
 hipError_t launch_step_site(const StepConsts &k, const Levels<R> &L, int model, hipStream_t st);
@@ -151,14 +159,14 @@ template <typename R>
 hipError_t launch_global_step(const ax_params &p, void *state, size_t pitch, int n, hipStream_t st);
 size_t global_energy_blocks(const ax_params &p);   /* partial-sum blocks of launch_global_energy */
 template <typename R>
-hipError_t launch_global_energy(const ax_params &p, const void *state, size_t pitch, int n, double *part,
-                                double *out3, hipStream_t st);
+hipError_t launch_global_energy(const ax_params &p, const void *state, size_t pitch, int n, Partials &part,
+                                hipStream_t st);
 
 template <typename T>
-hipError_t launch_diag(const DiagConsts &k, const Levels<T> &L, double *part, double *out3, hipStream_t st);
+hipError_t launch_diag(const DiagConsts &k, const Levels<T> &L, Partials &part, hipStream_t st);
 /* Abelian-Higgs: energy/Gauss march, with phase != NULL also the FP32 edge
  * values [3][V] (forward edge phase + link angle, ax_wind.h); launch_wind_phase turns them into windings (the field into out when
- * out != NULL, the counts into out3; ex, ez: x and y, z not periodic) */
+ * out != NULL, the counts into part; ex, ez: x and y, z not periodic) */
 /* x planes per wave of the diagnostics and winding marches (us per
  * ax_diagnostics call without / with windings; this rule against the best of
  * 1 ... 32 planes: 64^3 27.5 / 41.8 against 27.4 / 41.7, 101^3 56.7 / 99
@@ -168,19 +176,18 @@ inline int diag_xseg(int nx, int ny, int nz) { return tile_xseg(nx, ny, nz, 32);
 bool use_diag_march(const ax_params &p);
 size_t diag_part_blocks(const ax_params &p);
 template <typename T>
-hipError_t launch_diag_march(const DiagConsts &k, const Levels<T> &L, float *phase, double *part, double *out3,
+hipError_t launch_diag_march(const DiagConsts &k, const Levels<T> &L, float *phase, Partials &part, hipStream_t st);
+hipError_t launch_wind_phase(int nx, int ny, int nz, int ex, int ez, const float *E, int8_t *out, Partials &part,
                              hipStream_t st);
-hipError_t launch_wind_phase(int nx, int ny, int nz, int ex, int ez, const float *E, int8_t *out, double *part,
-                             double *out3, hipStream_t st);
 /* the FP32 edge values of field (fr, fi) of charge q into E, then the
  * windings from them, as launch_wind_phase */
 template <typename T>
 hipError_t launch_edge_winding(int nx, int ny, int nz, int ex, int ez, const T *fr, const T *fi, const T *tx,
-                               const T *ty, const T *tz, double q, float *E, int8_t *out, double *part, double *out3,
+                               const T *ty, const T *tz, double q, float *E, int8_t *out, Partials &part,
                                hipStream_t st);
 template <typename T>
 hipError_t launch_winding(int nx, int ny, int nz, const T *fr, const T *fi, const T *tx, const T *ty, const T *tz,
-                          double q, int ex, int ez, int8_t *out, double *part, double *out3, hipStream_t st);
+                          double q, int ex, int ez, int8_t *out, Partials &part, hipStream_t st);
 /* Crossings: sites of one wave's group (a multiple of 64), and the groups of
  * a lattice, which is how many counts (bcount) and offsets (boff)
  * launch_crossings uses.  512 sites a group, fewer where that would leave
@@ -202,7 +209,9 @@ struct EnergyConsts;
 int fused_work_items(int nx, int ny, int nz, int xseg);
 hipError_t launch_step_fused(const StepConsts &k, const Levels<double> &L, int xseg, hipStream_t st, int mode,
                              bool p2d, const FusedDiag &fd);
-hipError_t launch_sum3(const double *part, int nb, double *out3, hipStream_t st);
+/* the sums of a into out3 and, where b holds any, of b into outb3 (which
+ * may be pinned host memory) in one launch */
+hipError_t launch_sums(const Partials &a, double *out3, const Partials &b, double *outb3, hipStream_t st);
 hipError_t launch_level_div(int nx, int ny, int nz, const double *tx, const double *ty, const double *tz,
                             const EnergyConsts &ek, bool pow2, double *div, hipStream_t st);
 bool diag_pow2(double dx, double dy, double dz, double gg);
