@@ -601,29 +601,28 @@ template <typename T, bool PH, bool P2>
 __global__ void __launch_bounds__(64, sizeof(T) == 8 ? 3 : 1) diag_march_kernel(DiagConsts k, Levels<T> L, TileGrid g, float *phase,
                                                         double *part) {
   const int w = (int)blockIdx.x;
-  int zc, y, seg;
-  tile_item(g, k.ny, w, zc, y, seg);
+  const int lane = (int)(threadIdx.x & 63);
+  int chunk, seg;
+  if (!tile_item(g, w, chunk, seg)) {
+    if (lane < 3) part[3 * (size_t)w + lane] = 0;
+    return;
+  }
   const int x0 = seg * g.xseg, x1 = min(k.nx, x0 + g.xseg);
   const int NX = k.nx, NY = k.ny, NZ = k.nz;
-  const int lane = (int)(threadIdx.x & 63);
-  const int zr = zc * 64 + lane;
-  const bool act = zr < NZ;
-  const int z = act ? zr : NZ - 1;
-  const int ym = y == 0 ? NY - 1 : y - 1, yp = y == NY - 1 ? 0 : y + 1;
-  const bool in_yz = !(k.ex && (y == 0 || y == NY - 1)) && !(k.ez && (z == 0 || z == NZ - 1));
+  const LaneSite<true> ls(NY, NZ, (uint32_t)chunk * 64);
+  const bool act = ls.act;
+  const bool in_yz = !(k.ex && (ls.y == 0 || ls.y == NY - 1)) && !(k.ez && (ls.z == 0 || ls.z == NZ - 1));
   const uint32_t E = (uint32_t)sizeof(T);
-  const uint32_t oz = (uint32_t)z * E;
-  const uint32_t ozm = (uint32_t)(z == 0 ? NZ - 1 : z - 1) * E;
-  const uint32_t ozp = (uint32_t)(z == NZ - 1 ? 0 : z + 1) * E;
-  const uint32_t R0 = (uint32_t)y * NZ * E, RM = (uint32_t)ym * NZ * E, RP = (uint32_t)yp * NZ * E;
+  /* byte offsets in a plane of the site and of y+-1, z+-1 (in the lane for
+   * every nz: with scalar row offsets the march holds more registers) */
+  const uint32_t o0 = ls.col(0, 0, E), oyp = ls.col(1, 0, E), oym = ls.col(-1, 0, E);
+  const uint32_t ozp = ls.col(0, 1, E), ozm = ls.col(0, -1, E);
   const T *PR = L.cur[0], *PI = L.cur[1], *TX = L.cur[2], *TY = L.cur[3], *TZ = L.cur[4];
   const T *OPR = L.prv[0], *OPI = L.prv[1], *OTX = L.prv[2], *OTY = L.prv[3], *OTZ = L.prv[4];
-  /* value of field b in x plane x at (row, lane) byte offsets: the plane's
-   * 64-bit address is formed on the scalar unit, so planes of any size work */
+  /* value of field b in x plane x at offsets in it: the plane's 64-bit
+   * address is formed on the scalar unit, so planes of any size work */
   const size_t NYNZ = (size_t)NY * NZ;
-  auto ld_ = [NYNZ](const T *b, int x, uint32_t row, uint32_t off) {
-    return (double)ldo(b + (size_t)x * NYNZ, row, off);
-  };
+  auto ld_ = [NYNZ](const T *b, int x, uint32_t o) { return (double)ldo(b + (size_t)x * NYNZ, 0u, o); };
   const double dx = k.dx, dy = k.dy, dz = k.dz, dt = k.dt, gg = k.g;
   const size_t V = (size_t)NX * NY * NZ;
   const double dxx = dx * dx, dyy = dy * dy, dzz = dz * dz;
@@ -646,28 +645,29 @@ __global__ void __launch_bounds__(64, sizeof(T) == 8 ? 3 : 1) diag_march_kernel(
 
   /* carried from plane x-1: phi, theta_x (both levels), sin/cos theta_x */
   const int xm0 = x0 == 0 ? NX - 1 : x0 - 1;
-  double PRm = ld_(PR, xm0, R0, oz), PIm = ld_(PI, xm0, R0, oz);
-  double TXm = ld_(TX, xm0, R0, oz), oXm = ld_(OTX, xm0, R0, oz);
+  double PRm = ld_(PR, xm0, o0), PIm = ld_(PI, xm0, o0);
+  double TXm = ld_(TX, xm0, o0), oXm = ld_(OTX, xm0, o0);
   double sxm, cxm;
   ax_sincos(TXm, &sxm, &cxm);
-  double PRc = ld_(PR, x0, R0, oz), PIc = ld_(PI, x0, R0, oz);
-  double X = ld_(TX, x0, R0, oz), Y = ld_(TY, x0, R0, oz), Z = ld_(TZ, x0, R0, oz);
-  double rho_sum = 0, g_sum = 0, bad = 0;
+  double PRc = ld_(PR, x0, o0), PIc = ld_(PI, x0, o0);
+  double X = ld_(TX, x0, o0), Y = ld_(TY, x0, o0), Z = ld_(TZ, x0, o0);
+  double rho_sum = 0, g_sum = 0;
+  int bad = 0;
 
   for (int x = x0; x < x1; ++x) {
     const int xp = x == NX - 1 ? 0 : x + 1;
-    const double PRn = ld_(PR, xp, R0, oz), PIn = ld_(PI, xp, R0, oz);
-    const double TXn = ld_(TX, xp, R0, oz), TYn = ld_(TY, xp, R0, oz), TZn = ld_(TZ, xp, R0, oz);
-    const double oPR = ld_(OPR, x, R0, oz), oPI = ld_(OPI, x, R0, oz);
-    const double oX = ld_(OTX, x, R0, oz), oY = ld_(OTY, x, R0, oz), oZ = ld_(OTZ, x, R0, oz);
-    const double PRyp = ld_(PR, x, RP, oz), PIyp = ld_(PI, x, RP, oz);
-    const double TXyp = ld_(TX, x, RP, oz), TZyp = ld_(TZ, x, RP, oz);
-    const double PRzp = ld_(PR, x, R0, ozp), PIzp = ld_(PI, x, R0, ozp);
-    const double TXzp = ld_(TX, x, R0, ozp), TYzp = ld_(TY, x, R0, ozp);
-    const double PRym = ld_(PR, x, RM, oz), PIym = ld_(PI, x, RM, oz);
-    const double TYym = ld_(TY, x, RM, oz), oYym = ld_(OTY, x, RM, oz);
-    const double PRzm = ld_(PR, x, R0, ozm), PIzm = ld_(PI, x, R0, ozm);
-    const double TZzm = ld_(TZ, x, R0, ozm), oZzm = ld_(OTZ, x, R0, ozm);
+    const double PRn = ld_(PR, xp, o0), PIn = ld_(PI, xp, o0);
+    const double TXn = ld_(TX, xp, o0), TYn = ld_(TY, xp, o0), TZn = ld_(TZ, xp, o0);
+    const double oPR = ld_(OPR, x, o0), oPI = ld_(OPI, x, o0);
+    const double oX = ld_(OTX, x, o0), oY = ld_(OTY, x, o0), oZ = ld_(OTZ, x, o0);
+    const double PRyp = ld_(PR, x, oyp), PIyp = ld_(PI, x, oyp);
+    const double TXyp = ld_(TX, x, oyp), TZyp = ld_(TZ, x, oyp);
+    const double PRzp = ld_(PR, x, ozp), PIzp = ld_(PI, x, ozp);
+    const double TXzp = ld_(TX, x, ozp), TYzp = ld_(TY, x, ozp);
+    const double PRym = ld_(PR, x, oym), PIym = ld_(PI, x, oym);
+    const double TYym = ld_(TY, x, oym), oYym = ld_(OTY, x, oym);
+    const double PRzm = ld_(PR, x, ozm), PIzm = ld_(PI, x, ozm);
+    const double TZzm = ld_(TZ, x, ozm), oZzm = ld_(OTZ, x, ozm);
 
     /* site_energy_ah at s, operands by name */
     const double pr = PRc, pi = PIc;
@@ -742,10 +742,11 @@ __global__ void __launch_bounds__(64, sizeof(T) == 8 ? 3 : 1) diag_march_kernel(
       const double dY = link_phase_sc(pr, pi, PRyp, PIyp, sy, cy);
       const double dZ = link_phase_sc(pr, pi, PRzp, PIzp, sz, cz);
       if (act) {
-        const size_t s = ((size_t)x * NY + y) * NZ + z;
-        phase[s] = (float)(dX + X);   /* edge values e_a(s) (ax_wind.h) */
-        phase[V + s] = (float)(dY + Y);
-        phase[2 * V + s] = (float)(dZ + Z);
+        /* edge values e_a(s) (ax_wind.h) */
+        float *e = phase + (size_t)x * NYNZ;
+        sto(e, 0u, ls.p * 4u, (float)(dX + X));
+        sto(e + V, 0u, ls.p * 4u, (float)(dY + Y));
+        sto(e + 2 * V, 0u, ls.p * 4u, (float)(dZ + Z));
       }
     }
     if (act) {
@@ -757,14 +758,13 @@ __global__ void __launch_bounds__(64, sizeof(T) == 8 ? 3 : 1) diag_march_kernel(
         rho_sum += rho;
         g_sum += fabs(G);
       }
-      const double vals[10] = {PRc, PIc, X, Y, Z, oPR, oPI, oX, oY, oZ};
-#pragma unroll
-      for (int q = 0; q < 10; ++q) bad += isfinite(vals[q]) ? 0.0 : 1.0;
     }
+    const double vals[10] = {PRc, PIc, X, Y, Z, oPR, oPI, oX, oY, oZ};
+    bad += nonfinite(vals, act);
     PRm = PRc; PIm = PIc; TXm = X; oXm = oX; sxm = sx; cxm = cx;
     PRc = PRn; PIc = PIn; X = TXn; Y = TYn; Z = TZn;
   }
-  const double a = wave_sum(rho_sum), bsum = wave_sum(g_sum), c = wave_sum(bad);
+  const double a = wave_sum(rho_sum), bsum = wave_sum(g_sum), c = (double)bad;
   if (lane == 0) {
     part[3 * w] = a;
     part[3 * w + 1] = bsum;
@@ -779,13 +779,16 @@ __global__ void __launch_bounds__(64, sizeof(T) == 8 ? 3 : 1) diag_march_kernel(
 __global__ void __launch_bounds__(64) wind_march_kernel(int nx, int ny, int nz, const float *E, TileGrid g, int ex,
                                                         int ez, int8_t *out, double *part) {
   const int item = (int)blockIdx.x;
-  int zc, y, seg;
-  tile_item(g, ny, item, zc, y, seg);
+  int chunk, seg;
+  if (!tile_item(g, item, chunk, seg)) {
+    if (threadIdx.x < 3) part[3 * (size_t)item + threadIdx.x] = 0;
+    return;
+  }
   const int x0 = seg * g.xseg, x1 = min(nx, x0 + g.xseg);
-  const WindRow w(nx, ny, nz, y, zc);
+  const WindRow w(nx, ny, nz, chunk);
   double tot[3] = {0, 0, 0};
   /* plaquettes that would wrap across a non-periodic axis do not exist */
-  const bool ye = ex && y == ny - 1, ze = ez && w.z == nz - 1;
+  const bool ye = ex && w.y == ny - 1, ze = ez && w.z == nz - 1;
   wind_march(w, E, x0, x1, [&](int x, size_t s, const int *wn) {
     const bool xe = ex && x == nx - 1;
     const bool none[3] = {xe || ye, xe || ze, ye || ze};
@@ -819,50 +822,52 @@ template <typename T>
 __global__ void __launch_bounds__(64, sizeof(T) == 8 ? 3 : 1) moore_diag_march_kernel(DiagConsts k, Levels<T> L,
                                                                                    TileGrid g, double *part) {
   const int w = (int)blockIdx.x;
-  int zc, y, seg;
-  tile_item(g, k.ny, w, zc, y, seg);
+  const int lane = (int)(threadIdx.x & 63);
+  int chunk, seg;
+  if (!tile_item(g, w, chunk, seg)) {
+    if (lane < 3) part[3 * (size_t)w + lane] = 0;
+    return;
+  }
   const int x0 = seg * g.xseg, x1 = min(k.nx, x0 + g.xseg);
   const int NX = k.nx, NY = k.ny, NZ = k.nz;
-  const int lane = (int)(threadIdx.x & 63);
-  const int zr = zc * 64 + lane;
-  const bool act = zr < NZ;
-  const int z = act ? zr : NZ - 1;
-  const int ym = y == 0 ? NY - 1 : y - 1, yp = y == NY - 1 ? 0 : y + 1;
-  const bool in_yz = !(k.ex && (y == 0 || y == NY - 1)) && !(k.ez && (z == 0 || z == NZ - 1));
+  const LaneSite<true> ls(NY, NZ, (uint32_t)chunk * 64);
+  const bool act = ls.act;
+  const bool in_yz = !(k.ex && (ls.y == 0 || ls.y == NY - 1)) && !(k.ez && (ls.z == 0 || ls.z == NZ - 1));
   const uint32_t E = (uint32_t)sizeof(T);
-  const uint32_t oz = (uint32_t)z * E;
-  const uint32_t ozm = (uint32_t)(z == 0 ? NZ - 1 : z - 1) * E;
-  const uint32_t ozp = (uint32_t)(z == NZ - 1 ? 0 : z + 1) * E;
-  const uint32_t R0 = (uint32_t)y * NZ * E, RM = (uint32_t)ym * NZ * E, RP = (uint32_t)yp * NZ * E;
+  /* byte offsets in a plane of the site and of y+-1, z+-1 (in the lane for
+   * every nz: with scalar row offsets the march spills more) */
+  const uint32_t o0 = ls.col(0, 0, E), oyp = ls.col(1, 0, E), oym = ls.col(-1, 0, E);
+  const uint32_t ozp = ls.col(0, 1, E), ozm = ls.col(0, -1, E);
   const size_t NYNZ = (size_t)NY * NZ;
-  auto C = [&](int c, int x, uint32_t row, uint32_t off) { return (double)ldo(L.cur[c] + (size_t)x * NYNZ, row, off); };
-  auto P = [&](int c, int x, uint32_t row, uint32_t off) { return (double)ldo(L.prv[c] + (size_t)x * NYNZ, row, off); };
+  auto C = [&](int c, int x, uint32_t o) { return (double)ldo(L.cur[c] + (size_t)x * NYNZ, 0u, o); };
+  auto P = [&](int c, int x, uint32_t o) { return (double)ldo(L.prv[c] + (size_t)x * NYNZ, 0u, o); };
   const double dx = k.dx, dy = k.dy, dz = k.dz, dt = k.dt, gg = k.g;
   const double q[2] = {k.q1, k.q2};
   /* plane x-1 (carried): both scalars, theta_x of both levels; plane x */
   const int xm0 = x0 == 0 ? NX - 1 : x0 - 1;
-  double Fm[4], TXm = C(4, xm0, R0, oz), oXm = P(4, xm0, R0, oz), Fc[4], Tc[3];
+  double Fm[4], TXm = C(4, xm0, o0), oXm = P(4, xm0, o0), Fc[4], Tc[3];
   for (int c = 0; c < 4; ++c) {
-    Fm[c] = C(c, xm0, R0, oz);
-    Fc[c] = C(c, x0, R0, oz);
+    Fm[c] = C(c, xm0, o0);
+    Fc[c] = C(c, x0, o0);
   }
-  for (int a = 0; a < 3; ++a) Tc[a] = C(4 + a, x0, R0, oz);
-  double rho_sum = 0, g_sum = 0, bad = 0;
+  for (int a = 0; a < 3; ++a) Tc[a] = C(4 + a, x0, o0);
+  double rho_sum = 0, g_sum = 0;
+  int bad = 0;
   for (int x = x0; x < x1; ++x) {
     const int xp = x == NX - 1 ? 0 : x + 1;
     double Fn[4], Tn[3], Fo[4], Fy[4], Fz[4];
     for (int c = 0; c < 4; ++c) {
-      Fn[c] = C(c, xp, R0, oz);
-      Fo[c] = P(c, x, R0, oz);
-      Fy[c] = C(c, x, RM, oz);
-      Fz[c] = C(c, x, R0, ozm);
+      Fn[c] = C(c, xp, o0);
+      Fo[c] = P(c, x, o0);
+      Fy[c] = C(c, x, oym);
+      Fz[c] = C(c, x, ozm);
     }
-    for (int a = 0; a < 3; ++a) Tn[a] = C(4 + a, xp, R0, oz);
-    const double oX = P(4, x, R0, oz), oY = P(5, x, R0, oz), oZ = P(6, x, R0, oz);
-    const double TYym = C(5, x, RM, oz), oYym = P(5, x, RM, oz);
-    const double TZzm = C(6, x, R0, ozm), oZzm = P(6, x, R0, ozm);
-    const double TXyp = C(4, x, RP, oz), TZyp = C(6, x, RP, oz);
-    const double TXzp = C(4, x, R0, ozp), TYzp = C(5, x, R0, ozp);
+    for (int a = 0; a < 3; ++a) Tn[a] = C(4 + a, xp, o0);
+    const double oX = P(4, x, o0), oY = P(5, x, o0), oZ = P(6, x, o0);
+    const double TYym = C(5, x, oym), oYym = P(5, x, oym);
+    const double TZzm = C(6, x, ozm), oZzm = P(6, x, ozm);
+    const double TXyp = C(4, x, oyp), TZyp = C(6, x, oyp);
+    const double TXzp = C(4, x, ozp), TYzp = C(5, x, ozp);
     const double X = Tc[0], Y = Tc[1], Z = Tc[2];
 
     /* site_energy_moore at s, operands by name */
@@ -912,10 +917,9 @@ __global__ void __launch_bounds__(64, sizeof(T) == 8 ? 3 : 1) moore_diag_march_k
         rho_sum += rho;
         g_sum += absG;
       }
-      const double vals[14] = {Fc[0], Fc[1], Fc[2], Fc[3], X, Y, Z, Fo[0], Fo[1], Fo[2], Fo[3], oX, oY, oZ};
-#pragma unroll
-      for (int c = 0; c < 14; ++c) bad += isfinite(vals[c]) ? 0.0 : 1.0;
     }
+    const double vals[14] = {Fc[0], Fc[1], Fc[2], Fc[3], X, Y, Z, Fo[0], Fo[1], Fo[2], Fo[3], oX, oY, oZ};
+    bad += nonfinite(vals, act);
     for (int c = 0; c < 4; ++c) {
       Fm[c] = Fc[c];
       Fc[c] = Fn[c];
@@ -924,7 +928,7 @@ __global__ void __launch_bounds__(64, sizeof(T) == 8 ? 3 : 1) moore_diag_march_k
     oXm = oX;
     for (int a = 0; a < 3; ++a) Tc[a] = Tn[a];
   }
-  const double a = wave_sum(rho_sum), b = wave_sum(g_sum), c = wave_sum(bad);
+  const double a = wave_sum(rho_sum), b = wave_sum(g_sum), c = (double)bad;
   if (lane == 0) {
     part[3 * w] = a;
     part[3 * w + 1] = b;
@@ -994,10 +998,10 @@ hipError_t launch_crossings(int nx, int ny, int nz, double dx, double dy, double
 template <typename T>
 __global__ void __launch_bounds__(64) edge_march_kernel(int nx, int ny, int nz, const T *fr, const T *fi, const T *tx,
                                                         const T *ty, const T *tz, double q, TileGrid g, float *E) {
-  int zc, y, seg;
-  tile_item(g, ny, (int)blockIdx.x, zc, y, seg);
+  int chunk, seg;
+  if (!tile_item(g, (int)blockIdx.x, chunk, seg)) return;
   const int x0 = seg * g.xseg, x1 = min(nx, x0 + g.xseg);
-  const WindRow w(nx, ny, nz, y, zc);
+  const WindRow w(nx, ny, nz, chunk);
   (void)phase_march<T>(w, fr, fi, tx, ty, tz, E, x0, x1, q);
 }
 

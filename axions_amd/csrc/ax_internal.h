@@ -14,37 +14,82 @@ struct ax_lattice;
 
 namespace ax {
 
-/* Work items of a marching kernel: one 64-lane wave per (64-site z chunk,
- * row, x segment of xseg planes), numbered as make_tile_grid describes. */
+/* Work items of a marching kernel: one 64-lane wave per (chunk of 64
+ * consecutive sites of the (y, z) plane, x segment of xseg planes).  A chunk
+ * lies in one row where nz is a multiple of 64 and crosses rows otherwise.
+ *
+ * Workgroups are handed to the eight XCDs round-robin (workgroup w to XCD w
+ * mod 8), each XCD with its own L2.  With chunk = w mod nc, neighbouring
+ * chunks, which share the cache lines at their z edges and the rows at their
+ * y edges, would sit on different XCDs.  So XCD x gets the x-th eighth of each
+ * segment's chunks, a band of consecutive rows (512^3 FP64 reads 15.4 -> 12.9
+ * GB per step, FP32 9.0 -> 6.1 GB); where the chunks are no multiple of 8 a
+ * few of the workgroups find nothing to do. */
 struct TileGrid {
-  int nw;      /* z chunks per row */
+  int nc;      /* chunks of a plane */
   int xseg;    /* x planes marched by one wave */
-  int work;    /* nw * ny * nseg */
-  int per;     /* XCD-aware order: work items per XCD per x segment, 0 = natural order */
-  int rows;    /* 1: within an XCD's share, all chunks of a row together (chunk fastest) */
+  int work;    /* workgroups, with the empty ones */
+  int per;     /* chunks per XCD per x segment, 0 = natural order */
 };
 
-/* Work items of the marching kernels, one per (z chunk, y row, x segment).
- * Workgroups are handed to the eight XCDs round-robin (workgroup w to XCD
- * w mod 8), each XCD with its own L2.  In the natural order (z chunk
- * fastest) XCD x receives chunk x mod 8 of every row: neighbouring chunks of
- * a row, which share the cache lines at their z edges, sit on different
- * XCDs, and with fewer than 8 chunks per row even neighbouring rows do.  The
- * XCD-aware order gives XCD x the x-th eighth of each x segment's items:
- * with ny divisible by 8, a band of ny/8 consecutive rows with all their
- * chunks, chunk fastest (512^3 FP64 reads 15.4 -> 12.9 GB per step, FP32
- * 9.0 -> 6.1 GB); otherwise a run of consecutive rows of one chunk. */
+inline int tile_chunks(int ny, int nz) { return (int)(((long long)ny * nz + 63) / 64); }
+
 inline TileGrid make_tile_grid(int nx, int ny, int nz, int xseg) {
   TileGrid g;
   g.xseg = (xseg <= 0 || xseg > nx) ? nx : xseg;
-  g.nw = (nz + 63) / 64;
-  g.work = g.nw * ny * ((nx + g.xseg - 1) / g.xseg);
-  const char *o = getenv("AX_TILE_ORDER");        /* "natural" or "chunks" for measurements */
+  g.nc = tile_chunks(ny, nz);
+  const char *o = getenv("AX_TILE_ORDER");        /* "natural" for measurements */
   const bool natural = o && o[0] == 'n';
-  g.per = (!natural && (g.nw * ny) % 8 == 0) ? g.nw * ny / 8 : 0;
-  g.rows = !(o && o[0] == 'c') && ny % 8 == 0;
+  g.per = natural ? 0 : (g.nc + 7) / 8;
+  g.work = (natural ? g.nc : 8 * g.per) * ((nx + g.xseg - 1) / g.xseg);
   return g;
 }
+
+/* chunk and x segment of workgroup w; false for an empty one */
+__device__ __forceinline__ bool tile_item(const TileGrid &g, int w, int &chunk, int &seg) {
+  if (g.per) {
+    const int i = w >> 3;
+    seg = i / g.per;
+    chunk = (w & 7) * g.per + (i - seg * g.per);
+    return chunk < g.nc;
+  }
+  seg = w / g.nc;
+  chunk = w - seg * g.nc;
+  return true;
+}
+
+/* This lane's site of the chunk that begins at site p0 of the (y, z) plane.
+ * FLAT: chunks cross rows, so rows that are no multiple of 64 long leave no
+ * lanes idle (101^3: 160 waves a plane instead of 202); lanes past the
+ * plane's last site hold that site (act false).  Otherwise nz is a multiple
+ * of 64, a chunk lies in one row, and the byte offset of a neighbour in its
+ * plane splits into a scalar row part and a lane part (two to four VGPRs
+ * fewer). */
+template <bool FLAT>
+struct LaneSite {
+  uint32_t p;
+  int y, z, ym, yp, zm, zp, nz;
+  bool act;
+  __device__ __forceinline__ LaneSite(int ny, int nz_, uint32_t p0) : nz(nz_) {
+    const uint32_t n = (uint32_t)ny * nz_, q = p0 + (threadIdx.x & 63);
+    act = !FLAT || q < n;
+    p = act ? q : n - 1;
+    y = (int)((FLAT ? p : p0) / (uint32_t)nz_);
+    z = (int)(p - (uint32_t)y * nz_);
+    ym = y == 0 ? ny - 1 : y - 1;
+    yp = y == ny - 1 ? 0 : y + 1;
+    zm = z == 0 ? nz_ - 1 : z - 1;
+    zp = z == nz_ - 1 ? 0 : z + 1;
+  }
+  /* row and lane byte offsets of the site (y + r, z + c), elements of E bytes */
+  __device__ __forceinline__ uint32_t row(int r, uint32_t E) const {
+    return FLAT ? 0u : (uint32_t)(r < 0 ? ym : r > 0 ? yp : y) * nz * E;
+  }
+  __device__ __forceinline__ uint32_t col(int r, int c, uint32_t E) const {
+    const uint32_t zz = (uint32_t)(c < 0 ? zm : c > 0 ? zp : z);
+    return (FLAT ? (uint32_t)(r < 0 ? ym : r > 0 ? yp : y) * nz + zz : zz) * E;
+  }
+};
 
 /* n / d for n < 2^31 and d >= 2 by a multiplication: m = floor(2^(31+s)/d) + 1
  * with 2^(s-1) < d <= 2^s exceeds 2^(31+s)/d by less than 2^s/d <= 2, so the
@@ -61,44 +106,19 @@ __device__ __forceinline__ uint32_t quotient(uint32_t n, const FastDiv &f) { ret
 
 /* x planes per wave of a march over the whole lattice, at most cap.  A wave
  * pays a prologue worth about one plane, so long segments do the least work;
- * but a lattice of few rows then fills few of the chip's 1024 SIMDs, and
+ * but a lattice of few chunks then fills few of the chip's 1024 SIMDs, and
  * the launch ends with a tail that lasts as long as one segment.  With W
- * (64-site rows) x (planes) per SIMD, work W (1 + c / xseg) plus a tail of
+ * (chunks) x (planes) per SIMD, work W (1 + c / xseg) plus a tail of
  * xseg planes is least near xseg = sqrt(W), which is what the sweeps show
  * (AH FP64 step, us per step with 32 planes / with this rule / best of 1 ...
- * 32: 32^3 68 / 6.6 / 6.6, 64^3 64 / 12.6 / 12.6, 101^3 87 / 50 / 50, 128^3
- * 74 / 66 / 63, 160^3 150 / 136 / 135, 192^3 223 / 202 / 201, 256^3 475 /
- * 477 / 475).  The length is then evened out over the segments. */
+ * 32: 32^3 68 / 6.6 / 6.6, 64^3 64 / 12.6 / 12.6, 128^3 74 / 66 / 63, 192^3
+ * 223 / 202 / 201, 256^3 475 / 477 / 475).  The length is then evened out over the segments. */
 inline int tile_xseg(int nx, int ny, int nz, int cap) {
-  const double w = (double)((nz + 63) / 64) * ny * nx / 1024.0;
+  const double w = (double)tile_chunks(ny, nz) * nx / 1024.0;
   const double x = std::sqrt(w) + 0.5;
   const int xs = x >= cap ? cap : x < 1 ? 1 : (int)x;
   const int nseg = (nx + xs - 1) / xs;
   return (nx + nseg - 1) / nseg;
-}
-
-/* (z chunk, y row, x segment) of work item w in the order make_tile_grid chose */
-__device__ __forceinline__ void tile_item(const TileGrid &g, int ny, int w, int &zc, int &y, int &seg) {
-  if (g.per && g.rows) {
-    const int xcd = w & 7, i = w >> 3, s = i / g.per;
-    const int item = (s * 8 + xcd) * g.per + (i - s * g.per);   /* chunk + nw * (row + ny * segment) */
-    zc = item % g.nw;
-    const int r = item / g.nw;
-    y = r % ny;
-    seg = r / ny;
-  } else if (g.per) {
-    const int xcd = w & 7, i = w >> 3, s = i / g.per;
-    const int item = (s * 8 + xcd) * g.per + (i - s * g.per);   /* row + ny * (chunk + nw * segment) */
-    y = item % ny;
-    const int r = item / ny;
-    zc = r % g.nw;
-    seg = r / g.nw;
-  } else {
-    zc = w % g.nw;
-    const int r = w / g.nw;
-    y = r % ny;
-    seg = r / ny;
-  }
 }
 
 struct DiagConsts {
@@ -169,9 +189,9 @@ hipError_t launch_diag(const DiagConsts &k, const Levels<T> &L, Partials &part, 
  * out != NULL, the counts into part; ex, ez: x and y, z not periodic) */
 /* x planes per wave of the diagnostics and winding marches (us per
  * ax_diagnostics call without / with windings; this rule against the best of
- * 1 ... 32 planes: 64^3 27.5 / 41.8 against 27.4 / 41.7, 101^3 56.7 / 99
- * against 55.9 / 97, 160^3 125 / 244 against 125 / 244; with 32 planes at
- * 101^3 the energy march alone took 84, with this rule 35) */
+ * 1 ... 32 planes: 64^3 27.5 / 41.8 against 27.4 / 41.7, 160^3 125 / 244
+ * against 125 / 244; with 32 planes the energy march alone took 84 at 101^3,
+ * with this rule 35) */
 inline int diag_xseg(int nx, int ny, int nz) { return tile_xseg(nx, ny, nz, 32); }
 bool use_diag_march(const ax_params &p);
 size_t diag_part_blocks(const ax_params &p);

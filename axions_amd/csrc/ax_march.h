@@ -1,6 +1,6 @@
 /*
  * ax_march.h - the Abelian-Higgs site update as one 64-lane wave marching
- * along x over a 64-site z chunk of one (y) row.  Shared by the
+ * along x over a 64-site chunk of the (y, z) plane.  Shared by the
  * single-lattice tiled kernel (ax_step_tiled.hip) and the batched ensemble
  * kernel (ax_pool.hip).
  *
@@ -12,8 +12,9 @@
  *     iteration of the march, kept in registers;
  *   - z-backward trig (cos/sin theta_z(s-z) and the F_xz, F_yz sines at
  *     s-z) is lane - 1's own value, shifted across by DPP; the chunk's first
- *     lane takes values evaluated for the site before the chunk in one
- *     vector pass per few planes (one plane per lane, kept in LDS);
+ *     lane, and the first of a row inside it, take values evaluated for the
+ *     site before them in one vector pass per few planes (one plane and edge
+ *     per lane, kept in LDS);
  *   - y-backward values are recomputed from their operands with the same
  *     expressions the neighbour uses for its own forward values;
  *   - the six plaquette sines at s are computed once (the second sine of
@@ -31,16 +32,16 @@
  * instructions; the previous level's reads and the new level's writes carry
  * the streaming hint so that they do not push those rows out of L2.
  *
- * A chunk may be partial (nz not a multiple of 64): lanes past the row end
- * load the last site of the row and store nothing; values shifted from
- * lane - 1 only reach active lanes from active lanes, so partial chunks
- * need no special handling beyond that.
+ * A plane's last chunk may be partial: lanes past its end hold its last
+ * site and store nothing; values shifted from lane - 1 only reach active
+ * lanes from active lanes, so it needs no handling beyond that.
  */
 #ifndef AXIONS_AX_MARCH_H
 #define AXIONS_AX_MARCH_H
 
 #include "ax_device.h"
 #include "ax_energy.h"
+#include "ax_internal.h"   /* LaneSite */
 
 namespace ax {
 
@@ -162,10 +163,11 @@ struct MarchCarry {
   R TXm;               /* theta_x(s-x) (read only by the divergence of the fused diagnostics) */
 };
 
-/* What the site before a chunk (z0 - 1) contributes to the chunk's first
- * lane: sin/cos theta_z there and its F_xz, F_yz plaquette sines.  Every
- * other lane takes them from lane - 1, which evaluates them for its own
- * site with the same operands in the same order. */
+/* What the site (y, z - 1) contributes to a lane whose lane - 1 is not that
+ * site (the chunk's first, and the first of a row that begins inside it):
+ * sin/cos theta_z there and its F_xz, F_yz plaquette sines.  Every other
+ * lane takes them from lane - 1, which evaluates them for its own site with
+ * the same operands in the same order. */
 template <typename R>
 struct ZEdge {
   R s, c, qxz, qyz;
@@ -250,14 +252,23 @@ __device__ __forceinline__ uint64_t big_lanes(R d, R lim) {
   return __builtin_amdgcn_ballot_w64(!(fabs(d) <= lim));
 }
 
+/* A z-backward value: lane - 1's, on the lanes e0 the edge value (SEL: on
+ * any of them, else on lane 0 alone).  Every lane must call it. */
+template <bool SEL, typename R>
+__device__ __forceinline__ R z_back(R v, R edge, bool e0) {
+  const R s = lane_prev(v, edge);
+  return SEL && e0 ? edge : s;
+}
+
 /* One site of the fused in-place update (mpi_evolution.cpp:418-501) from its
  * operands g(Op), the carry from s-x, which it advances to s, and the
- * chunk-edge values ze (used by lane 0 only).  Every lane of the wave must
+ * chunk-edge values ze (used by the lanes e0).  Every lane of the wave must
  * call it (it votes across the wave with ballots and shifts values between
  * lanes). */
-template <typename R, bool POW2, typename G, bool TR = false>
+template <typename R, bool POW2, typename G, bool TR, bool SEL>
 __device__ __forceinline__ void ah_site_update(const MarchConsts<R> &k, bool plain, const G &g, MarchCarry<R> &m,
-                                               const ZEdge<R> &ze, SiteOut<R> &o, SiteTrig<R> *tr = nullptr) {
+                                               const ZEdge<R> &ze, bool e0, SiteOut<R> &o,
+                                               SiteTrig<R> *tr = nullptr) {
   typedef TrigR<R> T;
   const R dx2 = k.dx2, dy2 = k.dy2, dz2 = k.dz2, dt = k.dt, dt2 = k.dt2;
   const R hl = k.hl, eta2 = k.eta2, m2gg = k.m2gg, fric = k.fric, damp = k.damp;
@@ -268,7 +279,7 @@ __device__ __forceinline__ void ah_site_update(const MarchConsts<R> &k, bool pla
   T::sc(TYc, &sy, &cy);
   T::sc(TZc, &sz, &cz);
   T::sc(TYym, &sym_, &cym);
-  const R szm = lane_prev(sz, ze.s), czm = lane_prev(cz, ze.c);
+  const R szm = z_back<SEL, R>(sz, ze.s, e0), czm = z_back<SEL, R>(cz, ze.c, e0);
   /* plaquette angles, reference operand order */
   const R TYn = g(kTYn), TZn = g(kTZn), TXyp = g(kTXyp), TXzp = g(kTXzp), TZyp = g(kTZyp), TYzp = g(kTYzp);
   const R a_xy = TXc + TYn - TXyp - TYc;
@@ -300,7 +311,7 @@ __device__ __forceinline__ void ah_site_update(const MarchConsts<R> &k, bool pla
   }
   /* the second sines of F_xz, F_yz (arguments TXzm + TZxpzm - TXc - TZzm and
    * TYzm + TZypzm - TYc - TZzm) are lane - 1's first ones */
-  const R Qxz_m = lane_prev(Qxz, ze.qxz), Qyz_m = lane_prev(Qyz, ze.qyz);
+  const R Qxz_m = z_back<SEL, R>(Qxz, ze.qxz, e0), Qyz_m = z_back<SEL, R>(Qyz, ze.qyz, e0);
 
   /* gauge field first (frees the plaquette sines early) */
   const R fxy = mdiv<R, POW2>(Qxy - Qxy_m, dy2, k.inv_dy2);
@@ -391,8 +402,11 @@ __device__ __forceinline__ void march_prologue(Get G, int xm0, int x0, MarchCarr
  * offsets (one x plane of NY*NZ values is far below 4 GiB). */
 typedef __attribute__((address_space(3))) void lds_void;
 
-/* PF (FP64, whole 64-site chunks, planes small enough that three of them
- * fit 32-bit offsets): the ten values of a plane that come from HBM -- the
+/* FLAT: the wave's 64 sites cross rows (LaneSite); otherwise they are of one
+ * row, nz a multiple of 64.
+ *
+ * PF (FP64, not FLAT, planes small enough that three of them fit 32-bit
+ * offsets): the ten values of a plane that come from HBM -- the
  * previous level at (x, y) and the current level at (x+1, y) -- are loaded
  * one plane ahead straight into LDS (16 bytes per lane: lanes 0-31 carry
  * one field's 64 sites, lanes 32-63 another's), so their latency overlaps
@@ -423,26 +437,41 @@ __device__ __forceinline__ double march_wave_sum(double v) {
   return v;
 }
 
-template <typename R, bool POW2, int PLAIN, bool BIG = false, bool PF = false, int MODE = 0, bool P2D = false>
+/* How many of the active lanes' n values are not finite: one compare each,
+ * the lane masks combined and counted on the scalar unit, which keeps the
+ * running count out of the vector registers. */
+template <int N>
+__device__ __forceinline__ int nonfinite(const double (&v)[N], bool act) {
+  uint64_t any = 0, m[N];
+#pragma unroll
+  for (int q = 0; q < N; ++q) {
+    m[q] = __builtin_amdgcn_ballot_w64(act && !isfinite(v[q]));
+    any |= m[q];
+  }
+  int n = 0;
+  if (any)
+    for (int q = 0; q < N; ++q) n += __popcll(m[q]);
+  return n;
+}
+
+template <typename R, bool POW2, int PLAIN, bool BIG = false, bool PF = false, int MODE = 0, bool P2D = false,
+          bool FLAT = false>
 __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R> &L, int NX, int NY, int NZ,
-                                         int y, int zc, int x0, int x1, bool zfix = false,
+                                         uint32_t p0, int x0, int x1, bool xfix = false, bool zfix = false,
                                          FusedDiag fd = FusedDiag{}, int item = 0) {
-  static_assert(!PF || (sizeof(R) == 8 && !BIG), "the prefetch path is FP64 with 32-bit plane offsets");
+  static_assert(!PF || (sizeof(R) == 8 && !BIG && !FLAT), "the prefetch path is FP64 with 32-bit plane offsets");
   static_assert(MODE == 0 || (sizeof(R) == 8 && !BIG), "the fused diagnostics are FP64");
   const int lane = (int)(threadIdx.x & 63);
-  const int zr = zc * 64 + lane;
-  const bool inz = zr < NZ;
-  const int z = inz ? zr : NZ - 1;
-  /* zfix: z not periodic, the z = 0 and NZ-1 sites are not stepped */
-  const bool act = inz && !(zfix && (zr == 0 || zr == NZ - 1));
-  const int ym = y == 0 ? NY - 1 : y - 1, yp = y == NY - 1 ? 0 : y + 1;
+  const uint32_t NYNZ = (uint32_t)NY * (uint32_t)NZ;
+  const LaneSite<FLAT> ls(NY, NZ, p0);
+  const uint32_t p = ls.p;
+  const int y0 = (int)(p0 / (uint32_t)NZ), y = ls.y, z = ls.z;
+  /* xfix, zfix: x and y, z not periodic; their face sites are not stepped */
+  const bool act = ls.act && !(zfix && (z == 0 || z == NZ - 1)) && !(xfix && (y == 0 || y == NY - 1));
   const uint32_t E = (uint32_t)sizeof(R);
-  const uint32_t oz = (uint32_t)z * E;
-  const uint32_t ozm = (uint32_t)(z == 0 ? NZ - 1 : z - 1) * E;
-  const uint32_t ozp = (uint32_t)(z == NZ - 1 ? 0 : z + 1) * E;
-  const uint32_t PLB = (uint32_t)NY * (uint32_t)NZ * E;          /* plane bytes */
-  const uint32_t R0 = (uint32_t)y * NZ * E, RM = (uint32_t)ym * NZ * E, RP = (uint32_t)yp * NZ * E;
-  const R *PR = L.cur[0], *PI = L.cur[1], *TX = L.cur[2], *TY = L.cur[3], *TZ = L.cur[4];
+  const uint32_t PLB = NYNZ * E;          /* plane bytes */
+  auto row = [&](int r) { return ls.row(r, E); };
+  auto col = [&](int r, int c) { return ls.col(r, c, E); };
   const bool plain = PLAIN == 1 || (PLAIN == 2 && k.plain);
   /* current level c[0..4] = phi_r, phi_i, theta_x, theta_y, theta_z; previous
    * level o[0..4] (read once, then overwritten with level n+1) */
@@ -451,36 +480,34 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
     c[f] = plane_rsrc(L.cur[f]);
     o[f] = plane_rsrc(L.prv[f]);
   }
-  const size_t NYNZ = (size_t)NY * NZ;
   /* current level of field f in x plane x at (row byte offset, lane byte
    * offset); previous level (streaming); store of the new level */
-  auto LC = [&](int f, int x, uint32_t row, uint32_t lo) -> R {
-    if constexpr (BIG) return ldo(L.cur[f] + (size_t)x * NYNZ, row, lo);
-    else return bld<R>(c[f], lo, (uint32_t)x * PLB + row);
+  auto LC = [&](int f, int x, uint32_t ro, uint32_t lo) -> R {
+    if constexpr (BIG) return ldo(L.cur[f] + (size_t)x * NYNZ, ro, lo);
+    else return bld<R>(c[f], lo, (uint32_t)x * PLB + ro);
   };
-  auto LP = [&](int f, int x, uint32_t row, uint32_t lo) -> R {
-    if constexpr (BIG) return ldo((const R *)L.prv[f] + (size_t)x * NYNZ, row, lo);
-    else return bld<R, kStream>(o[f], lo, (uint32_t)x * PLB + row);
+  auto LP = [&](int f, int x, uint32_t ro, uint32_t lo) -> R {
+    if constexpr (BIG) return ldo((const R *)L.prv[f] + (size_t)x * NYNZ, ro, lo);
+    else return bld<R, kStream>(o[f], lo, (uint32_t)x * PLB + ro);
   };
-  auto SP = [&](int f, int x, uint32_t row, uint32_t lo, R v) {
-    if constexpr (BIG) sto(L.prv[f] + (size_t)x * NYNZ, row, lo, v);
-    else bst<R, kStream>(o[f], lo, (uint32_t)x * PLB + row, v);
+  auto SP = [&](int f, int x, uint32_t ro, uint32_t lo, R v) {
+    if constexpr (BIG) sto(L.prv[f] + (size_t)x * NYNZ, ro, lo, v);
+    else bst<R, kStream>(o[f], lo, (uint32_t)x * PLB + ro, v);
   };
+  const uint32_t R0 = row(0), RM = row(-1), RP = row(1);
+  const uint32_t oz = col(0, 0), ozp = col(0, 1), ozm = col(0, -1);          /* in row R0 */
+  const uint32_t pz = col(1, 0), mz = col(-1, 0), mzp = col(-1, 1);          /* in rows RP, RM, RM */
 
-  /* FP32: z+-1 operands come from the neighbouring lanes (DPP) instead of
-   * reloading shifted rows; only the two chunk-edge lanes load: lane 0 phi
-   * at the site before the chunk, lane `last` (the last active lane) phi,
-   * theta_x and theta_y at the site after it (the phi loads of both in the
-   * same instructions, separate ones when the chunk has a single site). */
-  const int z0 = zc * 64;
-  const int last = min(63, NZ - 1 - z0);
-  const bool e0 = lane == 0, eL = lane == last;
-  const uint32_t oe0 = (uint32_t)(z0 == 0 ? NZ - 1 : z0 - 1) * E;              /* site before the chunk */
-  const uint32_t oeL = (uint32_t)(z0 + last + 1 == NZ ? 0 : z0 + last + 1) * E;  /* site after it */
-  const uint32_t oe = e0 ? oe0 : oeL;
-  /* a one-site chunk (NZ = 64 m + 1): lane 0 is both edges and needs both
-   * sites (wave-uniform) */
-  const bool single = last == 0;
+  /* Lanes whose z - 1 (z + 1) site is not the lane before (after) them: the
+   * chunk's ends and, with FLAT, the ends of rows inside it.  FP32 takes z+-1
+   * operands from the neighbouring lanes (DPP) instead of reloading shifted
+   * rows; these lanes load phi there, and theta_x and theta_y at z + 1 (the
+   * phi loads of both in the same instructions, separate ones for a lane
+   * that is both). */
+  const bool e0 = lane == 0 || (FLAT && z == 0);
+  const bool eL = lane == 63 || (FLAT && z == NZ - 1);
+  const bool both = FLAT && e0 && eL;
+  const uint32_t oe = e0 ? ozm : ozp;
   auto load_plane = [&](int x, PlaneOps<R> &d, R PRc_, R PIc_, R TXc_, R TYc_, R TZc_) {
     const int xp = x == NX - 1 ? 0 : x + 1;
     if constexpr (!PF) {
@@ -489,18 +516,18 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
       d.oPR = LP(0, x, R0, oz); d.oPI = LP(1, x, R0, oz);
       d.oX = LP(2, x, R0, oz); d.oY = LP(3, x, R0, oz); d.oZ = LP(4, x, R0, oz);
     }
-    d.PRyp = LC(0, x, RP, oz); d.PIyp = LC(1, x, RP, oz);
-    d.PRym = LC(0, x, RM, oz); d.PIym = LC(1, x, RM, oz);
-    d.TXyp = LC(2, x, RP, oz); d.TZyp = LC(4, x, RP, oz);
-    d.TXym = LC(2, x, RM, oz); d.TYym = LC(3, x, RM, oz); d.TZym = LC(4, x, RM, oz);
-    d.TYxpym = LC(3, xp, RM, oz);
+    d.PRyp = LC(0, x, RP, pz); d.PIyp = LC(1, x, RP, pz);
+    d.PRym = LC(0, x, RM, mz); d.PIym = LC(1, x, RM, mz);
+    d.TXyp = LC(2, x, RP, pz); d.TZyp = LC(4, x, RP, pz);
+    d.TXym = LC(2, x, RM, mz); d.TYym = LC(3, x, RM, mz); d.TZym = LC(4, x, RM, mz);
+    d.TYxpym = LC(3, xp, RM, mz);
     if (sizeof(R) == 8) {
       /* FP64 is issue-bound: the shifts' extra VALU costs more than the
        * reloads (L1 hits) they save; FP32 gains from the fewer requests */
       d.PRzp = LC(0, x, R0, ozp); d.PIzp = LC(1, x, R0, ozp);
       d.PRzm = LC(0, x, R0, ozm); d.PIzm = LC(1, x, R0, ozm);
       d.TXzp = LC(2, x, R0, ozp); d.TYzp = LC(3, x, R0, ozp);
-      d.TYymzp = LC(3, x, RM, ozp);
+      d.TYymzp = LC(3, x, RM, mzp);
       return;
     }
     R ePR = PRc_, ePI = PIc_, eTX = TXc_, eTY = TYc_, eTYym = TYc_;
@@ -508,16 +535,17 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
       ePR = LC(0, x, R0, oe); ePI = LC(1, x, R0, oe);
     }
     if (eL) {
-      eTX = LC(2, x, R0, oeL); eTY = LC(3, x, R0, oeL);
-      eTYym = LC(3, x, RM, oeL);
+      eTX = LC(2, x, R0, ozp); eTY = LC(3, x, R0, ozp);
+      eTYym = LC(3, x, RM, mzp);
     }
-    R pPR = ePR, pPI = ePI;   /* phi after the chunk, for the edge lane */
-    if (single) {
-      pPR = LC(0, x, R0, oeL); pPI = LC(1, x, R0, oeL);
+    R pPR = ePR, pPI = ePI;   /* phi at z + 1 for the lanes eL */
+    if (both) {
+      pPR = LC(0, x, R0, ozp); pPI = LC(1, x, R0, ozp);
     }
-    d.PRzm = lane_prev(PRc_, ePR); d.PIzm = lane_prev(PIc_, ePI);
     /* the shifts run with every lane active (a DPP read of an inactive lane
-     * returns the old operand), then the edge lane takes its own load */
+     * returns the old operand), then the edge lanes take their own loads */
+    const R mPR = lane_prev(PRc_, ePR), mPI = lane_prev(PIc_, ePI);
+    d.PRzm = FLAT && e0 ? ePR : mPR; d.PIzm = FLAT && e0 ? ePI : mPI;
     const R nPR = lane_next(PRc_, ePR), nPI = lane_next(PIc_, ePI), nTX = lane_next(TXc_, eTX);
     const R nTY = lane_next(TYc_, eTY), nTYym = lane_next(d.TYym, eTYym);
     d.PRzp = eL ? pPR : nPR; d.PIzp = eL ? pPI : nPI;
@@ -527,41 +555,50 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
 
   /* ---- prologue: plane x0-1 quantities needed by plane x0 ---- */
   const int xm0 = x0 == 0 ? NX - 1 : x0 - 1;
-  const R *F[5] = {PR, PI, TX, TY, TZ};
   MarchCarry<R> m;
   march_prologue<R>([&](int a, int x, int dy, int dz) {
-    if constexpr (BIG) return ldo(F[a] + (size_t)x * NYNZ, dy ? RP : R0, dz ? ozp : oz);
-    else return ldo(F[a], (uint32_t)x * PLB + (dy ? RP : R0), dz ? ozp : oz);
+    return ldo(L.cur[a] + (size_t)x * NYNZ, dy ? RP : R0, dy ? pz : dz ? ozp : oz);
   }, xm0, x0, m);
-  const R *PRx0 = PR, *PIx0 = PI, *TXx0 = TX, *TYx0 = TY, *TZx0 = TZ;
-  uint32_t b0 = (uint32_t)x0 * PLB;
-  if constexpr (BIG) {
-    const size_t o0 = (size_t)x0 * NYNZ;
-    PRx0 += o0; PIx0 += o0; TXx0 += o0; TYx0 += o0; TZx0 += o0;
-    b0 = 0;
-  }
-  R PRc = ldo(PRx0, b0 + R0, oz), PIc = ldo(PIx0, b0 + R0, oz);
-  R TXc = ldo(TXx0, b0 + R0, oz), TYc = ldo(TYx0, b0 + R0, oz), TZc = ldo(TZx0, b0 + R0, oz);
+  auto first = [&](int f) { return ldo(L.cur[f] + (size_t)x0 * NYNZ, R0, oz); };
+  R PRc = first(0), PIc = first(1), TXc = first(2), TYc = first(3), TZc = first(4);
 
-  /* Lane 0's z-backward values (ZEdge) for EB planes at a time: lane j
-   * evaluates them at (xb + j, y, z0 - 1) with the operands and expressions
+  /* The z-backward values (ZEdge) of the lanes e0 for a block of planes at a
+   * time: lane j evaluates those of edge j mod ne in plane xb + j / ne, at the
+   * site (y, z - 1) before that edge's lane, with the operands and expressions
    * that site's own update uses, into LDS (the workgroup is this one wave).
-   * One vector evaluation per EB planes instead of a sincos and two sines
+   * Edge 0 is lane 0; with FLAT edge e > 0 is the first site of row y0 + e.
+   * One vector evaluation per block instead of a sincos and two sines
    * per plane.  The pass reads its planes' lines ahead of the march; over
    * longer blocks (16 planes: +0.4 GB FP64, +1.7 GB FP32 per 512^3 step)
    * they are evicted from L2 before the march reaches them and are read
    * twice, so the blocks are short.  Measured best: 4 planes in FP32, and
    * in FP64 with the LDS prefetch (512^3: 2 planes 3.697 ms, 3: 3.671, 4:
    * 3.663, 6: 3.668, 8: 3.674, 16: 3.706); 8 in FP64 before it. */
-  constexpr int EB = 4;
-  __shared__ ZEdge<R> zedge[EB];
-  const uint32_t em = R0 + oe0, emP = RP + oe0, ec = R0 + (uint32_t)z0 * E;
+  const int ne = FLAT ? 1 + (int)((min(p0 + 63, NYNZ - 1)) / (uint32_t)NZ) - y0 : 1;
+  const int EB = FLAT ? max(1, min(4, 64 / ne)) : 4;   /* NZ >= 3: ne <= 23 */
+  __shared__ ZEdge<R> zedge[FLAT ? 64 : 4];
+  const int mine = FLAT ? y - y0 : 0;   /* the edge of this lane, where it is one */
+  const int je = FLAT ? lane % ne : 0, jx = FLAT ? lane / ne : lane;
+  uint32_t em = R0, emP = RP, ec = R0;  /* the sites z - 1 in rows y, y + 1, and z, of edge je */
+  if constexpr (FLAT) {
+    const int ey = y0 + je, ez = je ? 0 : (int)(p0 - (uint32_t)y0 * NZ);
+    const int ezm = ez == 0 ? NZ - 1 : ez - 1, eyp = ey == NY - 1 ? 0 : ey + 1;
+    em = ((uint32_t)ey * NZ + ezm) * E;
+    emP = ((uint32_t)eyp * NZ + ezm) * E;
+    ec = ((uint32_t)ey * NZ + ez) * E;
+  } else {
+    const uint32_t z0 = p0 - (uint32_t)y0 * NZ, ezm = (z0 == 0 ? (uint32_t)NZ : z0) - 1;
+    em += ezm * E;
+    emP += ezm * E;
+    ec += z0 * E;
+  }
   auto edge_block = [&](int xb, int xe) {
-    const int xj = min(xb + lane, xe - 1);
+    const int xj = min(xb + jx, xe - 1);
     const int xjp = xj == NX - 1 ? 0 : xj + 1;
     R TZe, TXe, TYe, TZxe, TZye, TX0, TY0;
     if constexpr (BIG) {
       /* per-lane planes: 64-bit element offsets */
+      const R *TX = L.cur[2], *TY = L.cur[3], *TZ = L.cur[4];
       const size_t pj = (size_t)xj * NYNZ, pn = (size_t)xjp * NYNZ;
       const size_t iem = em / E, iemP = emP / E, iec = ec / E;
       TZe = TZ[pj + iem]; TXe = TX[pj + iem]; TYe = TY[pj + iem];
@@ -575,11 +612,11 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
     }
     ZEdge<R> e;
     TrigR<R>::sc(TZe, &e.s, &e.c);
-    e.qxz = TrigR<R>::sn(TXe + TZxe - TX0 - TZe);   /* a_xz at (xj, y, z0 - 1) */
+    e.qxz = TrigR<R>::sn(TXe + TZxe - TX0 - TZe);   /* a_xz at (xj, y, z - 1) */
     e.qyz = TrigR<R>::sn(TYe + TZye - TY0 - TZe);   /* a_yz there */
     e.tz = TZe;
     __syncthreads();   /* the previous block's values have been read */
-    if (lane < xe - xb) zedge[lane] = e;
+    if (jx < xe - xb) zedge[FLAT ? lane : jx] = e;
     __syncthreads();
   };
 
@@ -591,7 +628,7 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
    * phi_r and theta_x directly -- resources chosen at run time are held in
    * scalar registers of their own, which the loop then spills */
   const bool hi = lane >= 32;
-  const uint32_t lz = (uint32_t)(zc * 64) * 8u + 16u * (uint32_t)(lane & 31);
+  const uint32_t lz = p0 * 8u + 16u * (uint32_t)(lane & 31);
   auto pdelta = [&](const void *F, const void *G) -> uint32_t {
     const char *pF = (const char *)F, *pG = (const char *)G;
     return pF < pG ? (hi ? (uint32_t)(pG - pF) : 0u) : (hi ? 0u : (uint32_t)(pF - pG));
@@ -603,7 +640,7 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
   /* plane x's previous level and plane x+1's current level into pf[buf] */
   auto prefetch = [&](int x, int buf) {
     const int xp = x == NX - 1 ? 0 : x + 1;
-    const uint32_t so_ = (uint32_t)x * PLB + R0, sn_ = (uint32_t)xp * PLB + R0;
+    const uint32_t so_ = (uint32_t)x * PLB, sn_ = (uint32_t)xp * PLB;
     const uint32_t s2 = hi ? sn_ : so_;   /* pair 2: plane x (previous level), x+1 (current) */
     __builtin_amdgcn_raw_ptr_buffer_load_lds(o[0], (lds_void *)&pf[buf][0][0], 16, d0 + so_, 0, 0, kStream);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(o[2], (lds_void *)&pf[buf][1][0], 16, d1 + so_, 0, 0, kStream);
@@ -612,7 +649,8 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
     __builtin_amdgcn_raw_ptr_buffer_load_lds(c[2], (lds_void *)&pf[buf][4][0], 16, d4 + sn_, 0, 0, 0);
   };
   if constexpr (PF) prefetch(x0, x0 & 1);
-  double rho_sum = 0, g_sum = 0, bad = 0;   /* MODE 2 */
+  double rho_sum = 0, g_sum = 0;   /* MODE 2 */
+  int bad = 0;
   /* DEFER (FP64): plane x's five stores are issued at the top
    * of plane x+1 (after the prefetched values, where there are any, are
    * read).  Issued at the end of plane x they sit in the memory counter
@@ -631,10 +669,12 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
     SP(1, x, R0, oz, v.PI);
   };
 
+  int next = 0;   /* plane within the edge block (FLAT) */
   for (int x = x0; x < x1; ++x) {
-    const int i = (x - x0) % EB;
+    const int i = FLAT ? next : (x - x0) % 4;
     if (i == 0) edge_block(x, min(x1, x + EB));
-    const ZEdge<R> ze = zedge[i];
+    const ZEdge<R> ze = zedge[FLAT ? i * ne + mine : i];
+    next = i + 1 == EB ? 0 : i + 1;
     PlaneOps<R> D;
     if constexpr (PF) {
       const int buf = x & 1;
@@ -657,13 +697,15 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
     }
     SiteOut<R> out;
     if constexpr (MODE == 0) {
-      ah_site_update<R, POW2>(k, plain, RegOps<R>{D, PRc, PIc, TXc, TYc, TZc}, m, ze, out);
+      ah_site_update<R, POW2, RegOps<R>, false, FLAT>(k, plain, RegOps<R>{D, PRc, PIc, TXc, TYc, TZc}, m, ze, e0, out);
     } else {
       const MarchCarry<R> mb = m;   /* the carry from s-x, before the update advances it */
       SiteTrig<R> tr;
-      ah_site_update<R, POW2, RegOps<R>, true>(k, plain, RegOps<R>{D, PRc, PIc, TXc, TYc, TZc}, m, ze, out, &tr);
-      const size_t si = ((size_t)x * NY + y) * NZ + z;
-      const double TZzm = lane_prev((double)TZc, (double)ze.tz);   /* theta_z(s-z): lane - 1's own */
+      ah_site_update<R, POW2, RegOps<R>, true, FLAT>(k, plain, RegOps<R>{D, PRc, PIc, TXc, TYc, TZc}, m, ze, e0, out,
+                                                     &tr);
+      const size_t si = FLAT ? (size_t)x * NYNZ + p : ((size_t)x * NY + y) * NZ + z;
+      /* theta_z(s-z): lane - 1's own */
+      const double TZzm = z_back<FLAT, double>((double)TZc, (double)ze.tz, e0);
       const double divN = link_div<POW2>(fd.ek, TXc, mb.TXm, TYc, D.TYym, TZc, TZzm);
       if constexpr (MODE == 1) {
         if (act) fd.div[si] = divN;
@@ -679,16 +721,15 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
         const double dY = link_phase_sc(PRc, PIc, D.PRyp, D.PIyp, tr.sy, tr.cy);
         const double dZ = link_phase_sc(PRc, PIc, D.PRzp, D.PIzp, tr.sz, tr.cz);
         if (act) {
-          const size_t V = (size_t)NX * NY * NZ;
+          const size_t V = (size_t)NX * NYNZ;
           fd.phase[si] = (float)(dX + TXc);
           fd.phase[V + si] = (float)(dY + TYc);
           fd.phase[2 * V + si] = (float)(dZ + TZc);
           rho_sum += rho;
           g_sum += fabs(G);
-          const double vals[10] = {PRc, PIc, TXc, TYc, TZc, D.oPR, D.oPI, D.oX, D.oY, D.oZ};
-#pragma unroll
-          for (int q = 0; q < 10; ++q) bad += isfinite(vals[q]) ? 0.0 : 1.0;
         }
+        const double vals[10] = {PRc, PIc, TXc, TYc, TZc, D.oPR, D.oPI, D.oX, D.oY, D.oZ};
+        bad += nonfinite(vals, act);
       }
     }
     if constexpr (DEFER) pend = out;
@@ -699,7 +740,7 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
     if (x1 > x0 && act) store_out(x1 - 1, pend);
   }
   if constexpr (MODE == 2) {
-    const double a = march_wave_sum(rho_sum), b = march_wave_sum(g_sum), c = march_wave_sum(bad);
+    const double a = march_wave_sum(rho_sum), b = march_wave_sum(g_sum), c = (double)bad;
     if (lane == 0) {
       fd.part[3 * (size_t)item] = a;
       fd.part[3 * (size_t)item + 1] = b;

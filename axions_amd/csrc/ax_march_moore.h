@@ -1,8 +1,8 @@
 /*
  * ax_march_moore.h - the Moore-model update (mooreEvol.cpp:202-337: two
  * complex scalars with charges q1, q2 on one U(1) link field, no friction)
- * as a 64-lane wave marching along x over a z chunk of one row, like
- * ah_march.  Same arithmetic and operand order as moore_update in
+ * as a 64-lane wave marching along x over a 64-site chunk of the (y, z)
+ * plane, like ah_march.  Same arithmetic and operand order as moore_update in
  * ax_step.hip; the cos/sin of q_f theta_x(s-x) and the plaquette sines at
  * s-x come from the previous plane of the march, y/z-backward values are
  * recomputed, the six plaquette sines at s are computed once and take the
@@ -86,22 +86,23 @@ inline void moore_consts_from(const StepConsts &k, MooreConsts<R> &m) {
  * dz^2 through FixedDivisor; the caller has checked the current level's
  * band flag.  CHECK: OR 1 into *bad when a written value lies outside the
  * band (every lane of the wave must reach the end). */
-template <typename R, bool POW2, bool BUF = false, bool FASTDIV = false, bool CHECK = false>
-__device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Levels<R> &L, int NX, int NY, int NZ, int y,
-                                            int zc, int x0, int x1, bool zfix = false, int *bad = nullptr) {
+template <typename R, bool POW2, bool BUF, bool FLAT, bool FASTDIV = false, bool CHECK = false>
+__device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Levels<R> &L, int NX, int NY, int NZ,
+                                            uint32_t p0, int x0, int x1, bool xfix = false, bool zfix = false,
+                                            int *bad = nullptr) {
   typedef TrigR<R> T;
-  const int lane = (int)(threadIdx.x & 63);
-  const int zr = zc * 64 + lane;
-  const bool inz = zr < NZ;
-  const int z = inz ? zr : NZ - 1;
-  const bool act = inz && !(zfix && (zr == 0 || zr == NZ - 1));
-  const int ym = y == 0 ? NY - 1 : y - 1, yp = y == NY - 1 ? 0 : y + 1;
+  const uint32_t NYNZ = (uint32_t)NY * (uint32_t)NZ;
+  const LaneSite<FLAT> ls(NY, NZ, p0);
+  const int y = ls.y, z = ls.z;
+  /* xfix, zfix: x and y, z not periodic; their face sites are not stepped */
+  const bool act = ls.act && !(zfix && (z == 0 || z == NZ - 1)) && !(xfix && (y == 0 || y == NY - 1));
   const uint32_t E = (uint32_t)sizeof(R);
-  const uint32_t oz = (uint32_t)z * E;
-  const uint32_t ozm = (uint32_t)(z == 0 ? NZ - 1 : z - 1) * E;
-  const uint32_t ozp = (uint32_t)(z == NZ - 1 ? 0 : z + 1) * E;
-  const uint32_t PLB = (uint32_t)NY * (uint32_t)NZ * E;
-  const uint32_t R0 = (uint32_t)y * NZ * E, RM = (uint32_t)ym * NZ * E, RP = (uint32_t)yp * NZ * E;
+  const uint32_t PLB = NYNZ * E;          /* plane bytes */
+  auto row = [&](int r) { return ls.row(r, E); };
+  auto col = [&](int r, int c) { return ls.col(r, c, E); };
+  const uint32_t R0 = row(0), RM = row(-1), RP = row(1);
+  const uint32_t oz = col(0, 0), ozp = col(0, 1), ozm = col(0, -1);   /* in row R0 */
+  const uint32_t pz = col(1, 0), pzm = col(1, -1), mz = col(-1, 0), mzp = col(-1, 1);   /* in rows RP, RP, RM, RM */
   const R *F[7] = {L.cur[0], L.cur[1], L.cur[2], L.cur[3], L.cur[4], L.cur[5], L.cur[6]};
   R *O[7] = {L.prv[0], L.prv[1], L.prv[2], L.prv[3], L.prv[4], L.prv[5], L.prv[6]};
   const R *TX = F[4], *TY = F[5], *TZ = F[6];
@@ -131,7 +132,6 @@ __device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Level
   /* current-level value of field c in x plane x at (row byte offset ro,
    * lane offset lo); without BUF the plane's 64-bit address is formed on
    * the scalar unit, so planes of any size work */
-  const size_t NYNZ = (size_t)NY * NZ;
   auto LC = [&](int c, int x, uint32_t ro, uint32_t lo) -> R {
     if (BUF) return bld<R>(FR[c], lo, offC + (uint32_t)x * PLB + ro);
     return ldo(F[c] + (size_t)x * NYNZ, ro, lo);
@@ -145,7 +145,7 @@ __device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Level
     for (int c = 0; c < 4; ++c) Pm[c] = LG(F[c], xm0, R0, oz);
     const R X = LG(TX, xm0, R0, oz), Y = LG(TY, xm0, R0, oz), Z = LG(TZ, xm0, R0, oz);
     for (int f = 0; f < 2; ++f) T::sc(q[f] * X, &sxm[f], &cxm[f]);
-    Qyx_m = T::sn(Y + LG(TX, xm0, RP, oz) - LG(TY, x0, R0, oz) - X);
+    Qyx_m = T::sn(Y + LG(TX, xm0, RP, pz) - LG(TY, x0, R0, oz) - X);
     Qzx_m = T::sn(Z + LG(TX, xm0, R0, ozp) - LG(TZ, x0, R0, oz) - X);
   }
   R C[7];
@@ -157,12 +157,12 @@ __device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Level
     R Nx[7];
     for (int c = 0; c < 7; ++c) Nx[c] = LC(c, xp, R0, oz);
     const R X = C[4], Y = C[5], Z = C[6];
-    const R TXyp = LC(4, x, RP, oz), TZyp = LC(6, x, RP, oz);
+    const R TXyp = LC(4, x, RP, pz), TZyp = LC(6, x, RP, pz);
     const R TXzp = LC(4, x, R0, ozp), TYzp = LC(5, x, R0, ozp);
-    const R TXym = LC(4, x, RM, oz), TYym = LC(5, x, RM, oz), TZym = LC(6, x, RM, oz);
-    const R TYxpym = LC(5, xp, RM, oz), TYymzp = LC(5, x, RM, ozp);
+    const R TXym = LC(4, x, RM, mz), TYym = LC(5, x, RM, mz), TZym = LC(6, x, RM, mz);
+    const R TYxpym = LC(5, xp, RM, mz), TYymzp = LC(5, x, RM, mzp);
     const R TXzm = LC(4, x, R0, ozm), TYzm = LC(5, x, R0, ozm), TZzm = LC(6, x, R0, ozm);
-    const R TZxpzm = LC(6, xp, R0, ozm), TZypzm = LC(6, x, RP, ozm);
+    const R TZxpzm = LC(6, xp, R0, ozm), TZypzm = LC(6, x, RP, pzm);
 
     /* plaquette sines (mooreEvol.cpp:310-333 operand order) */
     const R a_xy = X + Nx[5] - TXyp - Y;
@@ -211,8 +211,8 @@ __device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Level
       T::sc(q[f] * TZzm, &szm, &czm);
       const R ar = C[cr], ai = C[ci];
       const R rxp = Nx[cr], ixp = Nx[ci];
-      const R ryp = LC(cr, x, RP, oz), iyp = LC(ci, x, RP, oz);
-      const R rym = LC(cr, x, RM, oz), iym = LC(ci, x, RM, oz);
+      const R ryp = LC(cr, x, RP, pz), iyp = LC(ci, x, RP, pz);
+      const R rym = LC(cr, x, RM, mz), iym = LC(ci, x, RM, mz);
       const R rzp = LC(cr, x, R0, ozp), izp = LC(ci, x, R0, ozp);
       const R rzm = LC(cr, x, R0, ozm), izm = LC(ci, x, R0, ozm);
       {

@@ -62,7 +62,7 @@ struct BatchEntry {
   uint64_t base;        /* device address of plane (component 0, level 0) */
   uint64_t pitch;       /* elements from one plane to the next */
   int32_t n;            /* lattice edge (n^3 sites) */
-  int32_t nw, xseg, nseg;
+  int32_t nc, xseg, nseg;   /* 64-site chunks of a plane; planes per segment; segments */
   int32_t work_begin;   /* first work item of this lattice */
   int32_t t0;           /* TimeStep at the start of the chunk */
   int32_t steps;        /* TimeSteps to take in this chunk (<= chunk length) */
@@ -107,7 +107,7 @@ __device__ __forceinline__ Levels<R> entry_levels(const BatchEntry &E, int t) {
 }
 
 template <typename R, bool POW2>
-__global__ void __launch_bounds__(64) pool_step_kernel(ax_params p, R lim, const BatchHeader *__restrict__ hdr,
+__global__ void __launch_bounds__(64, sizeof(R) == 8 ? 3 : 5) pool_step_kernel(ax_params p, R lim, const BatchHeader *__restrict__ hdr,
                                                        const BatchEntry *__restrict__ ent, int j) {
   const int count = hdr->count, work = hdr->work;
   /* XCD-aware order: the grid is resident at once and its workgroups are
@@ -126,13 +126,17 @@ __global__ void __launch_bounds__(64) pool_step_kernel(ax_params p, R lim, const
     const BatchEntry E = ent[e];
     if (j >= E.steps) continue;
     const int local = it - E.work_begin;
-    const int zc = local % E.nw, r = local / E.nw;
-    const int y = r % E.n, seg = r / E.n;
+    const int seg = local / E.nc, chunk = local - seg * E.nc;
     const int x0 = seg * E.xseg, x1 = min(E.n, x0 + E.xseg);
     const int t = E.t0 + j;
     MarchConsts<R> m;
     march_consts_from<R>(make_step_consts(p, t), lim, m);
-    ah_march<R, POW2, 2>(m, entry_levels<R>(E, t), E.n, E.n, E.n, y, zc, x0, x1);
+    const Levels<R> L = entry_levels<R>(E, t);
+    const uint32_t p0 = (uint32_t)chunk * 64;
+    /* FP64 takes chunks across rows for every n: both forms in one kernel
+     * would spill */
+    if (sizeof(R) == 8 || E.n % 64) ah_march<R, POW2, 2, false, false, 0, false, true>(m, L, E.n, E.n, E.n, p0, x0, x1);
+    else ah_march<R, POW2, 2>(m, L, E.n, E.n, E.n, p0, x0, x1);
   }
 }
 
@@ -187,11 +191,10 @@ __global__ void __launch_bounds__(64) pool_wind_pass_kernel(const BatchHeader *_
       ce = e;
     }
     const int local = it - E.work_begin;
-    const int zc = local % E.nw, r = local / E.nw;
-    const int y = r % E.n, seg = r / E.n;
+    const int seg = local / E.nc, chunk = local - seg * E.nc;
     const int x0 = seg * E.xseg, x1 = min(E.n, x0 + E.xseg);
     const Levels<T> L = entry_levels<T>(E, E.t0 + (which == 0 ? 0 : E.steps));   /* state after t TimeSteps */
-    const WindRow row(E.n, E.n, E.n, y, zc);
+    const WindRow row(E.n, E.n, E.n, chunk);
     if (WIND) {
       wind_march(row, (const float *)E.phase, x0, x1, [&](int, size_t, const int *wn) {
 #pragma unroll
@@ -533,7 +536,7 @@ int ax_pool::enqueue_chunk() {
     E.base = (uint64_t)(uintptr_t)(arena_base + r.off);
     E.pitch = lattice_pitch(V, esize, pad_bytes);
     E.n = r.n;
-    E.nw = (r.n + 63) / 64;
+    E.nc = tile_chunks(r.n, r.n);
     E.xseg = (r.xseg <= 0 || r.xseg > r.n) ? r.n : r.xseg;
     E.nseg = (r.n + E.xseg - 1) / E.xseg;
     E.work_begin = work;
@@ -542,7 +545,7 @@ int ax_pool::enqueue_chunk() {
     E.pre = r.pre_done ? 0 : 1;
     E.pad[0] = E.pad[1] = 0;
     E.phase = (uint64_t)(uintptr_t)(arena_base + r.off + lattice_phase_offset(r.n, esize, pad_bytes));
-    work += E.nw * r.n * E.nseg;
+    work += E.nc * E.nseg;
     c.items.push_back({id, E.t0, E.steps, E.pre});
     c.site_updates += (double)V * E.steps;
     if (r.wait_upload) {
@@ -560,7 +563,7 @@ int ax_pool::enqueue_chunk() {
     std::vector<int> nn(count), nw(count), xs(count);
     for (int k = 0; k < count; ++k) {
       nn[k] = ent[k].n;
-      nw[k] = ent[k].nw;
+      nw[k] = (ent[k].n + 63) / 64;
       xs[k] = ent[k].xseg;
     }
     fill_segments(count, nn.data(), nw.data(), xs.data(), 2LL * grid_step);
@@ -570,7 +573,7 @@ int ax_pool::enqueue_chunk() {
       E.xseg = xs[k];
       E.nseg = (E.n + E.xseg - 1) / E.xseg;
       E.work_begin = work;
-      work += E.nw * E.n * E.nseg;
+      work += E.nc * E.nseg;
     }
   }
   h->count = count;
@@ -793,20 +796,20 @@ int ax_pool::tune(int n, int *xseg, double *ms) {
     std::fill(tab.begin(), tab.end(), 0);
     BatchHeader *h = (BatchHeader *)tab.data();
     BatchEntry *ent = (BatchEntry *)(tab.data() + 64);
-    const int nw = (n + 63) / 64, nseg = (n + cand[ci] - 1) / cand[ci];
+    const int nc = tile_chunks(n, n), nseg = (n + cand[ci] - 1) / cand[ci];
     for (int k = 0; k < m; ++k) {
       BatchEntry *E = ent + k;
       E->base = (uint64_t)(uintptr_t)(base + (size_t)k * LB);
       E->pitch = pitch;
       E->n = n;
-      E->nw = nw;
+      E->nc = nc;
       E->xseg = cand[ci];
       E->nseg = nseg;
-      E->work_begin = k * nw * n * nseg;
+      E->work_begin = k * nc * nseg;
       E->steps = 1 << 30;
     }
     h->count = m;
-    h->work = m * nw * n * nseg;
+    h->work = m * nc * nseg;
     e = hipMemcpyAsync(dh, tab.data(), tab_bytes, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     for (int rep = 0; rep < reps && e == hipSuccess; ++rep) {

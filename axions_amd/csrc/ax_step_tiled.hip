@@ -1,9 +1,9 @@
 /*
  * ax_step_tiled.hip - Abelian-Higgs and Moore steps of one lattice, one
- * 64-lane wave per (64-site z chunk, y row, x segment) marching along x (the
- * updates themselves are ah_march in ax_march.h and moore_march in
- * ax_march_moore.h).  FP64 and FP32, every boundary (boundary planes and rows
- * are left to the boundary kernels).
+ * 64-lane wave per (chunk of 64 sites of the (y, z) plane, x segment) marching
+ * along x (the updates themselves are ah_march in ax_march.h and moore_march
+ * in ax_march_moore.h).  FP64 and FP32, every boundary (boundary planes and
+ * rows are left to the boundary kernels).
  *
  * Work items are numbered in the XCD-aware order of make_tile_grid
  * (ax_internal.h): each XCD takes bands of consecutive rows with all their
@@ -18,31 +18,29 @@
 
 namespace ax {
 
-/* The planes [x0, x1) and row y a work item steps; with non-periodic x/y
- * (ex) the boundary planes and rows are left alone (their neighbours would
- * wrap), evolution.cpp:161-186.  Returns false for an empty item. */
-__device__ __forceinline__ bool tile_range(const TileGrid &g, int nx, int ny, int ex, int w, int &zc, int &y,
-                                           int &x0, int &x1) {
+/* The chunk and the planes [x0, x1) a work item steps; with non-periodic x/y
+ * (ex) the boundary planes are left alone (their neighbours would wrap),
+ * evolution.cpp:161-186.  Returns false for an empty item. */
+__device__ __forceinline__ bool tile_range(const TileGrid &g, int nx, int ex, int w, int &chunk, int &x0, int &x1) {
   int seg;
-  tile_item(g, ny, w, zc, y, seg);
+  if (!tile_item(g, w, chunk, seg)) return false;
   x0 = seg * g.xseg;
   x1 = min(nx, x0 + g.xseg);
   if (ex) {
     x0 = max(x0, 1);
     x1 = min(x1, nx - 1);
-    if (y == 0 || y == ny - 1) return false;
   }
   return x0 < x1;
 }
 
-template <typename R, bool POW2, bool PLAIN, bool BIG, bool PF = false>
-__global__ void __launch_bounds__(64) ah_tiled_kernel(MarchConsts<R> k, Levels<R> L, int nx, int ny, int nz,
+template <typename R, bool POW2, bool PLAIN, bool BIG, bool PF, bool FLAT>
+__global__ void __launch_bounds__(64, sizeof(R) == 8 ? 3 : 1) ah_tiled_kernel(MarchConsts<R> k, Levels<R> L, int nx, int ny, int nz,
                                                       TileGrid g, int ex, int ez) {
-  const int w = (int)blockIdx.x;
-  if (w >= g.work) return;
-  int zc, y, x0, x1;
-  if (!tile_range(g, nx, ny, ex, w, zc, y, x0, x1)) return;
-  ah_march<R, POW2, PLAIN ? 1 : 0, BIG, PF>(k, L, nx, ny, nz, y, zc, x0, x1, ez != 0);
+  int chunk, x0, x1;
+  if (!tile_range(g, nx, ex, (int)blockIdx.x, chunk, x0, x1)) return;
+  const uint32_t p0 = (uint32_t)chunk * 64;
+  if (!FLAT && ex && (p0 < (uint32_t)nz || p0 >= (uint32_t)nz * (ny - 1))) return;   /* a boundary row */
+  ah_march<R, POW2, PLAIN ? 1 : 0, BIG, PF, 0, false, FLAT>(k, L, nx, ny, nz, p0, x0, x1, ex != 0, ez != 0);
 }
 
 /* FD: FP64 with divisors in the FixedDivisor range on a periodic lattice.
@@ -50,23 +48,23 @@ __global__ void __launch_bounds__(64) ah_tiled_kernel(MarchConsts<R> k, Levels<R
  * TimeStep mod 3: this step (TimeStep t) divides through FixedDivisor when
  * use_band is set and band[t % 3] is clear, ORs its output's check into
  * band[(t + 1) % 3] and clears band[(t + 2) % 3] for the next step. */
-template <typename R, bool POW2, bool BUF, bool FD>
+template <typename R, bool POW2, bool BUF, bool FD, bool FLAT>
 __global__ void __launch_bounds__(64, 3) moore_tiled_kernel(MooreConsts<R> k, Levels<R> L, int nx, int ny, int nz,
                                                          TileGrid g, int ex, int ez, int *band, int t,
                                                          int use_band) {
-  const int w = (int)blockIdx.x;
-  if (FD && w == 0 && threadIdx.x == 0) band[(t + 2) % 3] = 0;
-  if (w >= g.work) return;
-  int zc, y, x0, x1;
-  if (!tile_range(g, nx, ny, ex, w, zc, y, x0, x1)) return;
+  if (FD && blockIdx.x == 0 && threadIdx.x == 0) band[(t + 2) % 3] = 0;
+  int chunk, x0, x1;
+  if (!tile_range(g, nx, ex, (int)blockIdx.x, chunk, x0, x1)) return;
+  const uint32_t p0 = (uint32_t)chunk * 64;
+  if (!FLAT && ex && (p0 < (uint32_t)nz || p0 >= (uint32_t)nz * (ny - 1))) return;   /* a boundary row */
   if constexpr (FD) {
     int *out = band + (t + 1) % 3;
     if (use_band && band[t % 3] == 0)
-      moore_march<R, POW2, BUF, true, true>(k, L, nx, ny, nz, y, zc, x0, x1, ez != 0, out);
+      moore_march<R, POW2, BUF, FLAT, true, true>(k, L, nx, ny, nz, p0, x0, x1, false, false, out);
     else
-      moore_march<R, POW2, BUF, false, true>(k, L, nx, ny, nz, y, zc, x0, x1, ez != 0, out);
+      moore_march<R, POW2, BUF, FLAT, false, true>(k, L, nx, ny, nz, p0, x0, x1, false, false, out);
   } else {
-    moore_march<R, POW2, BUF>(k, L, nx, ny, nz, y, zc, x0, x1, ez != 0);
+    moore_march<R, POW2, BUF, FLAT>(k, L, nx, ny, nz, p0, x0, x1, ex != 0, ez != 0);
   }
 }
 
@@ -91,15 +89,21 @@ hipError_t launch_step_tiled_moore(const StepConsts &k, const Levels<R> &L, int 
                   moore_band_charge((int)k.q2) && getenv("AX_MOORE_PLAIN_DIV") == nullptr;
   *fd_used = fd;
   dim3 grid(g.work), block(64);
-#define AX_MRL(P2, B, FD)                                                                                     \
-  hipLaunchKernelGGL((moore_tiled_kernel<R, P2, B, FD>), grid, block, 0, st, m, L, k.nx, k.ny, k.nz, g, k.ex, k.ez, \
+  const bool flat = k.nz % 64 != 0;   /* as launch_step_tiled_ah */
+#define AX_MRK(P2, B, FD, FL)                                                                                      \
+  hipLaunchKernelGGL((moore_tiled_kernel<R, P2, B, FD, FL>), grid, block, 0, st, m, L, k.nx, k.ny, k.nz, g, k.ex, k.ez, \
                      band, t, use_band ? 1 : 0)
+#define AX_MRL(P2, B, FD)                  \
+  do {                                     \
+    if (flat) AX_MRK(P2, B, FD, true);     \
+    else AX_MRK(P2, B, FD, false);         \
+  } while (0)
   if (pow2 && buf) AX_MRL(true, true, false);
   else if (pow2) AX_MRL(true, false, false);
   else if (buf && fd) AX_MRL(false, true, true);
   else if (buf) AX_MRL(false, true, false);
-  else if (fd) AX_MRL(false, false, true);
   else AX_MRL(false, false, false);
+#undef AX_MRK
 #undef AX_MRL
   return hipGetLastError();
 }
@@ -134,9 +138,10 @@ int default_xseg(const ax_params &p) {
   return f32 ? (xs + 1) / 2 : xs;
 }
 
-/* The LDS prefetch of the FP64 march applies: whole 64-site chunks, three
- * field planes within 32-bit offsets, and the [comp][level] plane order its
- * phi and theta_x/theta_y pairs rely on (AX_NO_PREFETCH turns it off). */
+/* The LDS prefetch of the FP64 march applies: whole 64-site chunks (across
+ * rows it costs registers that spill: 200^3 251 us against 245 without),
+ * three field planes within 32-bit offsets, and the [comp][level] plane order
+ * its phi and theta_x/theta_y pairs rely on (AX_NO_PREFETCH turns it off). */
 template <typename R>
 static bool prefetch_ok(const StepConsts &k, const Levels<R> &L) {
   const bool order = L.cur[0] < L.cur[1] && L.cur[2] < L.cur[3] && L.prv[0] < L.prv[1] && L.prv[2] < L.prv[3];
@@ -155,37 +160,38 @@ hipError_t launch_step_tiled_ah(const StepConsts &k, const Levels<R> &L, int xse
    * forces it on smaller lattices, for tests) */
   const bool big = (size_t)k.nx * k.ny * k.nz * sizeof(R) >= ((size_t)1 << 32) || getenv("AX_BIG_PLANES") != nullptr;
   dim3 grid(g.work), block(64);
-#define AX_AHL(P2, PL, BG) \
-  hipLaunchKernelGGL((ah_tiled_kernel<R, P2, PL, BG>), grid, block, 0, st, m, L, k.nx, k.ny, k.nz, g, k.ex, k.ez)
   /* FP64, whole chunks and three planes within 32-bit offsets: the
    * previous level and the next plane are prefetched into LDS (ah_march; its
    * phi and theta_x/theta_y pairs rely on the [comp][level] plane order).
-   * Every variant keeps 3 waves per SIMD with it (161 VGPRs, with the stores
-   * issued one plane late). */
+   * Every variant keeps 3 waves per SIMD with it, with the stores issued one
+   * plane late. */
   const bool pf = sizeof(R) == 8 && !big && prefetch_ok(k, L);
-#define AX_AHPF(P2, PL)                                                                                     \
-  hipLaunchKernelGGL((ah_tiled_kernel<double, P2, PL, false, true>), grid, block, 0, st, m, L, k.nx, k.ny, k.nz, g, \
-                     k.ex, k.ez)
+  /* rows of whole chunks, whose row offsets stay scalars, else chunks across
+   * rows.  us per step with partial chunks at the row ends / across rows:
+   * FP64 101^3 50 / 43, 200^3 290 / 245, 300^3 949 / 781, 201x201x51 90 / 76;
+   * FP32 101^3 33 / 24, 200^3 162 / 121, 300^3 582 / 417 (those lattices'
+   * rows now keep to one XCD too) */
+  const bool flat = k.nz % 64 != 0;
+#define AX_AHK(P2, PL, BG, PF, FL)                                                                             \
+  hipLaunchKernelGGL((ah_tiled_kernel<R, P2, PL, BG, PF, FL>), grid, block, 0, st, m, L, k.nx, k.ny, k.nz, g, k.ex, \
+                     k.ez)
+#define AX_AHL(BG, PF, FL)                          \
+  do {                                              \
+    if (pow2 && m.plain) AX_AHK(true, true, BG, PF, FL);  \
+    else if (pow2) AX_AHK(true, false, BG, PF, FL);       \
+    else if (m.plain) AX_AHK(false, true, BG, PF, FL);    \
+    else AX_AHK(false, false, BG, PF, FL);                \
+  } while (0)
   if (pf) {
-    if constexpr (sizeof(R) == 8) {
-      if (pow2 && m.plain) AX_AHPF(true, true);
-      else if (pow2) AX_AHPF(true, false);
-      else if (m.plain) AX_AHPF(false, true);
-      else AX_AHPF(false, false);
-    }
+    if constexpr (sizeof(R) == 8) AX_AHL(false, true, false);
   } else if (big) {
-    if (pow2 && m.plain) AX_AHL(true, true, true);
-    else if (pow2) AX_AHL(true, false, true);
-    else if (m.plain) AX_AHL(false, true, true);
-    else AX_AHL(false, false, true);
+    AX_AHL(true, false, true);   /* its row offsets in the lane whatever nz: 168 VGPRs, else 199 */
   } else {
-    if (pow2 && m.plain) AX_AHL(true, true, false);
-    else if (pow2) AX_AHL(true, false, false);
-    else if (m.plain) AX_AHL(false, true, false);
+    if (flat) AX_AHL(false, false, true);
     else AX_AHL(false, false, false);
   }
 #undef AX_AHL
-#undef AX_AHPF
+#undef AX_AHK
   return hipGetLastError();
 }
 
@@ -194,14 +200,17 @@ hipError_t launch_step_tiled_ah(const StepConsts &k, const Levels<R> &L, int xse
  * ah_march.  One partial-sum triple per work item (MODE 2).  PF: the LDS
  * prefetch of the plain step (MODE 1 keeps 3 waves per SIMD with it, 167
  * VGPRs; MODE 2 runs at 2 either way). */
-template <bool POW2, bool P2D, int MODE, bool PF>
-__global__ void __launch_bounds__(64) ah_fused_kernel(MarchConsts<double> k, Levels<double> L, int nx, int ny, int nz,
+template <bool POW2, bool P2D, int MODE, bool PF, bool FLAT>
+__global__ void __launch_bounds__(64, MODE == 1 ? 3 : 2) ah_fused_kernel(MarchConsts<double> k, Levels<double> L, int nx, int ny, int nz,
                                                       TileGrid g, FusedDiag fd) {
   const int w = (int)blockIdx.x;
-  if (w >= g.work) return;
-  int zc, y, x0, x1;
-  if (!tile_range(g, nx, ny, 0, w, zc, y, x0, x1)) return;
-  ah_march<double, POW2, 2, false, PF, MODE, P2D>(k, L, nx, ny, nz, y, zc, x0, x1, false, fd, w);
+  int chunk, x0, x1;
+  if (!tile_range(g, nx, 0, w, chunk, x0, x1)) {
+    if (MODE == 2 && threadIdx.x < 3) fd.part[3 * (size_t)w + threadIdx.x] = 0;
+    return;
+  }
+  ah_march<double, POW2, 2, false, PF, MODE, P2D, FLAT>(k, L, nx, ny, nz, (uint32_t)chunk * 64, x0, x1, false, false, fd,
+                                                        w);
 }
 
 int fused_work_items(int nx, int ny, int nz, int xseg) { return make_tile_grid(nx, ny, nz, xseg).work; }
@@ -215,10 +224,14 @@ hipError_t launch_step_fused(const StepConsts &k, const Levels<double> &L, int x
   /* the plain step's prefetch conditions (launch_step_tiled_ah) */
   const bool pf = prefetch_ok(k, L);
   dim3 grid(g.work), block(64);
-#define AX_FL(P2, PD, MD)                                                                                      \
-  do {                                                                                                         \
-    if (pf) hipLaunchKernelGGL((ah_fused_kernel<P2, PD, MD, true>), grid, block, 0, st, m, L, k.nx, k.ny, k.nz, g, fd); \
-    else hipLaunchKernelGGL((ah_fused_kernel<P2, PD, MD, false>), grid, block, 0, st, m, L, k.nx, k.ny, k.nz, g, fd); \
+  const bool flat = k.nz % 64 != 0;
+#define AX_FK(P2, PD, MD, PF, FL)                                                                               \
+  hipLaunchKernelGGL((ah_fused_kernel<P2, PD, MD, PF, FL>), grid, block, 0, st, m, L, k.nx, k.ny, k.nz, g, fd)
+#define AX_FL(P2, PD, MD)                          \
+  do {                                             \
+    if (pf) AX_FK(P2, PD, MD, true, false);        \
+    else if (flat) AX_FK(P2, PD, MD, false, true); \
+    else AX_FK(P2, PD, MD, false, false);          \
   } while (0)
   if (mode == 1) {
     if (pow2) AX_FL(true, false, 1);
@@ -229,6 +242,7 @@ hipError_t launch_step_fused(const StepConsts &k, const Levels<double> &L, int x
     else AX_FL(false, false, 2);
   }
 #undef AX_FL
+#undef AX_FK
   return hipGetLastError();
 }
 

@@ -19,7 +19,8 @@
 #define AXIONS_AX_WIND_H
 
 #include "ax_device.h"
-#include "ax_march.h"   /* ldo */
+#include "ax_internal.h"   /* LaneSite */
+#include "ax_march.h"      /* ldo */
 
 namespace ax {
 
@@ -80,34 +81,29 @@ __device__ __forceinline__ void site_winding(int nx, int ny, int nz, const T *fr
   }
 }
 
-/* One 64-lane wave per (64-site z chunk zc, row y), marching along x over
- * the planes [x0, x1): lane l holds z = 64 zc + l (lanes past the row end
- * load the row's last site and emit nothing).  Plane x+1's values are loaded
- * once, as the next plane's centre, and carried; the y+1 and z+1 operands
- * are rows that neighbouring waves load too.  Plane addresses are formed on
- * the scalar unit (64-bit), row and lane offsets are 32-bit bytes. */
-struct WindRow {
-  int nx, ny, nz, y, z;
-  bool act;
+/* One 64-lane wave per chunk of 64 sites of the (y, z) plane (LaneSite),
+ * marching along x over the planes [x0, x1); lanes past the plane's end emit
+ * nothing.  Plane x+1's values are loaded once, as the next plane's centre,
+ * and carried; the y+1 and z+1 operands are rows that neighbouring waves load
+ * too.  Plane addresses are formed on the scalar unit (64-bit), offsets in
+ * the plane are 32-bit bytes. */
+struct WindRow : LaneSite<true> {
+  int nx;
   size_t nynz, V;
-  uint32_t r0, rp, z0, zp;   /* element offsets: row y, row y+1, lane z, z+1 */
-  __device__ WindRow(int nx_, int ny_, int nz_, int y_, int zc) : nx(nx_), ny(ny_), nz(nz_), y(y_) {
-    const int zr = zc * 64 + (int)(threadIdx.x & 63);
-    act = zr < nz;
-    z = act ? zr : nz - 1;
-    nynz = (size_t)ny * nz;
+  uint32_t o0, oy, oz;   /* element offsets of the site, y+1 and z+1 */
+  __device__ WindRow(int nx_, int ny_, int nz_, int chunk) : LaneSite<true>(ny_, nz_, (uint32_t)chunk * 64), nx(nx_) {
+    nynz = (size_t)ny_ * nz_;
     V = (size_t)nx * nynz;
-    r0 = (uint32_t)(y * nz);
-    rp = (uint32_t)((y == ny - 1 ? 0 : y + 1) * nz);
-    z0 = (uint32_t)z;
-    zp = (uint32_t)(z == nz - 1 ? 0 : z + 1);
+    o0 = p;
+    oy = col(1, 0, 1);
+    oz = col(0, 1, 1);
   }
-  /* field b (element type E) in x plane x at element offsets row, lane */
+  /* field b (element type E) in x plane x at element offset o */
   template <typename E>
-  __device__ double at(const E *b, int x, uint32_t row, uint32_t lane) const {
-    return (double)ldo(b + (size_t)x * nynz, row * (uint32_t)sizeof(E), lane * (uint32_t)sizeof(E));
+  __device__ double get(const E *b, int x, uint32_t o) const {
+    return (double)ldo(b + (size_t)x * nynz, 0u, o * (uint32_t)sizeof(E));
   }
-  __device__ size_t site(int x) const { return ((size_t)x * ny + y) * nz + z; }
+  __device__ size_t site(int x) const { return (size_t)x * nynz + p; }
 };
 
 /* The marching passes store, per edge, e_a(s) = delta_a(s) + theta_a(s)
@@ -136,14 +132,14 @@ struct WindRow {
 template <typename T>
 __device__ __forceinline__ int phase_march(const WindRow &w, const T *fr, const T *fi, const T *tx, const T *ty,
                                            const T *tz, float *E, int x0, int x1, double q = 1.0) {
-  double cr = w.at(fr, x0, w.r0, w.z0), ci = w.at(fi, x0, w.r0, w.z0);
+  double cr = w.get(fr, x0, w.o0), ci = w.get(fi, x0, w.o0);
   int bad = 0;
   for (int x = x0; x < x1; ++x) {
     const int xp = x == w.nx - 1 ? 0 : x + 1;
-    const double nr = w.at(fr, xp, w.r0, w.z0), ni = w.at(fi, xp, w.r0, w.z0);
-    const double yr = w.at(fr, x, w.rp, w.z0), yi = w.at(fi, x, w.rp, w.z0);
-    const double zr = w.at(fr, x, w.r0, w.zp), zi = w.at(fi, x, w.r0, w.zp);
-    const double X = q * w.at(tx, x, w.r0, w.z0), Y = q * w.at(ty, x, w.r0, w.z0), Z = q * w.at(tz, x, w.r0, w.z0);
+    const double nr = w.get(fr, xp, w.o0), ni = w.get(fi, xp, w.o0);
+    const double yr = w.get(fr, x, w.oy), yi = w.get(fi, x, w.oy);
+    const double zr = w.get(fr, x, w.oz), zi = w.get(fi, x, w.oz);
+    const double X = q * w.get(tx, x, w.o0), Y = q * w.get(ty, x, w.o0), Z = q * w.get(tz, x, w.o0);
     const double dX = link_phase(cr, ci, nr, ni, X);
     const double dY = link_phase(cr, ci, yr, yi, Y);
     const double dZ = link_phase(cr, ci, zr, zi, Z);
@@ -166,13 +162,13 @@ __device__ __forceinline__ int phase_march(const WindRow &w, const T *fr, const 
 template <typename Emit>
 __device__ __forceinline__ void wind_march(const WindRow &w, const float *E, int x0, int x1, Emit emit) {
   const float *EX = E, *EY = E + w.V, *EZ = E + 2 * w.V;
-  double cX = w.at(EX, x0, w.r0, w.z0), cY = w.at(EY, x0, w.r0, w.z0), cZ = w.at(EZ, x0, w.r0, w.z0);
+  double cX = w.get(EX, x0, w.o0), cY = w.get(EY, x0, w.o0), cZ = w.get(EZ, x0, w.o0);
   for (int x = x0; x < x1; ++x) {
     const int xp = x == w.nx - 1 ? 0 : x + 1;
     /* plane x+1 (next centre), row y+1, site z+1 */
-    const double nX = w.at(EX, xp, w.r0, w.z0), nY = w.at(EY, xp, w.r0, w.z0), nZ = w.at(EZ, xp, w.r0, w.z0);
-    const double yX = w.at(EX, x, w.rp, w.z0), yZ = w.at(EZ, x, w.rp, w.z0);
-    const double zX = w.at(EX, x, w.r0, w.zp), zY = w.at(EY, x, w.r0, w.zp);
+    const double nX = w.get(EX, xp, w.o0), nY = w.get(EY, xp, w.o0), nZ = w.get(EZ, xp, w.o0);
+    const double yX = w.get(EX, x, w.oy), yZ = w.get(EZ, x, w.oy);
+    const double zX = w.get(EX, x, w.oz), zY = w.get(EY, x, w.oz);
     int wn[3];
     wn[0] = (int)rint((cX + nY - yX - cY) * 0.15915494309189535);   /* (a, b) = (x, y) */
     wn[1] = (int)rint((cX + nZ - zX - cZ) * 0.15915494309189535);   /* (x, z) */
