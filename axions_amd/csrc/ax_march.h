@@ -26,8 +26,8 @@
  * Each field value is loaded once per step by the wave that owns it: plane
  * x+1 (current level) is loaded as the next iteration's centre and carried;
  * the y/z neighbour rows are meant to be cache hits (at 512^3 FP64 the L2 ->
- * fabric reads are 1.25x the algorithmic bytes without the LDS prefetch
- * below and 1.6x with it, part of them served by the Infinity Cache).  The loop's loads and stores are raw
+ * fabric reads are 1.23x the algorithmic bytes, part of them served by the
+ * Infinity Cache).  The loop's loads and stores are raw
  * buffer accesses (bld/bst below) whose addresses cost no vector
  * instructions; the previous level's reads and the new level's writes carry
  * the streaming hint so that they do not push those rows out of L2.
@@ -402,19 +402,30 @@ __device__ __forceinline__ void march_prologue(Get G, int xm0, int x0, MarchCarr
  * offsets (one x plane of NY*NZ values is far below 4 GiB). */
 typedef __attribute__((address_space(3))) void lds_void;
 
+/* 16 bytes of each lane, from voff + soff, straight into 1 KiB of LDS. */
+template <int AUX>
+__device__ __forceinline__ void row_pair(__amdgpu_buffer_rsrc_t r, double *lds, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)lds, 16, (int)voff, (int)soff, 0, AUX);
+}
+
 /* FLAT: the wave's 64 sites cross rows (LaneSite); otherwise they are of one
  * row, nz a multiple of 64.
  *
  * PF (FP64, not FLAT, planes small enough that three of them fit 32-bit
- * offsets): the ten values of a plane that come from HBM -- the
- * previous level at (x, y) and the current level at (x+1, y) -- are loaded
- * one plane ahead straight into LDS (16 bytes per lane: lanes 0-31 carry
- * one field's 64 sites, lanes 32-63 another's), so their latency overlaps
- * the previous plane's arithmetic without holding VGPRs.  The pairs
- * (previous phi_r, phi_i), (previous theta_x, theta_y), (previous theta_z,
- * current theta_z at x+1), (current phi_r, phi_i at x+1), (current theta_x,
- * theta_y at x+1) each lie within 4 GiB of their lower plane, whose buffer
- * resource the pair's load uses.  Measured at 512^3: 3.747 -> 3.713 ms. */
+ * offsets): the 19 rows a plane reads -- its previous level, its y-neighbour
+ * rows, plane x+1's own row and its theta_y one row back -- are loaded one
+ * plane ahead straight into LDS, two rows per request (16 bytes per lane:
+ * lanes 0-31 one row's 64 sites, lanes 32-63 another's; a request costs the
+ * address unit the same 14 cycles as one row of 8 bytes per lane), and z+-1
+ * operands come from the neighbouring lanes, their chunk-edge values from the
+ * edge pass.  So a plane takes 10 load requests (22 with the five rows from
+ * HBM alone in LDS), no load's latency is exposed, and y-neighbour rows are
+ * read one plane after their own wave reads them, not two: 512^3 L2 -> fabric
+ * reads 15.5 -> 13.2 GB per step, 3.755 -> 3.625 ms; 256^3 496 -> 474 us (the
+ * five rows: 3.747 -> 3.713 ms over none).  What bounds it then is the FP64
+ * arithmetic: 84 % of the issue slots, at the 1.7 GHz the card holds under
+ * it.  FP32, four rows per request, stays at its fabric bandwidth: 512^3
+ * 1.735 ms against 1.723 from registers. */
 /* MODE (FP64, periodic): 0 the step alone; 1 the step also stores the
  * divergence of its current level's links (FusedDiag::div), which the next
  * step's diagnostics need for level n-1 once that level is overwritten; 2
@@ -510,12 +521,10 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
   const uint32_t oe = e0 ? ozm : ozp;
   auto load_plane = [&](int x, PlaneOps<R> &d, R PRc_, R PIc_, R TXc_, R TYc_, R TZc_) {
     const int xp = x == NX - 1 ? 0 : x + 1;
-    if constexpr (!PF) {
-      d.PRn = LC(0, xp, R0, oz); d.PIn = LC(1, xp, R0, oz);
-      d.TXn = LC(2, xp, R0, oz); d.TYn = LC(3, xp, R0, oz); d.TZn = LC(4, xp, R0, oz);
-      d.oPR = LP(0, x, R0, oz); d.oPI = LP(1, x, R0, oz);
-      d.oX = LP(2, x, R0, oz); d.oY = LP(3, x, R0, oz); d.oZ = LP(4, x, R0, oz);
-    }
+    d.PRn = LC(0, xp, R0, oz); d.PIn = LC(1, xp, R0, oz);
+    d.TXn = LC(2, xp, R0, oz); d.TYn = LC(3, xp, R0, oz); d.TZn = LC(4, xp, R0, oz);
+    d.oPR = LP(0, x, R0, oz); d.oPI = LP(1, x, R0, oz);
+    d.oX = LP(2, x, R0, oz); d.oY = LP(3, x, R0, oz); d.oZ = LP(4, x, R0, oz);
     d.PRyp = LC(0, x, RP, pz); d.PIyp = LC(1, x, RP, pz);
     d.PRym = LC(0, x, RM, mz); d.PIym = LC(1, x, RM, mz);
     d.TXyp = LC(2, x, RP, pz); d.TZyp = LC(4, x, RP, pz);
@@ -580,6 +589,8 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
   const int mine = FLAT ? y - y0 : 0;   /* the edge of this lane, where it is one */
   const int je = FLAT ? lane % ne : 0, jx = FLAT ? lane / ne : lane;
   uint32_t em = R0, emP = RP, ec = R0;  /* the sites z - 1 in rows y, y + 1, and z, of edge je */
+  uint32_t emM = RM;                    /* PF: z + 64 in row y - 1; em is z + 64 in lanes 4-7 */
+  __shared__ R znbr[PF ? 4 : 1][8];     /* PF: phi at z - 1 and z + 64, theta_x, theta_y, theta_y(y - 1) at z + 64 */
   if constexpr (FLAT) {
     const int ey = y0 + je, ez = je ? 0 : (int)(p0 - (uint32_t)y0 * NZ);
     const int ezm = ez == 0 ? NZ - 1 : ez - 1, eyp = ey == NY - 1 ? 0 : ey + 1;
@@ -591,9 +602,14 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
     em += ezm * E;
     emP += ezm * E;
     ec += z0 * E;
+    if constexpr (PF) {
+      const uint32_t ezp = z0 + 64 == (uint32_t)NZ ? 0 : z0 + 64;
+      emM += ezp * E;
+      if (lane >= 4) em = R0 + ezp * E;
+    }
   }
   auto edge_block = [&](int xb, int xe) {
-    const int xj = min(xb + jx, xe - 1);
+    const int xj = min(xb + (PF ? jx & 3 : jx), xe - 1);
     const int xjp = xj == NX - 1 ? 0 : xj + 1;
     R TZe, TXe, TYe, TZxe, TZye, TX0, TY0;
     if constexpr (BIG) {
@@ -615,40 +631,54 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
     e.qxz = TrigR<R>::sn(TXe + TZxe - TX0 - TZe);   /* a_xz at (xj, y, z - 1) */
     e.qyz = TrigR<R>::sn(TYe + TZye - TY0 - TZe);   /* a_yz there */
     e.tz = TZe;
+    R PRe = 0, PIe = 0, TYme = 0;
+    if constexpr (PF) {
+      const uint32_t pj = (uint32_t)xj * PLB;
+      PRe = bld<R>(c[0], pj + em, 0); PIe = bld<R>(c[1], pj + em, 0); TYme = bld<R>(c[3], pj + emM, 0);
+    }
     __syncthreads();   /* the previous block's values have been read */
     if (jx < xe - xb) zedge[FLAT ? lane : jx] = e;
+    if constexpr (PF) {
+      if (lane < 8) {
+        R *nb = znbr[lane & 3];
+        const int side = lane >= 4 ? 2 : 0;
+        nb[side] = PRe;
+        nb[side + 1] = PIe;
+        if (side) { nb[4] = TXe; nb[5] = TYe; nb[6] = TYme; }
+      }
+    }
     __syncthreads();
   };
 
-  __shared__ double pf[PF ? 2 : 1][5][128];
-  /* per lane: the byte distance of its field of each pair from the pair's
-   * lower plane (lanes 32-63 take the second field).  Within a level phi_r
-   * lies below phi_i and theta_x below theta_y (the [comp][level] plane
-   * order; the launcher checks it), so those pairs use the resources of
-   * phi_r and theta_x directly -- resources chosen at run time are held in
-   * scalar registers of their own, which the loop then spills */
+  /* pf[k]: a pair of 64-site rows, lanes 0-31 loading the first and lanes
+   * 32-63 the second, whose byte distance from the first is in the lane's
+   * offset.  Fields lie at equal distances ([comp][level] plane order, which
+   * the launcher checks). */
+  enum Pair { fO01, fO23, fO4, fYP01, fYM01, fY2, fY4, fN01, fN23, fN34, kPairs };
+  __shared__ double pf[PF ? kPairs : 1][128];
   const bool hi = lane >= 32;
-  const uint32_t lz = p0 * 8u + 16u * (uint32_t)(lane & 31);
-  auto pdelta = [&](const void *F, const void *G) -> uint32_t {
-    const char *pF = (const char *)F, *pG = (const char *)G;
-    return pF < pG ? (hi ? (uint32_t)(pG - pF) : 0u) : (hi ? 0u : (uint32_t)(pF - pG));
+  const uint32_t vz = (p0 - (uint32_t)y0 * NZ) * 8u + 16u * (uint32_t)(lane & 31);
+  const uint32_t cs = (uint32_t)((const char *)L.cur[1] - (const char *)L.cur[0]);   /* from a field to the next */
+  const uint32_t vF = vz + (hi ? cs : 0), vY = vz + (hi ? RM : RP), vT = vz + (hi ? cs + R0 : RM);
+  /* plane x's previous level and y-neighbour rows, plane x+1's own row and its theta_y one row back */
+  auto prefetch = [&](int x) {
+    const uint32_t so_ = (uint32_t)x * PLB, sn_ = (x == NX - 1 ? 0u : (uint32_t)(x + 1)) * PLB;
+    row_pair<kStream>(o[0], pf[fO01], vF, so_ + R0);
+    row_pair<kStream>(o[2], pf[fO23], vF, so_ + R0);
+    row_pair<kStream>(o[4], pf[fO4], vz, so_ + R0);
+    row_pair<0>(c[0], pf[fYP01], vF, so_ + RP);
+    row_pair<0>(c[0], pf[fYM01], vF, so_ + RM);
+    row_pair<0>(c[2], pf[fY2], vY, so_);
+    row_pair<0>(c[4], pf[fY4], vY, so_);
+    row_pair<0>(c[0], pf[fN01], vF, sn_ + R0);
+    row_pair<0>(c[2], pf[fN23], vF, sn_ + R0);
+    row_pair<0>(c[3], pf[fN34], vT, sn_);
   };
-  const bool lo4 = L.prv[4] < L.cur[4];
-  const uint32_t d0 = pdelta(L.prv[0], L.prv[1]) + lz, d1 = pdelta(L.prv[2], L.prv[3]) + lz;
-  const uint32_t d2 = pdelta(L.prv[4], L.cur[4]) + lz, d3 = pdelta(L.cur[0], L.cur[1]) + lz;
-  const uint32_t d4 = pdelta(L.cur[2], L.cur[3]) + lz;
-  /* plane x's previous level and plane x+1's current level into pf[buf] */
-  auto prefetch = [&](int x, int buf) {
-    const int xp = x == NX - 1 ? 0 : x + 1;
-    const uint32_t so_ = (uint32_t)x * PLB, sn_ = (uint32_t)xp * PLB;
-    const uint32_t s2 = hi ? sn_ : so_;   /* pair 2: plane x (previous level), x+1 (current) */
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(o[0], (lds_void *)&pf[buf][0][0], 16, d0 + so_, 0, 0, kStream);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(o[2], (lds_void *)&pf[buf][1][0], 16, d1 + so_, 0, 0, kStream);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(lo4 ? o[4] : c[4], (lds_void *)&pf[buf][2][0], 16, d2 + s2, 0, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(c[0], (lds_void *)&pf[buf][3][0], 16, d3 + sn_, 0, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(c[2], (lds_void *)&pf[buf][4][0], 16, d4 + sn_, 0, 0, 0);
-  };
-  if constexpr (PF) prefetch(x0, x0 & 1);
+  R TYm = 0;   /* theta_y(s-y): the last plane's theta_y(s+x-y) */
+  if constexpr (PF) {
+    TYm = LC(3, x0, RM, mz);
+    prefetch(x0);
+  }
   double rho_sum = 0, g_sum = 0;   /* MODE 2 */
   int bad = 0;
   /* DEFER (FP64): plane x's five stores are issued at the top
@@ -657,7 +687,7 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
    * behind the prefetch, and the wait for the prefetched values (which the
    * compiler makes a full drain) also waits for them.  It also shortens the
    * live ranges the compiler keeps across the loop: every FP64 variant fits
-   * 161 VGPRs with the prefetch, 64-bit plane addressing 170 -> 160, so all
+   * 163 VGPRs with the prefetch, 64-bit plane addressing 170 -> 160, so all
    * keep 3 waves per SIMD.  FP32 is slower with it (+0.5 %). */
   constexpr bool DEFER = sizeof(R) == 8;
   SiteOut<R> pend{};
@@ -677,24 +707,32 @@ __device__ __forceinline__ void ah_march(const MarchConsts<R> &k, const Levels<R
     next = i + 1 == EB ? 0 : i + 1;
     PlaneOps<R> D;
     if constexpr (PF) {
-      const int buf = x & 1;
-      D.oPR = pf[buf][0][lane]; D.oPI = pf[buf][0][64 + lane];
-      D.oX = pf[buf][1][lane]; D.oY = pf[buf][1][64 + lane];
-      D.oZ = pf[buf][2][lane]; D.TZn = pf[buf][2][64 + lane];
-      D.PRn = pf[buf][3][lane]; D.PIn = pf[buf][3][64 + lane];
-      D.TXn = pf[buf][4][lane]; D.TYn = pf[buf][4][64 + lane];
+      D.oPR = pf[fO01][lane]; D.oPI = pf[fO01][64 + lane];
+      D.oX = pf[fO23][lane]; D.oY = pf[fO23][64 + lane]; D.oZ = pf[fO4][lane];
+      D.PRyp = pf[fYP01][lane]; D.PIyp = pf[fYP01][64 + lane];
+      D.PRym = pf[fYM01][lane]; D.PIym = pf[fYM01][64 + lane];
+      D.TXyp = pf[fY2][lane]; D.TXym = pf[fY2][64 + lane];
+      D.TZyp = pf[fY4][lane]; D.TZym = pf[fY4][64 + lane];
+      D.PRn = pf[fN01][lane]; D.PIn = pf[fN01][64 + lane];
+      D.TXn = pf[fN23][lane]; D.TYn = pf[fN23][64 + lane];
+      D.TYxpym = pf[fN34][lane]; D.TZn = pf[fN34][64 + lane];
+      D.TYym = TYm; TYm = D.TYxpym;
+      const R *nb = znbr[i];
+      D.PRzm = lane_prev(PRc, nb[0]); D.PIzm = lane_prev(PIc, nb[1]);
+      D.PRzp = lane_next(PRc, nb[2]); D.PIzp = lane_next(PIc, nb[3]);
+      D.TXzp = lane_next(TXc, nb[4]); D.TYzp = lane_next(TYc, nb[5]);
+      D.TYymzp = lane_next(D.TYym, nb[6]);
+      /* every value is in its register before the next plane's may land */
+      asm volatile("" ::"v"(D.oPR), "v"(D.oPI), "v"(D.oX), "v"(D.oY), "v"(D.oZ), "v"(D.PRyp), "v"(D.PIyp), "v"(D.PRym),
+                   "v"(D.PIym), "v"(D.TXyp), "v"(D.TXym), "v"(D.TZyp), "v"(D.TZym), "v"(D.PRn), "v"(D.PIn), "v"(D.TXn),
+                   "v"(D.TYn), "v"(D.TYxpym), "v"(D.TZn)
+                   : "memory");
     }
     if constexpr (DEFER) {
       if (x > x0 && act) store_out(x - 1, pend);
     }
-    load_plane(x, D, PRc, PIc, TXc, TYc, TZc);
-    if constexpr (PF) {
-      /* issued after the plane's own loads (the waits for those then leave
-       * these in flight) and unconditionally (a branch around them makes
-       * every later wait a full drain): the last plane fetches itself again,
-       * into the buffer not being read */
-      prefetch(x + 1 < x1 ? x + 1 : x, (x + 1) & 1);
-    }
+    if constexpr (PF) prefetch(x + 1 < x1 ? x + 1 : x);
+    else load_plane(x, D, PRc, PIc, TXc, TYc, TZc);
     SiteOut<R> out;
     if constexpr (MODE == 0) {
       ah_site_update<R, POW2, RegOps<R>, false, FLAT>(k, plain, RegOps<R>{D, PRc, PIc, TXc, TYc, TZc}, m, ze, e0, out);

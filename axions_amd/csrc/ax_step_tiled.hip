@@ -141,10 +141,12 @@ int default_xseg(const ax_params &p) {
 /* The LDS prefetch of the FP64 march applies: whole 64-site chunks (across
  * rows it costs registers that spill: 200^3 251 us against 245 without),
  * three field planes within 32-bit offsets, and the [comp][level] plane order
- * its phi and theta_x/theta_y pairs rely on (AX_NO_PREFETCH turns it off). */
+ * its pairs of rows rely on (AX_NO_PREFETCH turns it off). */
 template <typename R>
 static bool prefetch_ok(const StepConsts &k, const Levels<R> &L) {
-  const bool order = L.cur[0] < L.cur[1] && L.cur[2] < L.cur[3] && L.prv[0] < L.prv[1] && L.prv[2] < L.prv[3];
+  const ptrdiff_t cs = L.cur[1] - L.cur[0];   /* [comp][level]: two planes */
+  const bool order = cs > 0 && L.cur[3] - L.cur[2] == cs && L.cur[4] - L.cur[3] == cs && L.prv[1] - L.prv[0] == cs &&
+                     L.prv[3] - L.prv[2] == cs;
   return k.nz % 64 == 0 && order &&
          (size_t)k.nx * k.ny * k.nz * sizeof(double) * 3 + ((size_t)1 << 20) < ((size_t)1 << 32) &&
          getenv("AX_NO_PREFETCH") == nullptr;
@@ -160,11 +162,9 @@ hipError_t launch_step_tiled_ah(const StepConsts &k, const Levels<R> &L, int xse
    * forces it on smaller lattices, for tests) */
   const bool big = (size_t)k.nx * k.ny * k.nz * sizeof(R) >= ((size_t)1 << 32) || getenv("AX_BIG_PLANES") != nullptr;
   dim3 grid(g.work), block(64);
-  /* FP64, whole chunks and three planes within 32-bit offsets: the
-   * previous level and the next plane are prefetched into LDS (ah_march; its
-   * phi and theta_x/theta_y pairs rely on the [comp][level] plane order).
-   * Every variant keeps 3 waves per SIMD with it, with the stores issued one
-   * plane late. */
+  /* FP64, whole chunks and three planes within 32-bit offsets: a plane's
+   * rows are prefetched into LDS (ah_march).  Every variant keeps 3 waves per
+   * SIMD with it, with the stores issued one plane late. */
   const bool pf = sizeof(R) == 8 && !big && prefetch_ok(k, L);
   /* rows of whole chunks, whose row offsets stay scalars, else chunks across
    * rows.  us per step with partial chunks at the row ends / across rows:
@@ -198,7 +198,7 @@ hipError_t launch_step_tiled_ah(const StepConsts &k, const Levels<R> &L, int xse
 /* The FP64 periodic Abelian-Higgs step with its current level's divergence
  * stored (MODE 1) or its current level's diagnostics taken (MODE 2), see
  * ah_march.  One partial-sum triple per work item (MODE 2).  PF: the LDS
- * prefetch of the plain step (MODE 1 keeps 3 waves per SIMD with it, 167
+ * prefetch of the plain step (MODE 1 keeps 3 waves per SIMD with it, 168
  * VGPRs; MODE 2 runs at 2 either way). */
 template <bool POW2, bool P2D, int MODE, bool PF, bool FLAT>
 __global__ void __launch_bounds__(64, MODE == 1 ? 3 : 2) ah_fused_kernel(MarchConsts<double> k, Levels<double> L, int nx, int ny, int nz,
