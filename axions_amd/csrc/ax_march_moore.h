@@ -91,6 +91,15 @@ __device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Level
                                             uint32_t p0, int x0, int x1, bool xfix = false, bool zfix = false,
                                             int *bad = nullptr) {
   typedef TrigR<R> T;
+  /* Chunks across rows in FP64 without the band check: the neighbours' phi is
+   * loaded ahead of the plaquette sines, whose branch keeps the compiler from
+   * moving loads over it.  us per step late / early: dx^2 no power of two,
+   * faces fixed 201x201x51 155.5 / 142.8, 250^3 1023 / 899, 100^3 73.7 / 68.2,
+   * 50^3 13.5 / 11.9; powers of two, periodic 250^3 952 / 817, 100^3 62.2 /
+   * 55.5.  The other kernels are slower with it: whole chunks 256^3 845 / 931
+   * and (powers of two) 767 / 834, with the band check 250^3 824 / 875, 256^3
+   * 847 / 900; FP32 is the same. */
+  constexpr bool EARLY = sizeof(R) == 8 && BUF && FLAT && !CHECK;
   const uint32_t NYNZ = (uint32_t)NY * (uint32_t)NZ;
   const LaneSite<FLAT> ls(NY, NZ, p0);
   const int y = ls.y, z = ls.z;
@@ -164,6 +173,16 @@ __device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Level
     const R TXzm = LC(4, x, R0, ozm), TYzm = LC(5, x, R0, ozm), TZzm = LC(6, x, R0, ozm);
     const R TZxpzm = LC(6, xp, R0, ozm), TZypzm = LC(6, x, RP, pzm);
 
+    R Pyp[4], Pym[4], Pzp[4], Pzm[4];
+    auto phi_rows = [&](int f) {
+      for (int c = 2 * f; c < 2 * f + 2; ++c) {
+        Pyp[c] = LC(c, x, RP, pz); Pym[c] = LC(c, x, RM, mz);
+        Pzp[c] = LC(c, x, R0, ozp); Pzm[c] = LC(c, x, R0, ozm);
+      }
+    };
+    if (EARLY)
+      for (int f = 0; f < 2; ++f) phi_rows(f);
+
     /* plaquette sines (mooreEvol.cpp:310-333 operand order) */
     const R a_xy = X + Nx[5] - TXyp - Y;
     const R a_xz = X + Nx[6] - TXzp - Z;
@@ -211,10 +230,9 @@ __device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Level
       T::sc(q[f] * TZzm, &szm, &czm);
       const R ar = C[cr], ai = C[ci];
       const R rxp = Nx[cr], ixp = Nx[ci];
-      const R ryp = LC(cr, x, RP, pz), iyp = LC(ci, x, RP, pz);
-      const R rym = LC(cr, x, RM, mz), iym = LC(ci, x, RM, mz);
-      const R rzp = LC(cr, x, R0, ozp), izp = LC(ci, x, R0, ozp);
-      const R rzm = LC(cr, x, R0, ozm), izm = LC(ci, x, R0, ozm);
+      if (!EARLY) phi_rows(f);
+      const R ryp = Pyp[cr], iyp = Pyp[ci], rym = Pym[cr], iym = Pym[ci];
+      const R rzp = Pzp[cr], izp = Pzp[ci], rzm = Pzm[cr], izm = Pzm[ci];
       {
         R lxx = dvx(cx * rxp + sx * ixp - 2 * ar + cxm[f] * Pm[cr] - sxm[f] * Pm[ci]);
         R lyy = dvy(cy * ryp + sy * iyp - 2 * ar + cym * rym - sym_ * iym);
