@@ -117,6 +117,7 @@ struct ax_lattice {
   float *phase = nullptr;   /* FP32 edge values [3][V] of the marching diagnostics (ax_wind.h) */
   int *bcount = nullptr;
   long long *boff = nullptr;
+  uint64_t *bmask = nullptr;   /* face masks, where there is memory for them */
   long long *ctotal = nullptr;
   double *cxyz = nullptr;
   size_t cxyz_cap = 0;
@@ -275,6 +276,7 @@ void ax_destroy(ax_lattice *L) {
   if (L->phase) (void)hipFree(L->phase);
   if (L->bcount) (void)hipFree(L->bcount);
   if (L->boff) (void)hipFree(L->boff);
+  if (L->bmask) (void)hipFree(L->bmask);
   if (L->ctotal) (void)hipFree(L->ctotal);
   if (L->cxyz) (void)hipFree(L->cxyz);
   if (L->stream) (void)hipStreamDestroy(L->stream);
@@ -858,6 +860,10 @@ int ax_crossings(ax_lattice *L, double *xyz, size_t cap, size_t *count) {
       (void)hipGetLastError();   /* clear the sticky error of the failed call */
       return fail(AX_ENOMEM, "crossing scratch");
     }
+    if (hipMalloc((void **)&L->bmask, cross_mask_bytes(L->V)) != hipSuccess) {
+      (void)hipGetLastError();
+      L->bmask = nullptr;
+    }
   }
   if (cap > L->cxyz_cap) {
     if (L->cxyz) (void)hipFree(L->cxyz);
@@ -877,11 +883,13 @@ int ax_crossings(ax_lattice *L, double *xyz, size_t cap, size_t *count) {
   if (L->esize == 8) {
     const double *b = (const double *)L->state;
     e = launch_crossings<double>(p.nx, p.ny, p.nz, p.dx, p.dy, p.dz, b + (size_t)tN * L->pitch, b + (size_t)(2 + tN) * L->pitch,
-                                 ex, ez, L->bcount, L->boff, L->ctotal, L->cxyz, (long long)cap, L->stream, cap > 0);
+                                 ex, ez, L->bcount, L->boff, L->ctotal, L->cxyz, (long long)cap, L->bmask, L->stream,
+                                 cap > 0);
   } else {
     const float *b = (const float *)L->state;
     e = launch_crossings<float>(p.nx, p.ny, p.nz, p.dx, p.dy, p.dz, b + (size_t)tN * L->pitch, b + (size_t)(2 + tN) * L->pitch,
-                                ex, ez, L->bcount, L->boff, L->ctotal, L->cxyz, (long long)cap, L->stream, cap > 0);
+                                ex, ez, L->bcount, L->boff, L->ctotal, L->cxyz, (long long)cap, L->bmask, L->stream,
+                                 cap > 0);
   }
   if (e != hipSuccess) return hip_fail(e, "crossing launch");
   long long tot = 0;

@@ -290,7 +290,9 @@ __global__ void __launch_bounds__(256) winding_kernel(int nx, int ny, int nz, co
  * LDS as one contiguous run.  Two launches (counts, then points at their
  * offsets) with a scan in between.  512^3 FP64, 1.2 points a site: counts
  * 2.67 -> 1.56 ms, scan 0.92 -> 0.15, points 6.96 -> 2.94 (3.9 GB written);
- * FP32 2.63 -> 1.45, 0.92 -> 0.15, 6.29 -> 2.72.  Bound by instructions. */
+ * FP32 2.63 -> 1.45, 0.92 -> 0.15, 6.29 -> 2.72; with the faces handed on as
+ * masks the whole call 4.65 -> 3.88, FP32 4.15 -> 3.27 (301^3 FP64 0.98 ->
+ * 0.81, 101^3 78 -> 69 us).  Bound by instructions. */
 
 struct CrossGeom {
   int nx, ny, nz, ex, ez, x0, y0, z0;
@@ -408,11 +410,15 @@ __device__ __forceinline__ int face_roots(const double v00[2], const double v10[
   return n;
 }
 
-/* WRITE: the points of each group from its offset on; else its count. */
-template <typename T, bool WRITE>
+/* WRITE: the points of each group from its offset on; else its count.
+ * masks: three words per 64 sites, the lanes whose xy, xz, yz face is not
+ * known to hold no point.  The count pass stores them and the point pass
+ * (MASKED) takes its faces from them instead of reading and classifying
+ * every face again; without the memory for them it classifies. */
+template <typename T, bool WRITE, bool MASKED>
 __global__ void __launch_bounds__(64) cross_kernel(CrossGeom g, const T *__restrict__ fr, const T *__restrict__ fi,
                                                    int *__restrict__ count, const long long *__restrict__ offset,
-                                                   double *__restrict__ xyz, long long cap) {
+                                                   double *__restrict__ xyz, long long cap, uint64_t *masks) {
   /* consecutive groups on one XCD, so that rows y + 1 are read from its L2 */
   const uint32_t grp = (blockIdx.x & 7) * g.per + (blockIdx.x >> 3);
   if (grp >= g.groups) return;
@@ -473,31 +479,40 @@ __global__ void __launch_bounds__(64) cross_kernel(CrossGeom g, const T *__restr
 
   for (uint32_t c = 0; c < g.sites; c += 64) {
     if (base + c >= g.V) break;
-    const uint32_t s = min(base + c + lane, g.V - 1);
-    const uint32_t r = quotient(s, g.by_nz), i = quotient(r, g.by_ny);
-    const int k = (int)(s - r * nz), j = (int)(r - i * ny);
-    /* only the sites the bulk update covers (evolution.cpp:731-743) */
-    const bool bulk = base + c + lane < g.V &&
-                      !((g.ex && ((int)i == 0 || (int)i == nx - 1 || j == 0 || j == ny - 1)) ||
-                        (g.ez && (k == 0 || k == nz - 1)));
-    const int ip = wrapp((int)i, nx), jp = wrapp(j, ny), kp = wrapp(k, nz);
-    const uint32_t at7[7] = {s, id(ip, j, k), id((int)i, jp, k), id((int)i, j, kp), id(ip, jp, k), id(ip, j, kp),
-                             id((int)i, jp, kp)};
-    float re[7], im[7];
-#pragma unroll
-    for (int q = 0; q < 7; ++q) re[q] = (float)fr[at7[q]];
-#pragma unroll
-    for (int q = 0; q < 7; ++q) im[q] = (float)fi[at7[q]];
     uint64_t mask[3];   /* lanes whose xy, xz, yz face goes to the queue */
+    if constexpr (MASKED && WRITE) {
 #pragma unroll
-    for (int f = 0; f < 3; ++f) {
-      const int a = f == 2 ? 2 : 1, b = f == 0 ? 2 : 3, ab = 4 + f;
-      int n = 0;
-      const bool open = bulk && !one_sign(re[0], re[a], re[b], re[ab], g.k);
-      if (__builtin_amdgcn_ballot_w64(open) && open)
-        n = face_class(re[0], re[a], re[b], re[ab], im[0], im[a], im[b], im[ab], g.k);
-      if (!WRITE) own += n == 3 ? 0 : n;
-      mask[f] = __builtin_amdgcn_ballot_w64(WRITE ? n != 0 : n == 3);
+      for (int f = 0; f < 3; ++f) mask[f] = masks[3 * (size_t)((base + c) >> 6) + f];
+    } else {
+      const uint32_t s = min(base + c + lane, g.V - 1);
+      const uint32_t r = quotient(s, g.by_nz), i = quotient(r, g.by_ny);
+      const int k = (int)(s - r * nz), j = (int)(r - i * ny);
+      /* only the sites the bulk update covers (evolution.cpp:731-743) */
+      const bool bulk = base + c + lane < g.V &&
+                        !((g.ex && ((int)i == 0 || (int)i == nx - 1 || j == 0 || j == ny - 1)) ||
+                          (g.ez && (k == 0 || k == nz - 1)));
+      const int ip = wrapp((int)i, nx), jp = wrapp(j, ny), kp = wrapp(k, nz);
+      const uint32_t at7[7] = {s, id(ip, j, k), id((int)i, jp, k), id((int)i, j, kp), id(ip, jp, k), id(ip, j, kp),
+                               id((int)i, jp, kp)};
+      float re[7], im[7];
+#pragma unroll
+      for (int q = 0; q < 7; ++q) re[q] = (float)fr[at7[q]];
+#pragma unroll
+      for (int q = 0; q < 7; ++q) im[q] = (float)fi[at7[q]];
+      uint64_t some[3];
+#pragma unroll
+      for (int f = 0; f < 3; ++f) {
+        const int a = f == 2 ? 2 : 1, b = f == 0 ? 2 : 3, ab = 4 + f;
+        int n = 0;
+        const bool open = bulk && !one_sign(re[0], re[a], re[b], re[ab], g.k);
+        if (__builtin_amdgcn_ballot_w64(open) && open)
+          n = face_class(re[0], re[a], re[b], re[ab], im[0], im[a], im[b], im[ab], g.k);
+        if (!WRITE) own += n == 3 ? 0 : n;
+        some[f] = __builtin_amdgcn_ballot_w64(n != 0);
+        mask[f] = WRITE ? some[f] : __builtin_amdgcn_ballot_w64(n == 3);
+      }
+      if (MASKED && lane < 3)
+        masks[3 * (size_t)((base + c) >> 6) + lane] = lane == 0 ? some[0] : lane == 1 ? some[1] : some[2];
     }
     uint32_t at = tail;
 #pragma unroll
@@ -969,7 +984,7 @@ hipError_t launch_winding(int nx, int ny, int nz, const T *fr, const T *fi, cons
 template <typename T>
 hipError_t launch_crossings(int nx, int ny, int nz, double dx, double dy, double dz, const T *fr, const T *fi,
                             int ex, int ez, int *bcount, long long *boff, long long *total, double *xyz,
-                            long long cap, hipStream_t st, bool write) {
+                            long long cap, uint64_t *masks, hipStream_t st, bool write) {
   CrossGeom g;
   g.nx = nx; g.ny = ny; g.nz = nz; g.ex = ex; g.ez = ez;
   g.x0 = int(0.5 * (nx - 1)); g.y0 = int(0.5 * (ny - 1)); g.z0 = int(0.5 * (nz - 1));
@@ -986,9 +1001,14 @@ hipError_t launch_crossings(int nx, int ny, int nz, double dx, double dy, double
   const double k = std::max(0x1p-16, 0x1p-43 * h * h * h);
   g.k = k < 0x1p-8 ? (float)k : 2.0f;
   const dim3 grid(8 * g.per), block(64);
-  hipLaunchKernelGGL((cross_kernel<T, false>), grid, block, 0, st, g, fr, fi, bcount, boff, xyz, cap);
+#define AX_CROSS(W, M) \
+  hipLaunchKernelGGL((cross_kernel<T, W, M>), grid, block, 0, st, g, fr, fi, bcount, boff, xyz, cap, masks)
+  if (write && masks) AX_CROSS(false, true);
+  else AX_CROSS(false, false);
   hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, st, bcount, boff, (int)g.groups, total);
-  if (write) hipLaunchKernelGGL((cross_kernel<T, true>), grid, block, 0, st, g, fr, fi, bcount, boff, xyz, cap);
+  if (write && masks) AX_CROSS(true, true);
+  else if (write) AX_CROSS(true, false);
+#undef AX_CROSS
   return hipGetLastError();
 }
 
@@ -1085,7 +1105,7 @@ hipError_t launch_wind_phase(int nx, int ny, int nz, int ex, int ez, const float
                                         double, int, int, int8_t *, Partials &, hipStream_t);                   \
   template hipError_t launch_crossings<T>(int, int, int, double, double, double, const T *, const T *, int,     \
                                           int, int *, long long *, long long *, double *, long long,            \
-                                          hipStream_t, bool);                                                   \
+                                          uint64_t *, hipStream_t, bool);                                       \
   template hipError_t launch_diag_march<T>(const DiagConsts &, const Levels<T> &, float *, Partials &,          \
                                            hipStream_t);                                                        \
   template hipError_t launch_edge_winding<T>(int, int, int, int, int, const T *, const T *, const T *,          \

@@ -221,7 +221,9 @@ inline size_t cross_groups(size_t V) { return (V + cross_sites(V) - 1) / cross_s
 template <typename T>
 hipError_t launch_crossings(int nx, int ny, int nz, double dx, double dy, double dz, const T *fr, const T *fi,
                             int ex, int ez, int *bcount, long long *boff, long long *total, double *xyz,
-                            long long cap, hipStream_t st, bool write);
+                            long long cap, uint64_t *masks, hipStream_t st, bool write);
+/* the face masks (masks, may be null) of a lattice of V sites */
+inline size_t cross_mask_bytes(size_t V) { return (V + 63) / 64 * 3 * sizeof(uint64_t); }
 
 /* Fused diagnostics (ax_march.h MODE 1/2, FP64 periodic Abelian-Higgs) */
 struct FusedDiag;

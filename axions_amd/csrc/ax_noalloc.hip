@@ -6,7 +6,7 @@
  * ax_crossings allocates its per-group counts and offsets and its point
  * buffer on first use (and the point buffer again whenever the capacity
  * grows).  Here the points go straight into a device buffer the caller owns,
- * and the counts and offsets live in `scratch`, a fixed array in the
+ * and the counts, offsets and masks live in `scratch`, a fixed array in the
  * library's device code: no hipMalloc, hipFree or other allocating call is
  * made.  Every GPU the library runs on holds its own copy of the array
  * until the process ends; its device address is looked up once per device
@@ -15,8 +15,8 @@
  *
  * The array is shared by every call on a GPU: calls that overlap on one GPU
  * (different streams or host threads) race on it.  Nothing in it needs
- * clearing: each call's count pass writes every group count it later reads,
- * and the scan writes every offset.
+ * clearing: each call's count pass writes every group count and mask it later
+ * reads, and the scan writes every offset.
  */
 #include <climits>
 #include <mutex>
@@ -27,10 +27,12 @@ namespace ax {
 
 /* group counts (int) + group offsets (long long) of up to kNoallocBlocks
  * groups, 6 MiB; the lattices accepted, up to kNoallocBlocks * 256 = 2^27
- * sites (512^3), have at most 2^18 groups (cross_groups) */
+ * sites (512^3), have at most 2^18 groups (cross_groups); and their face
+ * masks, 48 MiB */
 constexpr size_t kNoallocBlocks = (size_t)1 << 19;
 constexpr size_t kNoallocCountBytes = kNoallocBlocks * sizeof(int);
-constexpr size_t kNoallocBytes = kNoallocCountBytes + kNoallocBlocks * sizeof(long long);
+constexpr size_t kNoallocMaskAt = kNoallocCountBytes + kNoallocBlocks * sizeof(long long);
+constexpr size_t kNoallocBytes = kNoallocMaskAt + kNoallocBlocks * 256 / 64 * 3 * sizeof(uint64_t);
 
 static __device__ __align__(256) unsigned char scratch[kNoallocBytes];
 
@@ -75,6 +77,7 @@ extern "C" int ax_crossings_noalloc(ax_lattice *L, double *xyz, size_t cap, int6
   if (rc) return rc;
   int *bcount = (int *)base;
   long long *boff = (long long *)(base + kNoallocCountBytes);
+  uint64_t *masks = (uint64_t *)(base + kNoallocMaskAt);
   rc = prepare_faces(L);
   if (rc) return rc;
   const bool glob = p.model == AX_MODEL_GLOBAL;
@@ -86,13 +89,13 @@ extern "C" int ax_crossings_noalloc(ax_lattice *L, double *xyz, size_t cap, int6
   if (p.precision == 64) {
     const double *b = (const double *)lattice_state(L);
     e = launch_crossings<double>(p.nx, p.ny, p.nz, p.dx, p.dy, p.dz, b + (size_t)tN * pitch, b + (size_t)(2 + tN) * pitch,
-                                 ex, ez, bcount, boff, (long long *)count, xyz, (long long)cap, lattice_stream(L),
-                                 cap > 0);
+                                 ex, ez, bcount, boff, (long long *)count, xyz, (long long)cap, masks,
+                                 lattice_stream(L), cap > 0);
   } else {
     const float *b = (const float *)lattice_state(L);
     e = launch_crossings<float>(p.nx, p.ny, p.nz, p.dx, p.dy, p.dz, b + (size_t)tN * pitch, b + (size_t)(2 + tN) * pitch,
-                                ex, ez, bcount, boff, (long long *)count, xyz, (long long)cap, lattice_stream(L),
-                                cap > 0);
+                                ex, ez, bcount, boff, (long long *)count, xyz, (long long)cap, masks,
+                                lattice_stream(L), cap > 0);
   }
   return e == hipSuccess ? AX_OK : hip_fail(e, "crossing launch");
 }

@@ -220,7 +220,7 @@ int ax_crossings(ax_lattice *lat, double *xyz, size_t cap, size_t *count);
  * doubles) owned by the caller; the total count goes to *count, a DEVICE
  * int64.  Enqueued on the handle's stream only (ax_sync before reading).
  * The lattice's device must be current.  Its per-group scratch is one fixed
- * array per GPU inside the library (6 MiB, held until the process ends), so
+ * array per GPU inside the library (54 MiB, held until the process ends), so
  * lattices above 2^27 sites (512^3) are refused (AX_EINVAL), and calls that
  * overlap on one GPU race on that array. */
 int ax_crossings_noalloc(ax_lattice *lat, double *xyz, size_t cap, int64_t *count);
