@@ -4,9 +4,10 @@
  * as a 64-lane wave marching along x over a 64-site chunk of the (y, z)
  * plane, like ah_march.  Same arithmetic and operand order as moore_update in
  * ax_step.hip; the cos/sin of q_f theta_x(s-x) and the plaquette sines at
- * s-x come from the previous plane of the march, y/z-backward values are
- * recomputed, the six plaquette sines at s are computed once and take the
- * short k = 0 form when the whole wave qualifies.
+ * s-x come from the previous plane of the march, y-backward values are
+ * recomputed, and so are z-backward ones where ZB below does not shift them
+ * over from lane - 1; the six plaquette sines at s are computed once and take
+ * the short k = 0 form when the whole wave qualifies.
  */
 #ifndef AXIONS_AX_MARCH_MOORE_H
 #define AXIONS_AX_MARCH_MOORE_H
@@ -77,6 +78,14 @@ inline void moore_consts_from(const StepConsts &k, MooreConsts<R> &m) {
   m.inv_dx2 = (R)1 / m.dx2; m.inv_dy2 = (R)1 / m.dy2; m.inv_dz2 = (R)1 / m.dz2;
 }
 
+/* What the site (y, z - 1) contributes to a chunk's first lane (ZEdge in
+ * ax_march.h): sin/cos of q_f theta_z there and its F_xz, F_yz plaquette
+ * sines. */
+template <typename R>
+struct MooreEdge {
+  R s[2], c[2], qxz, qyz;
+};
+
 /* BUF: the loop's loads and stores are raw buffer accesses, one resource per
  * field spanning both of its levels (planes 2c, 2c+1; the caller checks that
  * two planes fit 32-bit offsets), with the streaming hint on the previous
@@ -99,6 +108,14 @@ __device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Level
    * 55.5.  The other kernels are slower with it: whole chunks 256^3 845 / 931
    * and (powers of two) 767 / 834, with the band check 250^3 824 / 875, 256^3
    * 847 / 900; FP32 is the same. */
+  /* ZB: whole chunks with the band check take the z-backward cos/sin and
+   * sines from lane - 1, the chunk edge's from a pass over four planes
+   * (zedge), as ah_march, instead of evaluating them again: two of ten
+   * sincos and two of ten sines fewer; and the first charge's phi rows are
+   * loaded ahead of the plaquette sines.  us per step 256^3 854 -> 819 ->
+   * 813.5, 128^3 114 -> 111.  The other kernels lose: powers of two 256^3 766
+   * -> 800, chunks across rows with the check 150^3 181 -> 184 (registers). */
+  constexpr bool ZB = sizeof(R) == 8 && BUF && !FLAT && CHECK;
   constexpr bool EARLY = sizeof(R) == 8 && BUF && FLAT && !CHECK;
   const uint32_t NYNZ = (uint32_t)NY * (uint32_t)NZ;
   const LaneSite<FLAT> ls(NY, NZ, p0);
@@ -160,7 +177,31 @@ __device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Level
   R C[7];
   for (int c = 0; c < 7; ++c) C[c] = LG(F[c], x0, R0, oz);
 
+  /* ZB: lane j < 4 evaluates the edge of plane xb + j */
+  const bool e0 = (threadIdx.x & 63) == 0;
+  __shared__ MooreEdge<R> zedge[4];
+  auto edge_block = [&](int xb, int xe) {
+    const int j = (int)(threadIdx.x & 63), xj = min(xb + j, xe - 1);
+    const uint32_t z0 = p0 % (uint32_t)NZ, zm = (z0 == 0 ? (uint32_t)NZ : z0) - 1;
+    const uint32_t em = R0 + zm * E, emP = RP + zm * E, ec = R0 + z0 * E;   /* (y, z0 - 1), (y + 1, z0 - 1), (y, z0) */
+    const int xjp = xj == NX - 1 ? 0 : xj + 1;
+    auto at = [&](int c, int xx, uint32_t off) -> R { return bld<R>(FR[c], offC + (uint32_t)xx * PLB + off, 0); };
+    const R TZe = at(6, xj, em), TXe = at(4, xj, em), TYe = at(5, xj, em);
+    const R TZxe = at(6, xjp, em), TZye = at(6, xj, emP), TX0 = at(4, xj, ec), TY0 = at(5, xj, ec);
+    MooreEdge<R> e;
+    for (int f = 0; f < 2; ++f) T::sc(q[f] * TZe, &e.s[f], &e.c[f]);
+    e.qxz = T::sn(TXe + TZxe - TX0 - TZe);   /* a_xz at (xj, y, z - 1) */
+    e.qyz = T::sn(TYe + TZye - TY0 - TZe);   /* a_yz there */
+    __syncthreads();   /* the previous block's values have been read */
+    if (j < xe - xb) zedge[j] = e;
+    __syncthreads();
+  };
+
   for (int x = x0; x < x1; ++x) {
+    if constexpr (ZB) {
+      if (((x - x0) & 3) == 0) edge_block(x, min(x1, x + 4));
+    }
+    const MooreEdge<R> &ze = zedge[(x - x0) & 3];
     const int xp = x == NX - 1 ? 0 : x + 1;
     const uint32_t so = (uint32_t)x * PLB + R0;   /* BUF only */
     R Nx[7];
@@ -170,8 +211,14 @@ __device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Level
     const R TXzp = LC(4, x, R0, ozp), TYzp = LC(5, x, R0, ozp);
     const R TXym = LC(4, x, RM, mz), TYym = LC(5, x, RM, mz), TZym = LC(6, x, RM, mz);
     const R TYxpym = LC(5, xp, RM, mz), TYymzp = LC(5, x, RM, mzp);
-    const R TXzm = LC(4, x, R0, ozm), TYzm = LC(5, x, R0, ozm), TZzm = LC(6, x, R0, ozm);
-    const R TZxpzm = LC(6, xp, R0, ozm), TZypzm = LC(6, x, RP, pzm);
+    R TZzm = 0, b_xz = 0, b_yz = 0;
+    if constexpr (!ZB) {
+      const R TXzm = LC(4, x, R0, ozm), TYzm = LC(5, x, R0, ozm);
+      TZzm = LC(6, x, R0, ozm);
+      const R TZxpzm = LC(6, xp, R0, ozm), TZypzm = LC(6, x, RP, pzm);
+      b_xz = TXzm + TZxpzm - X - TZzm;
+      b_yz = TYzm + TZypzm - Y - TZzm;
+    }
 
     R Pyp[4], Pym[4], Pzp[4], Pzm[4];
     auto phi_rows = [&](int f) {
@@ -180,8 +227,8 @@ __device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Level
         Pzp[c] = LC(c, x, R0, ozp); Pzm[c] = LC(c, x, R0, ozm);
       }
     };
-    if (EARLY)
-      for (int f = 0; f < 2; ++f) phi_rows(f);
+    if (EARLY || ZB)
+      for (int f = 0; f < (EARLY ? 2 : 1); ++f) phi_rows(f);
 
     /* plaquette sines (mooreEvol.cpp:310-333 operand order) */
     const R a_xy = X + Nx[5] - TXyp - Y;
@@ -192,20 +239,24 @@ __device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Level
     const R a_zy = Z + TYzp - TZyp - Y;
     const R b_xy = TXym + TYxpym - X - TYym;
     const R b_zy = TZym + TYymzp - Z - TYym;
-    const R b_xz = TXzm + TZxpzm - X - TZzm;
-    const R b_yz = TYzm + TZypzm - Y - TZzm;
     R Qxy, Qxz, Qyx, Qyz, Qzx, Qzy, Qxy_m, Qzy_m, Qxz_m, Qyz_m;
     const uint64_t small = small_lanes(a_xy) & small_lanes(a_xz) & small_lanes(a_yx) & small_lanes(a_yz) &
                            small_lanes(a_zx) & small_lanes(a_zy) & small_lanes(b_xy) & small_lanes(b_zy) &
-                           small_lanes(b_xz) & small_lanes(b_yz);
+                           (ZB ? ~0ull : small_lanes(b_xz) & small_lanes(b_yz));
     if (small == __builtin_amdgcn_read_exec()) {
       Qxy = T::sn_small(a_xy); Qxz = T::sn_small(a_xz); Qyx = T::sn_small(a_yx);
       Qyz = T::sn_small(a_yz); Qzx = T::sn_small(a_zx); Qzy = T::sn_small(a_zy);
-      Qxy_m = T::sn_small(b_xy); Qzy_m = T::sn_small(b_zy); Qxz_m = T::sn_small(b_xz); Qyz_m = T::sn_small(b_yz);
+      Qxy_m = T::sn_small(b_xy); Qzy_m = T::sn_small(b_zy);
+      if constexpr (!ZB) { Qxz_m = T::sn_small(b_xz); Qyz_m = T::sn_small(b_yz); }
     } else {
       Qxy = T::sn(a_xy); Qxz = T::sn(a_xz); Qyx = T::sn(a_yx);
       Qyz = T::sn(a_yz); Qzx = T::sn(a_zx); Qzy = T::sn(a_zy);
-      Qxy_m = T::sn(b_xy); Qzy_m = T::sn(b_zy); Qxz_m = T::sn(b_xz); Qyz_m = T::sn(b_yz);
+      Qxy_m = T::sn(b_xy); Qzy_m = T::sn(b_zy);
+      if constexpr (!ZB) { Qxz_m = T::sn(b_xz); Qyz_m = T::sn(b_yz); }
+    }
+    if constexpr (ZB) {   /* the second sines of F_xz, F_yz are lane - 1's first ones */
+      Qxz_m = z_back<false, R>(Qxz, ze.qxz, e0);
+      Qyz_m = z_back<false, R>(Qyz, ze.qyz, e0);
     }
     const R fxy = dvy(Qxy - Qxy_m);
     const R fxz = dvz(Qxz - Qxz_m);
@@ -227,10 +278,15 @@ __device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Level
       T::sc(q[f] * Y, &sy, &cy);
       T::sc(q[f] * Z, &sz, &cz);
       T::sc(q[f] * TYym, &sym_, &cym);
-      T::sc(q[f] * TZzm, &szm, &czm);
+      if constexpr (ZB) {
+        szm = z_back<false, R>(sz, ze.s[f], e0);
+        czm = z_back<false, R>(cz, ze.c[f], e0);
+      } else {
+        T::sc(q[f] * TZzm, &szm, &czm);
+      }
       const R ar = C[cr], ai = C[ci];
       const R rxp = Nx[cr], ixp = Nx[ci];
-      if (!EARLY) phi_rows(f);
+      if (!EARLY && !(ZB && f == 0)) phi_rows(f);
       const R ryp = Pyp[cr], iyp = Pyp[ci], rym = Pym[cr], iym = Pym[ci];
       const R rzp = Pzp[cr], izp = Pzp[ci], rzm = Pzm[cr], izm = Pzm[ci];
       {
