@@ -589,7 +589,7 @@ __global__ void __launch_bounds__(1024) scan_kernel(const int *__restrict__ in, 
 }
 
 /* ------------------- marching diagnostics (Abelian-Higgs) -----------------
- * One 64-lane wave per (64-site z chunk, row, x segment) marching along x,
+ * One 64-lane wave per (chunk of 64 sites of a plane, x segment) marching along x,
  * as the step kernel.  Per site it evaluates the energy density and Gauss
  * residual with the expressions of site_energy_ah (the same per-site bits;
  * with x/y or z not periodic only the bulk region's terms are summed, as
@@ -825,7 +825,7 @@ __global__ void __launch_bounds__(64) wind_march_kernel(int nx, int ny, int nz, 
 /* ------------------ marching diagnostics (Moore model) -------------------
  * Energy density and Gauss residual of site_energy_moore (the same
  * expressions in the same order, so the same per-site terms) by one wave
- * per (64-site z chunk, row, x segment) marching along x: both scalars and
+ * per (chunk of 64 sites of a plane, x segment) marching along x: both scalars and
  * theta_x (both levels) of plane x-1 are carried from the previous plane,
  * and plane x+1's current level is loaded once, as the next plane's centre.
  * The site kernel reads the x-neighbour planes, which another pass over the

@@ -26,7 +26,7 @@
  * Each field value is loaded once per step by the wave that owns it: plane
  * x+1 (current level) is loaded as the next iteration's centre and carried;
  * the y/z neighbour rows are meant to be cache hits (at 512^3 FP64 the L2 ->
- * fabric reads are 1.23x the algorithmic bytes, part of them served by the
+ * fabric reads are 1.27x the algorithmic ones, part of them served by the
  * Infinity Cache).  The loop's loads and stores are raw
  * buffer accesses (bld/bst below) whose addresses cost no vector
  * instructions; the previous level's reads and the new level's writes carry
@@ -421,7 +421,7 @@ __device__ __forceinline__ void row_pair(__amdgpu_buffer_rsrc_t r, double *lds, 
  * edge pass.  So a plane takes 10 load requests (22 with the five rows from
  * HBM alone in LDS), no load's latency is exposed, and y-neighbour rows are
  * read one plane after their own wave reads them, not two: 512^3 L2 -> fabric
- * reads 15.5 -> 13.2 GB per step, 3.755 -> 3.625 ms; 256^3 496 -> 474 us (the
+ * reads 15.9 -> 13.6 GB per step, 3.755 -> 3.625 ms; 256^3 496 -> 474 us (the
  * five rows: 3.747 -> 3.713 ms over none).  What bounds it then is the FP64
  * arithmetic: 84 % of the issue slots, at the 1.7 GHz the card holds under
  * it.  FP32, four rows per request, stays at its fabric bandwidth: 512^3

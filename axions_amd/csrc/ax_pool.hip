@@ -5,7 +5,7 @@
  * Device side
  *   pool_step_kernel   persistent kernel; one launch advances every resident
  *                      lattice by one TimeStep.  Its work items are the
- *                      (z chunk, y row, x segment) marches of ah_march for all
+ *                      (64-site chunk, x segment) marches of ah_march for all
  *                      lattices back to back; a fixed grid of one-wave
  *                      workgroups strides through them.  Which lattices exist,
  *                      where their state lives, their timestep and tile shape
@@ -158,7 +158,7 @@ __device__ __forceinline__ void flush_counts(const int *v, unsigned long long *d
 }
 
 /* The winding passes march over the step kernel's work items (same table,
- * same XCD-aware order): item -> lattice, z chunk, row, x segment.  A
+ * same XCD-aware order): item -> lattice, 64-site chunk, x segment.  A
  * workgroup keeps its counts in registers while consecutive items belong to
  * one lattice and adds them to that lattice's counters when the lattice
  * changes.  which = 0: the state before the chunk's first step (lattices

@@ -124,8 +124,9 @@ bool use_tiled_ah(const ax_params &p) {
 
 /* x planes per wave: tile_xseg's rule, up to the length that is best on
  * large lattices (measured at 512^3 AH, 256^3 Moore, on one box each):
- * Abelian-Higgs FP64 32 (3.875 ms; 8: 3.95, 16: 3.90, 24: 3.88), FP32 16
- * (1.816 ms; 8: 1.834, 12: 1.823, 32: 1.826); Moore FP64 16 (0.963 ms; 4:
+ * Abelian-Higgs FP64 32 (3.607 ms; 8: 3.746, 16: 3.644, 24: 3.631, 48: 3.603;
+ * 256^3 32: 0.459, 16: 0.468), FP32 16 (1.737 ms; 8: 1.762, 12: 1.758, 32:
+ * 1.756); Moore FP64 16 (0.963 ms; 4:
  * 0.993, 8: 0.979, 32: 0.974), FP32 8 (0.422 ms; 32: 0.444).  Moore FP32 has
  * the cheapest prologue against a plane and takes half the rule's length
  * (128^3: 8 planes 72 us, 6 65, 3 60; 160^3: 8 135, 4 118). */
