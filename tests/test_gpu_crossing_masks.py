@@ -2,23 +2,42 @@
 masks: after other lattices' calls left theirs in the shared scratch, with a
 last chunk of 1..64 sites, more and fewer sites than a group, and room for no,
 some and all points, it writes the rows that ax_crossings returns."""
+import ctypes
+
 import numpy as np
 import pytest
-import torch
 
 import axions_amd as ax
 from axions_amd.lattice import lib
 
 pytestmark = pytest.mark.gpu
 
+hip = ctypes.CDLL("libamdhip64.so")
+hip.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
+hip.hipFree.argtypes = [ctypes.c_void_p]
+hip.hipMemcpy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+hip.hipMemset.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t]
+D2H = 2
+UNTOUCHED = np.uint64(0xFFFFFFFFFFFFFFFF)
+
 
 def noalloc(lat, cap):
-    pts = torch.full((max(cap, 1) + 1, 3), -7.0, dtype=torch.float64, device="cuda")
-    cnt = torch.zeros(1, dtype=torch.int64, device="cuda")
-    torch.cuda.synchronize()
-    assert lib.ax_crossings_noalloc(lat.handle, pts.data_ptr() if cap else None, cap, cnt.data_ptr()) == 0
-    lat.sync()
-    return int(cnt), pts.cpu().numpy()
+    """The count, and the bits of cap + 1 rows, of which the call may write cap."""
+    rows = np.empty((cap + 1, 3), dtype=np.uint64)
+    count = np.empty(1, dtype=np.int64)
+    buf = ctypes.c_void_p()
+    assert hip.hipMalloc(ctypes.byref(buf), rows.nbytes + 8) == 0
+    try:
+        assert hip.hipMemset(buf, 0xFF, rows.nbytes + 8) == 0
+        cnt = buf.value + rows.nbytes
+        rc = lib.ax_crossings_noalloc(lat.handle, buf if cap else None, cap, cnt)
+        assert rc == 0, lib.ax_last_error().decode()
+        lat.sync()
+        assert hip.hipMemcpy(rows.ctypes.data, buf, rows.nbytes, D2H) == 0
+        assert hip.hipMemcpy(count.ctypes.data, cnt, 8, D2H) == 0
+    finally:
+        assert hip.hipFree(buf) == 0
+    return int(count[0]), rows
 
 
 @pytest.mark.parametrize("precision", [64, 32])
@@ -37,7 +56,7 @@ def test_masked_points(shape, precision):
             n, _ = noalloc(lat, 0)
             assert n == total == len(want) > 0
             for cap in (1, n // 2, n):
-                got, pts = noalloc(lat, cap)
+                got, rows = noalloc(lat, cap)
                 assert got == n
-                assert np.array_equal(pts[:cap].view(np.uint64), want[:cap].view(np.uint64))
-                assert (pts[cap:] == -7.0).all()
+                assert np.array_equal(rows[:cap], want[:cap].view(np.uint64))
+                assert (rows[cap:] == UNTOUCHED).all()
