@@ -126,17 +126,21 @@ bool use_tiled_ah(const ax_params &p) {
  * large lattices (measured at 512^3 AH, 256^3 Moore, on one box each):
  * Abelian-Higgs FP64 32 (3.607 ms; 8: 3.746, 16: 3.644, 24: 3.631, 48: 3.603;
  * 256^3 32: 0.459, 16: 0.468), FP32 16 (1.737 ms; 8: 1.762, 12: 1.758, 32:
- * 1.756); Moore FP64 16 (0.963 ms; 4:
- * 0.993, 8: 0.979, 32: 0.974), FP32 8 (0.422 ms; 32: 0.444).  Moore FP32 has
- * the cheapest prologue against a plane and takes half the rule's length
- * (128^3: 8 planes 72 us, 6 65, 3 60; 160^3: 8 135, 4 118). */
+ * 1.756); Moore FP64 16
+ * (0.800 ms; 8: 0.807, 9: 0.808, 10 and 12: 0.800), FP32 8 (0.422 ms; 32:
+ * 0.444).  Moore's prologue is cheap against a plane, so below that it takes
+ * half the rule's length (rule / half, us: FP64 201x201x51 fixed 141.6 / 133.8,
+ * 100^3 fixed 70.1 / 65.4, 150^3 fixed 203 / 197, periodic 181 / 179, 200^3
+ * fixed 464 / 452, 128^3 110.5 / 108.1; FP32 128^3 65 / 60, 160^3 135 / 118),
+ * in FP64 from 3 planes on (64^3 2: 19.2, 1: 21.0). */
 int default_xseg(const ax_params &p) {
   const char *xe = getenv("AX_TILED_XSEG");
   if (xe) return atoi(xe);
   const bool f32 = p.precision == 32;
   if (p.model != AX_MODEL_MOORE) return tile_xseg(p.nx, p.ny, p.nz, f32 ? 16 : 32);
   const int xs = tile_xseg(p.nx, p.ny, p.nz, 16);
-  return f32 ? (xs + 1) / 2 : xs;
+  const bool at_cap = (long long)tile_chunks(p.ny, p.nz) * p.nx >= 240 * 1024;   /* the rule's length 15.5 or more */
+  return f32 || (xs > 2 && !at_cap) ? (xs + 1) / 2 : xs;
 }
 
 /* The LDS prefetch of the FP64 march applies: whole 64-site chunks (across
