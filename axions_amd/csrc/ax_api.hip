@@ -688,7 +688,7 @@ static bool fused_ok(const ax_lattice *L) {
  * divergence plane, the partial sums, the results and the edge values (the
  * output step stores them whether or not windings are wanted) */
 static int ensure_fused(ax_lattice *L, size_t npoints) {
-  const size_t items = (size_t)fused_work_items(L->p.nx, L->p.ny, L->p.nz, L->xseg);
+  const size_t items = tile_items_max(L->p.nx, L->p.ny, L->p.nz, L->xseg);
   auto grow = [&](double **buf, size_t *have, size_t want, const char *what) -> int {
     if (*have >= want) return AX_OK;
     if (*buf) (void)hipFree(*buf);
@@ -928,11 +928,12 @@ bool use_diag_march(const ax_params &p) {
   return p.model == AX_MODEL_AH && getenv("AX_DIAG_SITE_KERNEL") == nullptr;
 }
 
-/* partial-sum blocks any diagnostic pass of this lattice writes */
+/* partial-sum blocks any diagnostic pass of this lattice writes, in either
+ * work order */
 size_t diag_part_blocks(const ax_params &p) {
   const size_t V = (size_t)p.nx * p.ny * p.nz;
   const size_t site = (V + 255) / 256;
-  const size_t march = (size_t)make_tile_grid(p.nx, p.ny, p.nz, diag_xseg(p.nx, p.ny, p.nz)).work;
+  const size_t march = tile_items_max(p.nx, p.ny, p.nz, diag_xseg(p.nx, p.ny, p.nz));
   const size_t glob = p.model == AX_MODEL_GLOBAL ? global_energy_blocks(p) : 0;
   return std::max(site, std::max(march, glob));
 }

@@ -45,6 +45,14 @@ inline TileGrid make_tile_grid(int nx, int ny, int nz, int xseg) {
   return g;
 }
 
+/* Workgroups of a march in whichever order takes more: what a buffer of one
+ * entry per workgroup holds, so that it serves launches of either order
+ * (AX_TILE_ORDER is read at each launch). */
+inline size_t tile_items_max(int nx, int ny, int nz, int xseg) {
+  const int xs = (xseg <= 0 || xseg > nx) ? nx : xseg;
+  return (size_t)8 * ((tile_chunks(ny, nz) + 7) / 8) * ((nx + xs - 1) / xs);
+}
+
 /* chunk and x segment of workgroup w; false for an empty one */
 __device__ __forceinline__ bool tile_item(const TileGrid &g, int w, int &chunk, int &seg) {
   if (g.per) {
@@ -228,7 +236,7 @@ inline size_t cross_mask_bytes(size_t V) { return (V + 63) / 64 * 3 * sizeof(uin
 /* Fused diagnostics (ax_march.h MODE 1/2, FP64 periodic Abelian-Higgs) */
 struct FusedDiag;
 struct EnergyConsts;
-int fused_work_items(int nx, int ny, int nz, int xseg);
+int fused_work_items(int nx, int ny, int nz, int xseg);   /* of the launch, at most tile_items_max */
 hipError_t launch_step_fused(const StepConsts &k, const Levels<double> &L, int xseg, hipStream_t st, int mode,
                              bool p2d, const FusedDiag &fd);
 /* the sums of a into out3 and, where b holds any, of b into outb3 (which
