@@ -668,6 +668,13 @@ int ax_diagnostics(ax_lattice *L, int32_t want_winding, ax_diag *out) {
   else L->hres[0] = L->hres[1] = L->hres[2] = 0;   /* a global lattice before its first step */
   if (e == hipSuccess) e = hipStreamSynchronize(L->stream);
   if (e != hipSuccess) return hip_fail(e, "diag readback");
+  if (want_winding && std::isnan(L->hres[4])) {   /* links beyond the FP32 edge values (kEdgeExact) */
+    int rc = launch_site_winding(L, 0, nullptr, winds);
+    if (rc) return rc;
+    e = launch_sums(winds, L->hres + 4, {nullptr, 0}, nullptr, L->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(L->stream);
+    if (e != hipSuccess) return hip_fail(e, "winding readback");
+  }
   fill_diag(L, L->hres, L->timestep, want_winding != 0, out);
   return AX_OK;
 }
@@ -844,7 +851,15 @@ int ax_winding_field(ax_lattice *L, int32_t field, int8_t *out, size_t n) {
   Partials winds = {L->part + 3 * L->part_n, 0};
   if (!rc) rc = launch_winding_field(L, field, L->wind, winds);
   if (rc) return rc;
-  const hipError_t e = download(L, {{(const char *)L->wind, (char *)out, n, false}});
+  const std::vector<Run> map = {{(const char *)L->wind, (char *)out, n, false}};
+  const bool faces = L->p.boundary != AX_BC_PERIODIC || L->p.boundary_z != AX_BC_PERIODIC;
+  hipError_t e = faces ? launch_sums(winds, L->hres + 4, {nullptr, 0}, nullptr, L->stream) : hipSuccess;
+  if (e == hipSuccess) e = download(L, map);
+  if (e == hipSuccess && faces && std::isnan(L->hres[4])) {   /* as ax_diagnostics */
+    rc = launch_site_winding(L, field, L->wind, winds);
+    if (rc) return rc;
+    e = download(L, map);
+  }
   return e == hipSuccess ? AX_OK : hip_fail(e, "winding readback");
 }
 
@@ -973,7 +988,14 @@ int ensure_winding_buffer(ax_lattice *L) {
   return AX_OK;
 }
 
-int launch_winding_field(ax_lattice *L, int field, int8_t *out, Partials &part) {
+/* Operands of field's windings in planes of the state: phi (re, im) from c,
+ * the links from t. */
+struct WindingArgs {
+  int ex, ez;
+  double q;
+  size_t c[2], t[3];
+};
+static WindingArgs winding_args(const ax_lattice *L, int field) {
   const ax_params &p = L->p;
   const bool glob = p.model == AX_MODEL_GLOBAL;
   const int tN = glob ? L->timestep % 2 : (L->timestep + 1) % 2;
@@ -982,38 +1004,50 @@ int launch_winding_field(ax_lattice *L, int field, int8_t *out, Partials &part) 
   /* global model: no links; charge 0 makes every link phase exp(0) (the
    * momentum planes only stand in as finite link operands) */
   const double q = p.model == AX_MODEL_AH ? 1.0 : glob ? 0.0 : (double)(field == 0 ? p.q1 : p.q2);
-  hipError_t e;
   auto P = [&](int c) { return glob && c >= 2 ? (size_t)4 * L->pitch : (size_t)(c * 2 + tN) * L->pitch; };
-  const int ex = !glob && p.boundary != AX_BC_PERIODIC, ez = !glob && p.boundary_z != AX_BC_PERIODIC;
-  /* the marching edge-value passes (ax_wind.h; three edge phases a site and
-   * the same integers as the site kernel, which evaluates nine: 256^3 FP64
-   * with absorbing faces 0.78 ms against 0.20 within the energy march), while
-   * memory holds the edge values */
-  if (getenv("AX_DIAG_SITE_KERNEL") == nullptr && ensure_phase_buffer(L) == AX_OK) {
-    if (L->esize == 8) {
-      const double *b = (const double *)L->state;
-      e = launch_edge_winding<double>(p.nx, p.ny, p.nz, ex, ez, b + P(c0), b + P(c0 + 1), b + P(t0), b + P(t0 + 1),
-                                      b + P(t0 + 2), q, L->phase, out, part, L->stream);
-    } else {
-      const float *b = (const float *)L->state;
-      e = launch_edge_winding<float>(p.nx, p.ny, p.nz, ex, ez, b + P(c0), b + P(c0 + 1), b + P(t0), b + P(t0 + 1),
-                                     b + P(t0 + 2), q, L->phase, out, part, L->stream);
-    }
-    return e == hipSuccess ? AX_OK : hip_fail(e, "winding launch");
-  }
+  return {!glob && p.boundary != AX_BC_PERIODIC, !glob && p.boundary_z != AX_BC_PERIODIC, q,
+          {P(c0), P(c0 + 1)}, {P(t0), P(t0 + 1), P(t0 + 2)}};
+}
+
+int launch_site_winding(ax_lattice *L, int field, int8_t *out, Partials &part) {
+  const ax_params &p = L->p;
+  const WindingArgs w = winding_args(L, field);
   if (!out) {   /* the site kernel stores the field whether wanted or not */
     int rc = ensure_winding_buffer(L);
     if (rc) return rc;
     out = L->wind;
   }
+  hipError_t e;
   if (L->esize == 8) {
     const double *b = (const double *)L->state;
-    e = launch_winding<double>(p.nx, p.ny, p.nz, b + P(c0), b + P(c0 + 1), b + P(t0), b + P(t0 + 1), b + P(t0 + 2), q,
-                               ex, ez, out, part, L->stream);
+    e = launch_winding<double>(p.nx, p.ny, p.nz, b + w.c[0], b + w.c[1], b + w.t[0], b + w.t[1], b + w.t[2], w.q, w.ex,
+                               w.ez, out, part, L->stream);
   } else {
     const float *b = (const float *)L->state;
-    e = launch_winding<float>(p.nx, p.ny, p.nz, b + P(c0), b + P(c0 + 1), b + P(t0), b + P(t0 + 1), b + P(t0 + 2), q,
-                              ex, ez, out, part, L->stream);
+    e = launch_winding<float>(p.nx, p.ny, p.nz, b + w.c[0], b + w.c[1], b + w.t[0], b + w.t[1], b + w.t[2], w.q, w.ex,
+                              w.ez, out, part, L->stream);
+  }
+  return e == hipSuccess ? AX_OK : hip_fail(e, "winding launch");
+}
+
+int launch_winding_field(ax_lattice *L, int field, int8_t *out, Partials &part) {
+  /* the marching edge-value passes (ax_wind.h; three edge phases a site and
+   * the same integers as the site kernel, which evaluates nine: 256^3 FP64
+   * with absorbing faces 0.78 ms against 0.20 within the energy march), while
+   * memory holds the edge values */
+  if (getenv("AX_DIAG_SITE_KERNEL") != nullptr || ensure_phase_buffer(L) != AX_OK)
+    return launch_site_winding(L, field, out, part);
+  const ax_params &p = L->p;
+  const WindingArgs w = winding_args(L, field);
+  hipError_t e;
+  if (L->esize == 8) {
+    const double *b = (const double *)L->state;
+    e = launch_edge_winding<double>(p.nx, p.ny, p.nz, w.ex, w.ez, b + w.c[0], b + w.c[1], b + w.t[0], b + w.t[1],
+                                    b + w.t[2], w.q, L->phase, out, part, L->stream);
+  } else {
+    const float *b = (const float *)L->state;
+    e = launch_edge_winding<float>(p.nx, p.ny, p.nz, w.ex, w.ez, b + w.c[0], b + w.c[1], b + w.t[0], b + w.t[1],
+                                   b + w.t[2], w.q, L->phase, out, part, L->stream);
   }
   return e == hipSuccess ? AX_OK : hip_fail(e, "winding launch");
 }

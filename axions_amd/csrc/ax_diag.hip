@@ -790,9 +790,10 @@ __global__ void __launch_bounds__(64, sizeof(T) == 8 ? 3 : 1) diag_march_kernel(
 /* Windings of the current level from the edge values the marching
  * diagnostics stored (wind_march, ax_wind.h): one wave per work item of
  * the tile grid, carrying plane x+1's values.  out (the winding field
- * [3][V]) may be null when only the counts are wanted. */
+ * [3][V]) may be null when only the counts are wanted.  An edge value above
+ * lim (kEdgeExact, or infinity) turns the counts into a NaN. */
 __global__ void __launch_bounds__(64) wind_march_kernel(int nx, int ny, int nz, const float *E, TileGrid g, int ex,
-                                                        int ez, int8_t *out, double *part) {
+                                                        int ez, double lim, int8_t *out, double *part) {
   const int item = (int)blockIdx.x;
   int chunk, seg;
   if (!tile_item(g, item, chunk, seg)) {
@@ -804,7 +805,7 @@ __global__ void __launch_bounds__(64) wind_march_kernel(int nx, int ny, int nz, 
   double tot[3] = {0, 0, 0};
   /* plaquettes that would wrap across a non-periodic axis do not exist */
   const bool ye = ex && w.y == ny - 1, ze = ez && w.z == nz - 1;
-  wind_march(w, E, x0, x1, [&](int x, size_t s, const int *wn) {
+  const double big = wind_march(w, E, x0, x1, [&](int x, size_t s, const int *wn) {
     const bool xe = ex && x == nx - 1;
     const bool none[3] = {xe || ye, xe || ze, ye || ze};
 #pragma unroll
@@ -814,6 +815,7 @@ __global__ void __launch_bounds__(64) wind_march_kernel(int nx, int ny, int nz, 
       tot[pl] += (double)(v < 0 ? -v : v);
     }
   });
+  if (big > lim) tot[0] = NAN;
   const double a = wave_sum(tot[0]), b = wave_sum(tot[1]), c = wave_sum(tot[2]);
   if ((threadIdx.x & 63) == 0) {
     part[3 * item] = a;
@@ -1094,7 +1096,8 @@ hipError_t launch_wind_phase(int nx, int ny, int nz, int ex, int ez, const float
                              hipStream_t st) {
   /* part holds 3 doubles per work item (diag_part_blocks) */
   const TileGrid g = make_tile_grid(nx, ny, nz, diag_xseg(nx, ny, nz));
-  hipLaunchKernelGGL(wind_march_kernel, dim3(g.work), dim3(64), 0, st, nx, ny, nz, E, g, ex, ez, out, part.p);
+  const double lim = ex || ez ? kEdgeExact : INFINITY;
+  hipLaunchKernelGGL(wind_march_kernel, dim3(g.work), dim3(64), 0, st, nx, ny, nz, E, g, ex, ez, lim, out, part.p);
   part.n = g.work;
   return hipGetLastError();
 }

@@ -167,7 +167,10 @@ int ensure_phase_buffer(ax_lattice *L);
 hipError_t launch_march_diag(ax_lattice *L, bool phases, Partials &part);
 hipError_t launch_phase_winding(ax_lattice *L, int8_t *out, Partials &part);
 int prepare_faces(ax_lattice *L);
-/* the Neumann faces prepared (prepare_faces); out may be null */
+/* the Neumann faces prepared (prepare_faces); out may be null.  With faces
+ * the counts are NaN where FP32 edge values did not hold the links, and
+ * launch_site_winding evaluates the windings then (the counts and out). */
+int launch_site_winding(ax_lattice *L, int field, int8_t *out, Partials &part);
 int launch_winding_field(ax_lattice *L, int field, int8_t *out, Partials &part);
 
 template <typename R>
@@ -193,8 +196,10 @@ hipError_t launch_global_energy(const ax_params &p, const void *state, size_t pi
 template <typename T>
 hipError_t launch_diag(const DiagConsts &k, const Levels<T> &L, Partials &part, hipStream_t st);
 /* Abelian-Higgs: energy/Gauss march, with phase != NULL also the FP32 edge
- * values [3][V] (forward edge phase + link angle, ax_wind.h); launch_wind_phase turns them into windings (the field into out when
- * out != NULL, the counts into part; ex, ez: x and y, z not periodic) */
+ * values [3][V] (forward edge phase + link angle, ax_wind.h);
+ * launch_wind_phase turns them into windings (the field into out when out !=
+ * NULL, the counts into part; ex, ez: x and y, z not periodic, and the counts
+ * are NaN where an edge value exceeds kEdgeExact) */
 /* x planes per wave of the diagnostics and winding marches (us per
  * ax_diagnostics call without / with windings; this rule against the best of
  * 1 ... 32 planes: 64^3 27.5 / 41.8 against 27.4 / 41.7, 160^3 125 / 244

@@ -115,9 +115,13 @@ struct WindRow : LaneSite<true> {
  * to a multiple of 2 pi; the exact phases of phi telescope around the
  * plaquette, so site_winding's sum lies within rounding of some 2 pi K.
  * The regrouped sum differs from it by rounding only -- half an ulp of
- * |delta + theta| per FP32 e, at most 2^-24 |e| -- far below pi for any
- * link angle below 2^20, so both round to K.  (Non-finite fields are
- * counted separately and fail the run.)  Computing delta any other way
+ * |delta + theta| per FP32 e, at most 1/4 each and 1 in the sum of four
+ * while |e| stays below kEdgeExact = 2^23, where pi is the limit -- so both
+ * round to K.  Beyond it the integers go wrong (link angles up to 1e8: 29 %
+ * of the plaquettes).  Lattices with faces, whose windings are evaluated
+ * again in FP64 then, are watched for it (wind_march's result); periodic
+ * ones, whose output steps leave no state to go back to, are not.
+ * (Non-finite fields are counted separately and fail the run.)  Computing delta any other way
  * (another atan2, FP32) would not keep this: an edge phase near +-pi may
  * then land on the other branch, 2 pi away.  FP32 e halves the bytes the
  * step writes and the winding pass reads. */
@@ -158,11 +162,14 @@ __device__ __forceinline__ int phase_march(const WindRow &w, const T *fr, const 
 
 /* Windings of the xy, xz, yz plaquettes of one wave's march from the stored
  * edge values E[a V + s] = e_a(s) of the same level (above).  emit(x, s, w) is
- * called for each of the lane's sites. */
+ * called for each of the lane's sites.  Returns the largest |e| of the lane's
+ * sites. */
+constexpr double kEdgeExact = 0x1p23;
 template <typename Emit>
-__device__ __forceinline__ void wind_march(const WindRow &w, const float *E, int x0, int x1, Emit emit) {
+__device__ __forceinline__ double wind_march(const WindRow &w, const float *E, int x0, int x1, Emit emit) {
   const float *EX = E, *EY = E + w.V, *EZ = E + 2 * w.V;
   double cX = w.get(EX, x0, w.o0), cY = w.get(EY, x0, w.o0), cZ = w.get(EZ, x0, w.o0);
+  double big = 0;
   for (int x = x0; x < x1; ++x) {
     const int xp = x == w.nx - 1 ? 0 : x + 1;
     /* plane x+1 (next centre), row y+1, site z+1 */
@@ -174,8 +181,10 @@ __device__ __forceinline__ void wind_march(const WindRow &w, const float *E, int
     wn[1] = (int)rint((cX + nZ - zX - cZ) * 0.15915494309189535);   /* (x, z) */
     wn[2] = (int)rint((cY + yZ - zY - cZ) * 0.15915494309189535);   /* (y, z) */
     if (w.act) emit(x, w.site(x), wn);
+    big = fmax(big, fmax(fmax(fabs(cX), fabs(cY)), fabs(cZ)));
     cX = nX; cY = nY; cZ = nZ;
   }
+  return big;
 }
 
 }  // namespace ax

@@ -200,7 +200,10 @@ int ax_step_diag(ax_lattice *lat, int32_t nsteps, int32_t every, int32_t want_wi
 /* Per-plaquette winding numbers of the current state, 3*nx*ny*nz int8 in
  * [plane][x][y][z] order, plane 0 = xy, 1 = xz, 2 = yz (plaquette spanned
  * from site s along the two axes).  No counterpart in the reference; see
- * the library documentation for the definition. */
+ * the library documentation for the definition.  Periodic lattices (and the
+ * ensemble pool) form them from FP32 edge values and are exact for link
+ * angles (times the charge) below 2^23 in magnitude; lattices with faces are
+ * evaluated in FP64 beyond that. */
 int ax_winding(ax_lattice *lat, int8_t *out, size_t n);
 /* Same for a chosen scalar: field 0 = phi (AH) or phi1 (Moore, links
  * scaled by q1), field 1 = phi2 (Moore, links scaled by q2). */
