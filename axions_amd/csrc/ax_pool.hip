@@ -106,8 +106,14 @@ __device__ __forceinline__ Levels<R> entry_levels(const BatchEntry &E, int t) {
   return L;
 }
 
+/* Waves per SIMD: FP32 five, FP64 two.  Both forms of the FP64 march take 185
+ * VGPRs; with three waves they spill, and the row-crossing form alone spilled
+ * 18 of them for every n.  ps per site update, a full pool, three waves
+ * and the row-crossing form alone / two waves and both forms: 64^3 38.5 /
+ * 30.9, 96^3 38.7 / 31.7, 100^3 41.6 / 32.6, 128^3 37.0 / 29.5; one lattice
+ * of 64^3 68.9 / 51.7, of 129^3 49.9 / 39.1. */
 template <typename R, bool POW2>
-__global__ void __launch_bounds__(64, sizeof(R) == 8 ? 3 : 5) pool_step_kernel(ax_params p, R lim, const BatchHeader *__restrict__ hdr,
+__global__ void __launch_bounds__(64, sizeof(R) == 8 ? 2 : 5) pool_step_kernel(ax_params p, R lim, const BatchHeader *__restrict__ hdr,
                                                        const BatchEntry *__restrict__ ent, int j) {
   const int count = hdr->count, work = hdr->work;
   /* XCD-aware order: the grid is resident at once and its workgroups are
@@ -133,9 +139,9 @@ __global__ void __launch_bounds__(64, sizeof(R) == 8 ? 3 : 5) pool_step_kernel(a
     march_consts_from<R>(make_step_consts(p, t), lim, m);
     const Levels<R> L = entry_levels<R>(E, t);
     const uint32_t p0 = (uint32_t)chunk * 64;
-    /* FP64 takes chunks across rows for every n: both forms in one kernel
-     * would spill */
-    if (sizeof(R) == 8 || E.n % 64) ah_march<R, POW2, 2, false, false, 0, false, true>(m, L, E.n, E.n, E.n, p0, x0, x1);
+    /* whole chunks keep their row offsets on the scalar unit, as in the
+     * single-lattice kernels */
+    if (E.n % 64) ah_march<R, POW2, 2, false, false, 0, false, true>(m, L, E.n, E.n, E.n, p0, x0, x1);
     else ah_march<R, POW2, 2>(m, L, E.n, E.n, E.n, p0, x0, x1);
   }
 }
