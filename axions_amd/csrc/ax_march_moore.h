@@ -117,13 +117,13 @@ __device__ __forceinline__ void moore_march(const MooreConsts<R> &k, const Level
    * -> 800, chunks across rows with the check 150^3 181 -> 184 (registers). */
   constexpr bool ZB = sizeof(R) == 8 && BUF && !FLAT && CHECK;
   constexpr bool EARLY = sizeof(R) == 8 && BUF && FLAT && !CHECK;
-  const uint32_t NYNZ = (uint32_t)NY * (uint32_t)NZ;
+  const size_t NYNZ = (size_t)NY * NZ;
   const LaneSite<FLAT> ls(NY, NZ, p0);
   const int y = ls.y, z = ls.z;
   /* xfix, zfix: x and y, z not periodic; their face sites are not stepped */
   const bool act = ls.act && !(zfix && (z == 0 || z == NZ - 1)) && !(xfix && (y == 0 || y == NY - 1));
   const uint32_t E = (uint32_t)sizeof(R);
-  const uint32_t PLB = NYNZ * E;          /* plane bytes */
+  const uint32_t PLB = (uint32_t)NYNZ * E;          /* plane bytes */
   auto row = [&](int r) { return ls.row(r, E); };
   auto col = [&](int r, int c) { return ls.col(r, c, E); };
   const uint32_t R0 = row(0), RM = row(-1), RP = row(1);
