@@ -44,6 +44,7 @@ struct GlobalGeom {
   int periodic;          /* 1: all sites updated, periodic wrap; 0: Neumann x/y faces */
   double dx, dy, dz, dt;
   uint32_t V, per, eper;   /* sites; blocks of the step and of the energy per XCD */
+  uint32_t eruns;          /* runs of 256 threads' sites a block of the energy takes */
   bool wide;               /* two sites a thread */
   FastDiv by_nz, by_ny;
 };
@@ -210,8 +211,14 @@ __global__ void __launch_bounds__(256) global_step_kernel(GlobalGeom g, GlobalCo
 }
 
 /* o: the pre-step field, n: the step's result, m: its momentum.  A block
- * takes kEnergyRuns consecutive runs of 256 threads' sites. */
-constexpr int kEnergyRuns = 4;
+ * takes g.eruns consecutive runs of 256 threads' sites: four, which leaves a
+ * fourth of the partial sums, while the chip still gets four blocks a CU, and
+ * fewer on small lattices, where one run after another is what the call waits
+ * for (us per ax_diagnostics, FP64, periodic, dx 0.7, four runs / this rule:
+ * 16^3 23.6 / 18.3, 33x47x80 24.6 / 19.2, 64^3 24.6 / 21.8, 128^3 and more
+ * have four either way; one site a block's thread, without runs: 20.1, 21.6,
+ * 24.2). */
+constexpr uint32_t kEnergyRuns = 4;
 template <typename R, bool POW2, int W>
 __global__ void __launch_bounds__(256) global_energy_kernel(GlobalGeom g, GlobalConsts<R> c, const R *__restrict__ ar,
                                                             const R *__restrict__ ai, const R *__restrict__ br,
@@ -223,8 +230,8 @@ __global__ void __launch_bounds__(256) global_energy_kernel(GlobalGeom g, Global
   const uint32_t blk = (blockIdx.x & 7) * g.eper + (blockIdx.x >> 3);
   const R *o[2] = {ar, ai}, *n[2] = {br, bi}, *m[2] = {mr, mi};
 #pragma unroll 1
-  for (int run = 0; run < kEnergyRuns; ++run) {
-    const GlobalSite<W> q(g, blk * kEnergyRuns + run);
+  for (uint32_t run = 0; run < g.eruns; ++run) {
+    const GlobalSite<W> q(g, blk * g.eruns + run);
     /* a neighbour holds its new value when it is an updated site earlier in
      * loop order (x, then y, then z): x - 1 and y - 1 unless they wrap or are
      * faces, z - 1 unless it wraps; x + 1, y + 1, z + 1 only where they wrap */
@@ -299,7 +306,8 @@ static GlobalGeom geom_of(const ax_params &p) {
   g.wide = p.nz % 2 == 0;
   const uint32_t runs = (g.V + 255) / 256 / (g.wide ? 2 : 1) + 1;   /* of 256 threads */
   g.per = (runs + 7) / 8;
-  g.eper = ((runs + kEnergyRuns - 1) / kEnergyRuns + 7) / 8;
+  g.eruns = std::min(kEnergyRuns, (runs + 1023) / 1024);
+  g.eper = ((runs + g.eruns - 1) / g.eruns + 7) / 8;
   g.by_nz = fast_div((uint32_t)p.nz);
   g.by_ny = fast_div((uint32_t)p.ny);
   return g;
