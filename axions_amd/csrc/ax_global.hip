@@ -99,11 +99,12 @@ __global__ void __launch_bounds__(256) global_bc_kernel(GlobalGeom g, R *pr, R *
   qi[d] = vi;
 }
 
-/* W sites of a thread: one, or two neighbours along z (nz even, so that both
- * lie in one row and their 16 (FP64) or 8 bytes are aligned).  A request
- * takes the addresser the same time whatever a lane's width, and both kernels
- * were bound by it (busy 78 % of the launch): with two sites a lane issues 9
- * instead of 20 requests per site (step), 11 instead of 26 (energy). */
+/* W sites of a thread: one, or two neighbours along z (nz and the planes'
+ * pitch even, so that both lie in one row and their 16 (FP64) or 8 bytes are
+ * aligned).  A request takes the addresser the same time whatever a lane's
+ * width, and both kernels were bound by it (busy 78 % of the launch): with two
+ * sites a lane issues 9 instead of 20 requests per site (step), 11 instead of
+ * 26 (energy). */
 template <typename R, int W>
 struct Sites {
   typedef R vec __attribute__((ext_vector_type(W)));
@@ -297,13 +298,14 @@ __global__ void __launch_bounds__(256) global_energy_kernel(GlobalGeom g, Global
   }
 }
 
-static GlobalGeom geom_of(const ax_params &p) {
+/* pitch: of the planes, whose two-site loads need it even as well */
+static GlobalGeom geom_of(const ax_params &p, size_t pitch) {
   GlobalGeom g;
   g.nx = p.nx; g.ny = p.ny; g.nz = p.nz;
   g.periodic = p.boundary == AX_BC_PERIODIC;
   g.dx = p.dx; g.dy = p.dy; g.dz = p.dz; g.dt = p.dt;
   g.V = (uint32_t)p.nx * p.ny * p.nz;
-  g.wide = p.nz % 2 == 0;
+  g.wide = p.nz % 2 == 0 && pitch % 2 == 0;
   const uint32_t runs = (g.V + 255) / 256 / (g.wide ? 2 : 1) + 1;   /* of 256 threads */
   g.per = (runs + 7) / 8;
   g.eruns = std::min(kEnergyRuns, (runs + 1023) / 1024);
@@ -313,7 +315,7 @@ static GlobalGeom geom_of(const ax_params &p) {
   return g;
 }
 
-size_t global_energy_blocks(const ax_params &p) { return (size_t)8 * geom_of(p).eper; }
+size_t global_energy_blocks(const ax_params &p) { return (size_t)8 * std::max(geom_of(p, 0).eper, geom_of(p, 1).eper); }
 
 template <typename R>
 static GlobalConsts<R> consts_of(const ax_params &p) {
@@ -342,7 +344,7 @@ hipError_t launch_global_step(const ax_params &p, void *state, size_t pitch, int
   R *ar = b + (size_t)(0 + cur) * pitch, *ai = b + (size_t)(2 + cur) * pitch;
   R *br = b + (size_t)(0 + nw) * pitch, *bi = b + (size_t)(2 + nw) * pitch;
   R *mr = b + 4 * pitch, *mi = b + 5 * pitch;
-  const GlobalGeom g = geom_of(p);
+  const GlobalGeom g = geom_of(p, pitch);
   if (!g.periodic) {
     const int nbs = 2 * p.ny * p.nz + 2 * (p.nx - 2) * p.nz;
     hipLaunchKernelGGL((global_bc_kernel<R>), dim3((nbs + 255) / 256), dim3(256), 0, st, g, ar, ai, br, bi);
@@ -365,7 +367,7 @@ hipError_t launch_global_energy(const ax_params &p, const void *state, size_t pi
                                 hipStream_t st) {
   const R *b = (const R *)state;
   const int cur = n % 2, nw = 1 - cur;   /* the pre-step field of TimeStep n and its result */
-  const GlobalGeom g = geom_of(p);
+  const GlobalGeom g = geom_of(p, pitch);
   const GlobalConsts<R> k = consts_of<R>(p);
   const dim3 grid(8 * g.eper), block(256);   /* part holds 3 doubles each (diag_part_blocks) */
 #define AX_GE(P2, W)                                                                                              \

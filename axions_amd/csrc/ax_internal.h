@@ -196,7 +196,7 @@ hipError_t launch_step_tiled_moore(const StepConsts &k, const Levels<R> &L, int 
 
 template <typename R>
 hipError_t launch_global_step(const ax_params &p, void *state, size_t pitch, int n, hipStream_t st);
-size_t global_energy_blocks(const ax_params &p);   /* partial-sum blocks of launch_global_energy */
+size_t global_energy_blocks(const ax_params &p);   /* partial-sum blocks of launch_global_energy, whatever the pitch */
 template <typename R>
 hipError_t launch_global_energy(const ax_params &p, const void *state, size_t pitch, int n, Partials &part,
                                 hipStream_t st);
