@@ -15,7 +15,6 @@
 #include <string.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cstdlib>
 #include <cstdio>
 #include <new>
@@ -25,6 +24,7 @@
 #include <vector>
 
 #include "ax_device.h"
+#include "ax_download.h"
 #include "ax_energy.h"
 #include "ax_internal.h"
 #include "ax_march.h"
@@ -351,112 +351,16 @@ int ax_set_state(ax_lattice *L, const double *host, size_t n) {
   return e == hipSuccess ? AX_OK : hip_fail(e, "set_state");
 }
 
-/* One run of a download: n values at dev, as they are (bytes) or floats
- * widened to doubles, to host. */
-struct Run {
-  const char *dev;
-  char *host;
-  size_t n;
-  bool widen;
-};
-
-/* Device to host, waiting for it.  The runtime takes pageable memory through
- * its own staging with one thread (17 GB/s here); runs of kDirect bytes or
- * more in all go through pinned memory in pieces instead, kCopiers threads
- * each with two pieces, one arriving while the other is copied out and, for
- * FP32 lattices, widened.  State of 64^3 FP64 (21 MB) 1.33 -> 0.78 ms, of 64^3
- * FP32 1.03 -> 0.42, of 160^3 FP64 (328 MB) 32 -> 11. */
-constexpr size_t kDirect = (size_t)4 << 20;
-constexpr size_t kPiece = (size_t)1 << 20;
-constexpr int kCopiers = 4;
-
-static hipError_t download(ax_lattice *L, const std::vector<Run> &runs) {
-  struct Piece {
-    const char *dev;
-    char *host;
-    size_t n;   /* device bytes */
-    bool widen;
-  };
-  std::vector<Piece> pieces;
-  size_t total = 0;
-  for (const Run &r : runs) {
-    const size_t bytes = r.widen ? 4 * r.n : r.n;
-    total += bytes;
-    for (size_t o = 0; o < bytes; o += kPiece)
-      pieces.push_back({r.dev + o, r.host + (r.widen ? 2 * o : o), std::min(kPiece, bytes - o), r.widen});
-  }
-  if (total >= kDirect && !L->stage &&
-      hipHostMalloc((void **)&L->stage, 2 * kCopiers * kPiece, hipHostMallocDefault) != hipSuccess) {
-    (void)hipGetLastError();   /* clear the sticky error of the failed call */
-    L->stage = nullptr;
-  }
-  auto out = [](const Piece &p, const char *from) {
-    if (!p.widen) {
-      memcpy(p.host, from, p.n);
-      return;
-    }
-    const float *f = (const float *)from;
-    double *d = (double *)p.host;
-    for (size_t i = 0; i < p.n / 4; ++i) d[i] = f[i];
-  };
-  if (total < kDirect || !L->stage) {
-    std::vector<char> tmp;
-    hipError_t e = hipSuccess;
-    for (size_t i = 0; i < pieces.size() && e == hipSuccess; ++i) {
-      const Piece &p = pieces[i];
-      if (p.widen) tmp.resize(kPiece);
-      e = hipMemcpyAsync(p.widen ? tmp.data() : p.host, p.dev, p.n, hipMemcpyDeviceToHost, L->stream);
-      if (e == hipSuccess && p.widen) {
-        e = hipStreamSynchronize(L->stream);
-        if (e == hipSuccess) out(p, tmp.data());
-      }
-    }
-    const hipError_t w = hipStreamSynchronize(L->stream);
-    return e == hipSuccess ? w : e;
-  }
-  std::atomic<int> failed{(int)hipSuccess};
-  auto copier = [&](int t) {
-    hipEvent_t ev[2] = {nullptr, nullptr};
-    hipError_t e = hipSetDevice(L->device);
-    for (int q = 0; q < 2 && e == hipSuccess; ++q) e = hipEventCreateWithFlags(&ev[q], hipEventDisableTiming);
-    auto fetch = [&](size_t i, int q) {
-      char *to = L->stage + (size_t)(2 * t + q) * kPiece;
-      if (e == hipSuccess) e = hipMemcpyAsync(to, pieces[i].dev, pieces[i].n, hipMemcpyDeviceToHost, L->stream);
-      if (e == hipSuccess) e = hipEventRecord(ev[q], L->stream);
-    };
-    if ((size_t)t < pieces.size()) fetch(t, 0);
-    int q = 0;
-    for (size_t i = t; i < pieces.size() && e == hipSuccess; i += kCopiers, q ^= 1) {
-      if (i + kCopiers < pieces.size()) fetch(i + kCopiers, q ^ 1);
-      if (e == hipSuccess) e = hipEventSynchronize(ev[q]);
-      if (e == hipSuccess) out(pieces[i], L->stage + (size_t)(2 * t + q) * kPiece);
-    }
-    if (e != hipSuccess) failed = (int)e;
-    for (hipEvent_t x : ev)
-      if (x) (void)hipEventDestroy(x);
-  };
-  std::vector<std::thread> th;
-  try {
-    for (int t = 1; t < kCopiers; ++t) th.emplace_back(copier, t);
-  } catch (...) {   /* no more threads: their pieces are taken below */
-  }
-  copier(0);
-  for (int t = (int)th.size() + 1; t < kCopiers; ++t) copier(t);
-  for (auto &x : th) x.join();
-  const hipError_t w = hipStreamSynchronize(L->stream);
-  return failed != (int)hipSuccess ? (hipError_t)failed.load() : w;
-}
-
 int ax_get_state(ax_lattice *L, double *host, size_t n) {
   if (!L || !host) return fail(AX_EINVAL, "NULL argument");
   const size_t want = (size_t)host_planes(L) * L->V;
   if (n != want) return fail(AX_EINVAL, "state length %zu != %zu", n, want);
-  std::vector<Run> runs;
+  Run runs[14];   /* Moore: seven components of two levels */
   const bool widen = L->esize == 4;
   for (int m = 0; m < host_planes(L); ++m)
-    runs.push_back({(const char *)L->state + (size_t)device_plane(L, m) * L->pitch * L->esize,
-                    (char *)(host + (size_t)m * L->V), widen ? L->V : L->V * 8, widen});
-  const hipError_t e = download(L, runs);
+    runs[m] = {(const char *)L->state + (size_t)device_plane(L, m) * L->pitch * L->esize,
+               (char *)(host + (size_t)m * L->V), widen ? L->V : L->V * 8, widen};
+  const hipError_t e = download(L->device, L->stream, L->stage, runs, host_planes(L));
   return e == hipSuccess ? AX_OK : hip_fail(e, "get_state");
 }
 
@@ -851,14 +755,14 @@ int ax_winding_field(ax_lattice *L, int32_t field, int8_t *out, size_t n) {
   Partials winds = {L->part + 3 * L->part_n, 0};
   if (!rc) rc = launch_winding_field(L, field, L->wind, winds);
   if (rc) return rc;
-  const std::vector<Run> map = {{(const char *)L->wind, (char *)out, n, false}};
+  const Run map = {(const char *)L->wind, (char *)out, n, false};
   const bool faces = L->p.boundary != AX_BC_PERIODIC || L->p.boundary_z != AX_BC_PERIODIC;
   hipError_t e = faces ? launch_sums(winds, L->hres + 4, {nullptr, 0}, nullptr, L->stream) : hipSuccess;
-  if (e == hipSuccess) e = download(L, map);
+  if (e == hipSuccess) e = download(L->device, L->stream, L->stage, &map, 1);
   if (e == hipSuccess && faces && std::isnan(L->hres[4])) {   /* as ax_diagnostics */
     rc = launch_site_winding(L, field, L->wind, winds);
     if (rc) return rc;
-    e = download(L, map);
+    e = download(L->device, L->stream, L->stage, &map, 1);
   }
   return e == hipSuccess ? AX_OK : hip_fail(e, "winding readback");
 }
@@ -914,7 +818,8 @@ int ax_crossings(ax_lattice *L, double *xyz, size_t cap, size_t *count) {
   *count = (size_t)tot;
   size_t nw = std::min(cap, (size_t)tot);
   if (nw) {
-    e = download(L, {{(const char *)L->cxyz, (char *)xyz, nw * 3 * sizeof(double), false}});
+    const Run points = {(const char *)L->cxyz, (char *)xyz, nw * 3 * sizeof(double), false};
+    e = download(L->device, L->stream, L->stage, &points, 1);
     if (e != hipSuccess) return hip_fail(e, "crossing readback");
   }
   return AX_OK;
