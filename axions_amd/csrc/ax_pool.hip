@@ -566,13 +566,12 @@ int ax_pool::enqueue_chunk() {
   if (count == 0) return AX_OK;
   /* two items per workgroup of the persistent grid (fill_segments) */
   if (work < 2 * grid_step) {
-    std::vector<int> nn(count), nw(count), xs(count);
+    std::vector<int> nn(count), xs(count);
     for (int k = 0; k < count; ++k) {
       nn[k] = ent[k].n;
-      nw[k] = (ent[k].n + 63) / 64;
       xs[k] = ent[k].xseg;
     }
-    fill_segments(count, nn.data(), nw.data(), xs.data(), 2LL * grid_step);
+    fill_segments(count, nn.data(), nullptr, xs.data(), 2LL * grid_step);
     work = 0;
     for (int k = 0; k < count; ++k) {
       BatchEntry &E = ent[k];

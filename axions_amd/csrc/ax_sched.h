@@ -122,16 +122,20 @@ inline double xi_of(double wxy, double wxz, double wyz, double sites, double dx,
 
 /* The chunk fill.  The tuned segments are chosen for a full pool; with few
  * lattices resident they leave workgroups of the persistent grid idle.  For
- * count lattices of edge n[k] with nw[k] z chunks of 64 and segments of
- * xseg[k] planes, halve the longest segments (never below floor planes)
- * until the chunk has at least want work items or every segment is at
- * floor; xseg is updated in place and the chunk's work items (nw n nseg
- * summed) returned.  The partition of a lattice does not change its
- * results. */
+ * count lattices of edge n[k] and segments of xseg[k] planes, halve the
+ * longest segments (never below floor planes) until the chunk has at least
+ * want work items or every segment is at floor; xseg is updated in place and
+ * the chunk's work items returned.  An item is a segment of a 64-site chunk of
+ * the plane, chunks crossing rows (nw null, the pool's marches), or of one of
+ * the nw[k] chunks of each row.  The partition of a lattice does not change
+ * its results. */
 inline long long fill_segments(int count, const int *n, const int *nw, int *xseg, long long want, int floor = 4) {
   auto items = [&]() {
     long long w = 0;
-    for (int k = 0; k < count; ++k) w += (long long)nw[k] * n[k] * ((n[k] + xseg[k] - 1) / xseg[k]);
+    for (int k = 0; k < count; ++k) {
+      const long long plane = nw ? (long long)nw[k] * n[k] : ((long long)n[k] * n[k] + 63) / 64;
+      w += plane * ((n[k] + xseg[k] - 1) / xseg[k]);
+    }
     return w;
   };
   long long work = items();
