@@ -11,8 +11,8 @@
  *                   counterpart) and their absolute sum.
  *  crossing kernels the bilinear face-crossing test of
  *                   mpi_evolution.cpp:536-789, in FP32 with an error bound
- *                   first, in FP64 where it is needed, compacted in site
- *                   order.
+ *                   first, in FP64 where it is needed (ax_cross.h),
+ *                   compacted in site order.
  *
  * The diagnostics must read the current level of every neighbour and the
  * previous level (the Gauss law needs the neighbours' previous level,
@@ -21,6 +21,7 @@
  */
 #include <algorithm>
 
+#include "ax_cross.h"
 #include "ax_energy.h"
 #include "ax_internal.h"
 #include "ax_march.h"
@@ -301,114 +302,6 @@ struct CrossGeom {
   double dx, dy, dz;
   float k;                          /* face_class's relative error bound; >= 1: solve every face in FP64 */
 };
-
-/* How many roots face_roots finds on the face with corners v.. of Re phi
- * and Im phi: 0, 1 or 2, or 3 if FP32 cannot tell.
- *
- * In coordinates p, q in [0, 1] of the face, phi_c = A + B p + C q + D p q;
- * the roots have a q^2 + b q + c = 0 and p = -(A0 + C0 q)/(B0 + D0 q), which
- * are face_roots' equations scaled and shifted.  With S the product of the
- * two largest |phi_c| of the corners, FP32 leaves a, b and c off by at most
- * about 2^-18 S.  face_roots works in lattice coordinates: with h the
- * largest coordinate in spacings and e = 2^-53, its rounding acts like errors
- * of up to some 2^8 e h^3 S in these coefficients.  The launcher takes k =
- * max(2^-16, 2^10 e h^3), above both; k S is followed through the
- * discriminant, q and p, and a value within its bound of a decision (or
- * not finite, or out of FP32's middle range) is left undecided, some 1e-4
- * of the faces.
- *
- * Re phi of one sign settles a face by itself: a point is kept only where
- * p = -(A0 + C0 q)/(B0 + D0 q) lies on it, that is where Re phi, a mean of
- * the corners there, vanishes within rounding. */
-__device__ __forceinline__ bool one_sign(float a, float b, float c, float d, float k) {
-  const float lo = fminf(fminf(a, b), fminf(c, d)), hi = fmaxf(fmaxf(a, b), fmaxf(c, d));
-  return (lo > 1e-6f && lo > k * hi && hi < 1e6f) || (hi < -1e-6f && hi < k * lo && lo > -1e6f);
-}
-__device__ __forceinline__ int face_class(float r00, float r10, float r01, float r11, float i00, float i10, float i01,
-                                          float i11, float k) {
-  const float m0 = fmaxf(fmaxf(fabsf(r00), fabsf(r10)), fmaxf(fabsf(r01), fabsf(r11)));
-  const float m1 = fmaxf(fmaxf(fabsf(i00), fabsf(i10)), fmaxf(fabsf(i01), fabsf(i11)));
-  const float B0 = r10 - r00, C0 = r01 - r00, D0 = (r11 - r10) - C0;
-  const float B1 = i10 - i00, C1 = i01 - i00, D1 = (i11 - i10) - C1;
-  const float a = D1 * C0 - D0 * C1;
-  const float b = (D1 * r00 - D0 * i00) + (B1 * C0 - B0 * C1);
-  const float c = B1 * r00 - B0 * i00;
-  const float E = k * (m0 * m1);
-  const float disc = b * b - 4 * (a * c);
-  const float F = E * (4 * fabsf(b) + 8 * (fabsf(a) + fabsf(c)) + 16 * E);
-  /* not finite makes disc + F NaN or infinite and the tests below fail */
-  const bool sane = m0 > 1e-6f && m1 > 1e-6f && m0 < 1e6f && m1 < 1e6f && fabsf(disc) < 1e30f && k < 1;
-  if (sane && disc < -F) return 0;
-  if (!(sane && disc > 2 * F && fabsf(a) > 16 * E)) return 3;
-  const float root = __builtin_amdgcn_sqrtf(disc), inv = __builtin_amdgcn_rcpf(2 * a);
-  const float eq = (3 * E + F * __builtin_amdgcn_rcpf(root)) * fabsf(2 * inv) * 1.01f + 1e-5f;
-  const float en = m0 * (2 * k + 2 * eq), ed = 2 * en;
-  int n = 0;
-  bool sure = true;
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    const float q = ((s ? -root : root) - b) * inv;
-    const float num = -(r00 + C0 * q), den = B0 + D0 * q;
-    const float t0 = den < 0 ? -num : num, t1 = fabsf(den) - t0;
-    const bool in = q > eq && q < 1 - eq && t0 > en && t1 > en + ed;
-    const bool out = q < -eq || q > 1 + eq || (fabsf(den) > ed && (t0 < -en || t1 < -(en + ed)));
-    n += in ? 1 : 0;
-    sure = sure && (in || out);
-  }
-  return sure ? n : 3;
-}
-
-/* Solve the face of mpi_evolution.cpp:552-623: its roots inside the face
- * (0..2), the + root before the - root. */
-__device__ __forceinline__ int face_roots(const double v00[2], const double v10[2], const double v01[2],
-                                          const double v11[2], double u, double du, double w, double dw,
-                                          double &r1, double &r2, double &q1, double &q2) {
-  double c1[2], c2[2], c3[2], c4[2];
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    c1[c] = v11[c] - v10[c] - v01[c] + v00[c];
-    c2[c] = (w + dw) * (v10[c] - v00[c]) + w * (v01[c] - v11[c]);
-    c3[c] = (u + du) * (v01[c] - v00[c]) + u * (v10[c] - v11[c]);
-    c4[c] = (u + du) * ((w + dw) * v00[c] - w * v01[c]) - u * ((w + dw) * v10[c] - w * v11[c]);
-  }
-  const double a = c1[1] * c3[0] - c1[0] * c3[1];
-  const double b = c1[1] * c4[0] + c2[1] * c3[0] - c1[0] * c4[1] - c2[0] * c3[1];
-  const double c = c2[1] * c4[0] - c2[0] * c4[1];
-  const double disc = b * b - 4 * a * c;
-  auto inside = [&](double s2, double &s1) {
-    s1 = 0;
-    if (!(s2 >= w && s2 <= w + dw)) return false;
-    s1 = -(c3[0] * s2 + c4[0]) / (c1[0] * s2 + c2[0]);
-    return s1 >= u && s1 <= u + du;
-  };
-  int n = 0;
-  if (a == 0) {
-    if (b != 0) {
-      r2 = -c / b;
-      n = inside(r2, r1) ? 1 : 0;
-    }
-  } else if (disc >= 0) {
-    const double root = sqrt(disc);
-    double s1, s2 = (-b + root) / (2 * a);
-    if (inside(s2, s1)) {
-      r1 = s1;
-      r2 = s2;
-      n = 1;
-    }
-    s2 = (-b - root) / (2 * a);
-    if (inside(s2, s1)) {
-      if (n) {
-        q1 = s1;
-        q2 = s2;
-      } else {
-        r1 = s1;
-        r2 = s2;
-      }
-      ++n;
-    }
-  }
-  return n;
-}
 
 /* WRITE: the points of each group from its offset on; else its count.
  * masks: three words per 64 sites, the lanes whose xy, xz, yz face is not
@@ -997,11 +890,7 @@ hipError_t launch_crossings(int nx, int ny, int nz, double dx, double dy, double
   g.by_nz = fast_div((uint32_t)nz);
   g.by_ny = fast_div((uint32_t)ny);
   g.dx = dx; g.dy = dy; g.dz = dz;
-  /* face_class's bound, h = n/2 + 2 spacings; where it would decide little,
-   * every face is solved */
-  const double h = 0.5 * std::max(nx, std::max(ny, nz)) + 2;
-  const double k = std::max(0x1p-16, 0x1p-43 * h * h * h);
-  g.k = k < 0x1p-8 ? (float)k : 2.0f;
+  g.k = cross_bound(nx, ny, nz, dx, dy, dz);
   const dim3 grid(8 * g.per), block(64);
 #define AX_CROSS(W, M) \
   hipLaunchKernelGGL((cross_kernel<T, W, M>), grid, block, 0, st, g, fr, fi, bcount, boff, xyz, cap, masks)

@@ -1,0 +1,54 @@
+"""The crossings' face classification on the CPU (axions_amd/csrc/ax_cross.h):
+a face that FP32 settles has the number of roots that the FP64 equations find,
+which is what puts every later point at its place.  Random phases, smooth
+fields, scales apart, zeros on edges, close pairs, one sign of Re phi and nearly
+linear equations, on lattices from 3 to 1283 sites an edge, with the device's
+square root and reciprocal off by up to one unit in the last place."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+KINDS = ["random phases", "scales", "smooth", "edges", "pairs", "one sign", "linear"]
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("ax_cross") / "libcross.so")
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-ffp-contract=off", "-o", so,
+                           os.path.join(HERE, "csrc", "cross_harness.cpp")])
+    L = ctypes.CDLL(so)
+    L.check_faces.argtypes = [ctypes.c_int, ctypes.c_longlong, ctypes.c_uint] + [ctypes.c_int] * 3 + [
+        ctypes.c_double, ctypes.c_int, ctypes.c_float, ctypes.POINTER(ctypes.c_longlong)]
+    L.cross_bound.restype = ctypes.c_float
+    L.cross_bound.argtypes = [ctypes.c_int] * 3 + [ctypes.c_double] * 3
+    return L
+
+
+def check(lib, kind, n, seed, shape, d, fp32=0, k=0.0):
+    out = (ctypes.c_longlong * 3)()
+    lib.check_faces(kind, n, seed, *shape, d, fp32, k, out)
+    return [v / n for v in out]
+
+
+@pytest.mark.parametrize("kind", range(len(KINDS)), ids=KINDS)
+@pytest.mark.parametrize("shape,d", [((3, 3, 3), 0.5), ((101, 90, 64), 0.7), ((512, 512, 512), 0.5),
+                                     ((1001, 64, 1283), 0.25)])
+def test_settled_faces_have_their_roots(lib, kind, shape, d):
+    for fp32 in (0, 1):
+        assert check(lib, kind, 200000, 7 + kind, shape, d, fp32)[1] == 0, (KINDS[kind], shape, fp32)
+
+
+def test_spacings_whose_products_leave_the_range(lib):
+    """(spacing)^4 underflows or overflows in the FP64 equations: nothing is
+    settled in FP32 then, whose own coordinates know no spacing."""
+    for d in (1e-90, 1e90):
+        assert lib.cross_bound(64, 64, 64, 0.5, d, 0.5) == 2.0
+        undecided, wrong, signed = check(lib, 0, 20000, 3, (64, 64, 64), d)
+        assert undecided == 1 and wrong == 0 and signed == 0
+    # with an ordinary lattice's bound they would be settled wrongly
+    assert check(lib, 0, 20000, 3, (64, 64, 64), 1e-90, k=lib.cross_bound(64, 64, 64, 0.5, 0.5, 0.5))[1] > 0.1
+    assert lib.cross_bound(512, 512, 512, 0.5, 0.25, 0.7) == 2.0 ** -16
+    assert lib.cross_bound(64, 64, 1 << 20, 0.5, 0.5, 0.5) == 2.0
