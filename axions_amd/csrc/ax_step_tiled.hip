@@ -9,6 +9,7 @@
  * (ax_internal.h): each XCD takes bands of consecutive rows with all their
  * chunks, so y-neighbour rows and chunk-edge lines are read from its own L2.
  */
+#include <algorithm>
 #include <cstdlib>
 #include <limits>
 
@@ -113,10 +114,10 @@ template hipError_t launch_step_tiled_moore<double>(const StepConsts &, const Le
 template hipError_t launch_step_tiled_moore<float>(const StepConsts &, const Levels<float> &, int, hipStream_t, int *,
                                                    int, bool, bool *);
 
-/* Every Abelian-Higgs and Moore lattice marches, whatever its z tail (a
- * last chunk of 1..63 sites runs with its other lanes idle) and whatever
- * its plane size (planes of 4 GiB or more take the 64-bit plane addressing
- * of ah_march and moore_march). */
+/* Every Abelian-Higgs and Moore lattice marches, whatever its plane (chunks
+ * cross rows, and the last of a plane may run with lanes idle) and whatever
+ * its size (planes of 4 GiB or more take the 64-bit plane addressing of
+ * ah_march and moore_march). */
 bool use_tiled_ah(const ax_params &p) {
   return (p.model == AX_MODEL_AH || p.model == AX_MODEL_MOORE) && p.nx >= 3 && p.ny >= 3 &&
          getenv("AX_FORCE_SITE_KERNEL") == nullptr;
@@ -126,21 +127,25 @@ bool use_tiled_ah(const ax_params &p) {
  * large lattices (measured at 512^3 AH, 256^3 Moore, on one box each):
  * Abelian-Higgs FP64 32 (3.607 ms; 8: 3.746, 16: 3.644, 24: 3.631, 48: 3.603;
  * 256^3 32: 0.459, 16: 0.468), FP32 16 (1.737 ms; 8: 1.762, 12: 1.758, 32:
- * 1.756); Moore FP64 16
- * (0.800 ms; 8: 0.807, 9: 0.808, 10 and 12: 0.800), FP32 8 (0.422 ms; 32:
- * 0.444).  Moore's prologue is cheap against a plane, so below that it takes
- * half the rule's length (rule / half, us: FP64 201x201x51 fixed 141.6 / 133.8,
- * 100^3 fixed 70.1 / 65.4, 150^3 fixed 203 / 197, periodic 181 / 179, 200^3
- * fixed 464 / 452, 128^3 110.5 / 108.1; FP32 128^3 65 / 60, 160^3 135 / 118),
- * in FP64 from 3 planes on (64^3 2: 19.2, 1: 21.0). */
+ * 1.756); Moore FP32 8 (0.422 ms; 32: 0.444).  Moore's prologue is cheap
+ * against a plane, so it takes half the rule's length (rule / half, us: FP64
+ * 201x201x51 fixed 141.6 / 133.8, 100^3 fixed 70.1 / 65.4, 150^3 fixed 203 /
+ * 197, periodic 181 / 179, 200^3 fixed 464 / 452, 128^3 110.5 / 108.1; FP32
+ * 128^3 65 / 60, 160^3 135 / 118), in FP64 from 3 planes on (64^3 2: 19.2, 1:
+ * 21.0).  On whole chunks in FP64 longer segments catch up from about 10
+ * planes on, so it is the rule's length less 4 there, up to 12 (periodic, half
+ * / this / 16 planes: 192^3 356 / 354 / 364, 128x300x192 366 / 365 / 388, 256^3
+ * 814 / 804 / 804); across rows half is best or within 1 % (250^3 814, 11
+ * planes 826, 16 823; 260^3 889, 882, 881; 300^3 1344, 1354, 1351; fixed 250^3
+ * 889, 896, 897; 300^3 1464, 1459, 1469). */
 int default_xseg(const ax_params &p) {
   const char *xe = getenv("AX_TILED_XSEG");
   if (xe) return atoi(xe);
   const bool f32 = p.precision == 32;
   if (p.model != AX_MODEL_MOORE) return tile_xseg(p.nx, p.ny, p.nz, f32 ? 16 : 32);
-  const int xs = tile_xseg(p.nx, p.ny, p.nz, 16);
-  const bool at_cap = (long long)tile_chunks(p.ny, p.nz) * p.nx >= 240 * 1024;   /* the rule's length 15.5 or more */
-  return f32 || (xs > 2 && !at_cap) ? (xs + 1) / 2 : xs;
+  const int xs = tile_xseg(p.nx, p.ny, p.nz, 16), half = (xs + 1) / 2;
+  if (f32) return half;
+  return xs <= 2 ? xs : p.nz % 64 == 0 ? std::max(half, xs - 4) : half;
 }
 
 /* The LDS prefetch of the FP64 march applies: whole 64-site chunks (across
