@@ -40,9 +40,20 @@ def test_partial_buffers_hold_either_order(shape, model, monkeypatch):
             assert items(nx, ny, nz, xs) <= room, (shape, made, launched)
 
 
+@pytest.mark.parametrize("shape", [(4000, 3, 3), (1000, 10, 10), (200, 20, 20), (400, 30, 30)])
+def test_narrow_planes_have_no_empty_workgroups(shape, monkeypatch):
+    """Planes of a few chunks: as many workgroups as chunks and segments, not
+    eight XCD shares of which most are empty."""
+    order(monkeypatch, "")
+    nx, ny, nz = shape
+    chunks = -(-ny * nz // 64)
+    for xs in (1, 4, 32):
+        assert lib._ZN2ax16fused_work_itemsEiiii(nx, ny, nz, xs) == chunks * -(-nx // xs)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("precision", [64, 32])
-@pytest.mark.parametrize("shape", SHAPES[:4])
+@pytest.mark.parametrize("shape", SHAPES[:4] + [(300, 3, 3), (100, 10, 10)])
 def test_orders_of_creation_and_launch_may_differ(shape, precision, monkeypatch):
     """State, windings and sums: the same whichever order a lattice was
     created and whichever it is stepped and diagnosed in."""
