@@ -39,35 +39,47 @@
 
 namespace ax {
 
+/* What a kernel needs of the lattice, and no more: a small lattice's steps are
+ * as fast as the host can launch them, and every argument byte goes over the
+ * bus (Neumann faces, two launches a step, us: 16^3 FP32 7.4 with all of the
+ * lattice's constants for each kernel, 6.5 with its own). */
 struct GlobalGeom {
   int nx, ny, nz;
   int periodic;          /* 1: all sites updated, periodic wrap; 0: Neumann x/y faces */
-  double dx, dy, dz, dt;
-  uint32_t V, per, eper;   /* sites; blocks of the step and of the energy per XCD */
-  uint32_t eruns;          /* runs of 256 threads' sites a block of the energy takes */
-  bool wide;               /* two sites a thread */
+  uint32_t V, per;       /* sites; blocks per XCD */
   FastDiv by_nz, by_ny;
 };
 
+/* dx^2, dy^2, dz^2 or, with POW2, their reciprocals */
 template <typename R>
-struct GlobalConsts {
-  R dx2, dy2, dz2, ix2, iy2, iz2;   /* dx*dx ... and their reciprocals */
-  R tx, ty, tz, itx, ity, itz;      /* 2 dx ... */
-  R dt;
+struct GlobalLap {
+  R x, y, z;
+};
+
+template <typename R>
+struct GlobalEnergy {
+  R tx, ty, tz;          /* 2 dx ..., with POW2 their reciprocals */
+  double dt, vol;        /* vol = dx dy dz */
+  uint32_t runs;         /* of 256 threads' sites a block takes */
 };
 
 template <typename R, bool POW2>
-__device__ __forceinline__ R glap(const GlobalConsts<R> &k, R f, R xp, R xm, R yp, R ym, R zp, R zm, R mag) {
-  R xx = mdiv<R, POW2>(xp - 2 * f + xm, k.dx2, k.ix2);
-  R yy = mdiv<R, POW2>(yp - 2 * f + ym, k.dy2, k.iy2);
-  R zz = mdiv<R, POW2>(zp - 2 * f + zm, k.dz2, k.iz2);
+__device__ __forceinline__ R gdiv(R a, R d) {
+  return mdiv<R, POW2>(a, d, d);
+}
+
+template <typename R, bool POW2>
+__device__ __forceinline__ R glap(const GlobalLap<R> &k, R f, R xp, R xm, R yp, R ym, R zp, R zm, R mag) {
+  R xx = gdiv<R, POW2>(xp - 2 * f + xm, k.x);
+  R yy = gdiv<R, POW2>(yp - 2 * f + ym, k.y);
+  R zz = gdiv<R, POW2>(zp - 2 * f + zm, k.z);
   return xx + yy + zz - (mag - 1) * f;
 }
 
 template <typename R>
-__global__ void __launch_bounds__(256) global_bc_kernel(GlobalGeom g, R *pr, R *pi, R *qr, R *qi) {
+__global__ void __launch_bounds__(256) global_bc_kernel(int nx, int ny, int nz, R *pr, R *pi, R *qr,
+                                                        R *qi) {
   /* boundary sites: the two x faces (all j), then the two y faces at interior x */
-  const int nz = g.nz, ny = g.ny, nx = g.nx;
   const int nxf = 2 * ny * nz, nyf = 2 * (nx - 2) * nz;
   const int t = blockIdx.x * 256 + threadIdx.x;
   if (t >= nxf + nyf) return;
@@ -176,7 +188,7 @@ struct GlobalSite {
 };
 
 template <typename R, bool POW2, int W>
-__global__ void __launch_bounds__(256) global_step_kernel(GlobalGeom g, GlobalConsts<R> c, const R *__restrict__ ar,
+__global__ void __launch_bounds__(256) global_step_kernel(GlobalGeom g, GlobalLap<R> c, R dt, const R *__restrict__ ar,
                                                           const R *__restrict__ ai, R *__restrict__ br,
                                                           R *__restrict__ bi, R *__restrict__ mr, R *__restrict__ mi) {
   typedef Sites<R, W> S;
@@ -201,8 +213,8 @@ __global__ void __launch_bounds__(256) global_step_kernel(GlobalGeom g, GlobalCo
     for (int e = 0; e < W; ++e) {
       const R mag = here[0].v[e] * here[0].v[e] + here[1].v[e] * here[1].v[e];
       const R t = glap<R, POW2>(c, here[v].v[e], xp[v].v[e], xm[v].v[e], yp[v].v[e], ym[v].v[e], zp.v[e], zm.v[e], mag);
-      p.v[e] = mom[v].v[e] + t * c.dt;
-      o.v[e] = here[v].v[e] + p.v[e] * c.dt;
+      p.v[e] = mom[v].v[e] + t * dt;
+      o.v[e] = here[v].v[e] + p.v[e] * dt;
     }
     if (q.on) {
       p.store(m[v], q.s);
@@ -212,7 +224,7 @@ __global__ void __launch_bounds__(256) global_step_kernel(GlobalGeom g, GlobalCo
 }
 
 /* o: the pre-step field, n: the step's result, m: its momentum.  A block
- * takes g.eruns consecutive runs of 256 threads' sites: four, which leaves a
+ * takes w.runs consecutive runs of 256 threads' sites: four, which leaves a
  * fourth of the partial sums, while the chip still gets four blocks a CU, and
  * fewer on small lattices, where one run after another is what the call waits
  * for (us per ax_diagnostics, FP64, periodic, dx 0.7, four runs / this rule:
@@ -221,18 +233,19 @@ __global__ void __launch_bounds__(256) global_step_kernel(GlobalGeom g, GlobalCo
  * 24.2). */
 constexpr uint32_t kEnergyRuns = 4;
 template <typename R, bool POW2, int W>
-__global__ void __launch_bounds__(256) global_energy_kernel(GlobalGeom g, GlobalConsts<R> c, const R *__restrict__ ar,
-                                                            const R *__restrict__ ai, const R *__restrict__ br,
-                                                            const R *__restrict__ bi, const R *__restrict__ mr,
-                                                            const R *__restrict__ mi, double *__restrict__ part) {
+__global__ void __launch_bounds__(256) global_energy_kernel(GlobalGeom g, GlobalLap<R> c, GlobalEnergy<R> w,
+                                                            const R *__restrict__ ar, const R *__restrict__ ai,
+                                                            const R *__restrict__ br, const R *__restrict__ bi,
+                                                            const R *__restrict__ mr, const R *__restrict__ mi,
+                                                            double *__restrict__ part) {
   typedef Sites<R, W> S;
   __shared__ double sh[2][4];
   double rho = 0, bad = 0;
-  const uint32_t blk = (blockIdx.x & 7) * g.eper + (blockIdx.x >> 3);
+  const uint32_t blk = (blockIdx.x & 7) * g.per + (blockIdx.x >> 3);
   const R *o[2] = {ar, ai}, *n[2] = {br, bi}, *m[2] = {mr, mi};
 #pragma unroll 1
-  for (uint32_t run = 0; run < g.eruns; ++run) {
-    const GlobalSite<W> q(g, blk * g.eruns + run);
+  for (uint32_t run = 0; run < w.runs; ++run) {
+    const GlobalSite<W> q(g, blk * w.runs + run);
     /* a neighbour holds its new value when it is an updated site earlier in
      * loop order (x, then y, then z): x - 1 and y - 1 unless they wrap or are
      * faces, z - 1 unless it wraps; x + 1, y + 1, z + 1 only where they wrap */
@@ -261,22 +274,22 @@ __global__ void __launch_bounds__(256) global_energy_kernel(GlobalGeom g, Global
       for (int e = 0; e < W; ++e) {
         const R mag = here[0].v[e] * here[0].v[e] + here[1].v[e] * here[1].v[e];
         t[v][e] = glap<R, POW2>(c, here[v].v[e], xp.v[e], xm.v[e], yp.v[e], ym.v[e], zp.v[e], zm.v[e], mag);
-        gx[v][e] = mdiv<R, POW2>(xps.v[e] - xms.v[e], c.tx, c.itx);
-        gy[v][e] = mdiv<R, POW2>(yps.v[e] - yms.v[e], c.ty, c.ity);
-        gz[v][e] = mdiv<R, POW2>(zps.v[e] - zms.v[e], c.tz, c.itz);
+        gx[v][e] = gdiv<R, POW2>(xps.v[e] - xms.v[e], w.tx);
+        gy[v][e] = gdiv<R, POW2>(yps.v[e] - yms.v[e], w.ty);
+        gz[v][e] = gdiv<R, POW2>(zps.v[e] - zms.v[e], w.tz);
       }
     }
 #pragma unroll
     for (int e = 0; e < W; ++e) {
       const R mag = here[0].v[e] * here[0].v[e] + here[1].v[e] * here[1].v[e];
-      const double r0 = (double)mom[0].v[e] - 0.5 * (double)t[0][e] * g.dt;
-      const double r1 = (double)mom[1].v[e] - 0.5 * (double)t[1][e] * g.dt;
+      const double r0 = (double)mom[0].v[e] - 0.5 * (double)t[0][e] * w.dt;
+      const double r1 = (double)mom[1].v[e] - 0.5 * (double)t[1][e] * w.dt;
       const double dm = (double)mag - 1;
       const double gx0 = gx[0][e], gx1 = gx[1][e], gy0 = gy[0][e], gy1 = gy[1][e], gz0 = gz[0][e], gz1 = gz[1][e];
       const double r = r0 * r0 + r1 * r1 + gx0 * gx0 + gx1 * gx1 + gy0 * gy0 + gy1 * gy1 + gz0 * gz0 + gz1 * gz1 +
                        0.5 * (dm * dm);
       if (q.on) {
-        rho += g.dx * g.dy * g.dz * r;
+        rho += w.vol * r;
         bad += (isfinite((double)now[0].v[e]) && isfinite((double)now[1].v[e]) && isfinite((double)mom[0].v[e]) &&
                 isfinite((double)mom[1].v[e])) ? 0.0 : 1.0;
       }
@@ -285,10 +298,10 @@ __global__ void __launch_bounds__(256) global_energy_kernel(GlobalGeom g, Global
   /* fixed-order block sums */
   rho = march_wave_sum(rho);
   bad = march_wave_sum(bad);
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
   if (l == 0) {
-    sh[0][w] = rho;
-    sh[1][w] = bad;
+    sh[0][wv] = rho;
+    sh[1][wv] = bad;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -298,43 +311,43 @@ __global__ void __launch_bounds__(256) global_energy_kernel(GlobalGeom g, Global
   }
 }
 
-/* pitch: of the planes, whose two-site loads need it even as well */
-static GlobalGeom geom_of(const ax_params &p, size_t pitch) {
+/* How a lattice's kernels are launched. */
+struct GlobalPlan {
   GlobalGeom g;
+  bool wide;             /* two sites a thread */
+  uint32_t eper, eruns;  /* blocks of the energy per XCD, runs of one */
+};
+/* pitch: of the planes, whose two-site loads need it even as well */
+static GlobalPlan plan_of(const ax_params &p, size_t pitch) {
+  GlobalPlan q;
+  GlobalGeom &g = q.g;
   g.nx = p.nx; g.ny = p.ny; g.nz = p.nz;
   g.periodic = p.boundary == AX_BC_PERIODIC;
-  g.dx = p.dx; g.dy = p.dy; g.dz = p.dz; g.dt = p.dt;
   g.V = (uint32_t)p.nx * p.ny * p.nz;
-  g.wide = p.nz % 2 == 0 && pitch % 2 == 0;
-  const uint32_t runs = (g.V + 255) / 256 / (g.wide ? 2 : 1) + 1;   /* of 256 threads */
+  q.wide = p.nz % 2 == 0 && pitch % 2 == 0;
+  const uint32_t runs = (g.V + 255) / 256 / (q.wide ? 2 : 1) + 1;   /* of 256 threads */
   g.per = (runs + 7) / 8;
-  g.eruns = std::min(kEnergyRuns, (runs + 1023) / 1024);
-  g.eper = ((runs + g.eruns - 1) / g.eruns + 7) / 8;
+  q.eruns = std::min(kEnergyRuns, (runs + 1023) / 1024);
+  q.eper = ((runs + q.eruns - 1) / q.eruns + 7) / 8;
   g.by_nz = fast_div((uint32_t)p.nz);
   g.by_ny = fast_div((uint32_t)p.ny);
-  return g;
+  return q;
 }
 
-size_t global_energy_blocks(const ax_params &p) { return (size_t)8 * std::max(geom_of(p, 0).eper, geom_of(p, 1).eper); }
+size_t global_energy_blocks(const ax_params &p) { return (size_t)8 * std::max(plan_of(p, 0).eper, plan_of(p, 1).eper); }
 
+/* dx^2 ... and 2 dx ...; true when every one is a power of two with a normal
+ * reciprocal, and then the reciprocals */
 template <typename R>
-static GlobalConsts<R> consts_of(const ax_params &p) {
-  GlobalConsts<R> k;
-  k.dx2 = (R)(p.dx * p.dx); k.dy2 = (R)(p.dy * p.dy); k.dz2 = (R)(p.dz * p.dz);
-  k.tx = 2 * (R)p.dx; k.ty = 2 * (R)p.dy; k.tz = 2 * (R)p.dz;
-  k.ix2 = 1 / k.dx2; k.iy2 = 1 / k.dy2; k.iz2 = 1 / k.dz2;
-  k.itx = 1 / k.tx; k.ity = 1 / k.ty; k.itz = 1 / k.tz;
-  k.dt = (R)p.dt;
-  return k;
-}
-
-/* every divisor a power of two with a normal reciprocal */
-template <typename R>
-static bool pow2_of(const GlobalConsts<R> &k) {
-  const R d[6] = {k.dx2, k.dy2, k.dz2, k.tx, k.ty, k.tz};
-  for (R v : d)
-    if (!is_pow2(v) || !std::isnormal(v) || !std::isnormal(1 / v)) return false;
-  return true;
+static bool consts_of(const ax_params &p, GlobalLap<R> &l, R t[3]) {
+  R d[6] = {(R)(p.dx * p.dx), (R)(p.dy * p.dy), (R)(p.dz * p.dz), 2 * (R)p.dx, 2 * (R)p.dy, 2 * (R)p.dz};
+  bool p2 = true;
+  for (R v : d) p2 = p2 && is_pow2(v) && std::isnormal(v) && std::isnormal(1 / v);
+  if (p2)
+    for (R &v : d) v = 1 / v;
+  l = {d[0], d[1], d[2]};
+  for (int a = 0; a < 3; ++a) t[a] = d[3 + a];
+  return p2;
 }
 
 template <typename R>
@@ -344,19 +357,20 @@ hipError_t launch_global_step(const ax_params &p, void *state, size_t pitch, int
   R *ar = b + (size_t)(0 + cur) * pitch, *ai = b + (size_t)(2 + cur) * pitch;
   R *br = b + (size_t)(0 + nw) * pitch, *bi = b + (size_t)(2 + nw) * pitch;
   R *mr = b + 4 * pitch, *mi = b + 5 * pitch;
-  const GlobalGeom g = geom_of(p, pitch);
-  if (!g.periodic) {
+  const GlobalPlan q = plan_of(p, pitch);
+  if (!q.g.periodic) {
     const int nbs = 2 * p.ny * p.nz + 2 * (p.nx - 2) * p.nz;
-    hipLaunchKernelGGL((global_bc_kernel<R>), dim3((nbs + 255) / 256), dim3(256), 0, st, g, ar, ai, br, bi);
+    hipLaunchKernelGGL((global_bc_kernel<R>), dim3((nbs + 255) / 256), dim3(256), 0, st, p.nx, p.ny, p.nz, ar, ai, br, bi);
   }
-  const GlobalConsts<R> k = consts_of<R>(p);
-  const dim3 grid(8 * g.per), block(256);
+  GlobalLap<R> l;
+  R t[3];
+  const bool p2 = consts_of<R>(p, l, t);
+  const dim3 grid(8 * q.g.per), block(256);
 #define AX_GS(P2, W) \
-  hipLaunchKernelGGL((global_step_kernel<R, P2, W>), grid, block, 0, st, g, k, ar, ai, br, bi, mr, mi)
-  const bool p2 = pow2_of(k);
-  if (p2 && g.wide) AX_GS(true, 2);
+  hipLaunchKernelGGL((global_step_kernel<R, P2, W>), grid, block, 0, st, q.g, l, (R)p.dt, ar, ai, br, bi, mr, mi)
+  if (p2 && q.wide) AX_GS(true, 2);
   else if (p2) AX_GS(true, 1);
-  else if (g.wide) AX_GS(false, 2);
+  else if (q.wide) AX_GS(false, 2);
   else AX_GS(false, 1);
 #undef AX_GS
   return hipGetLastError();
@@ -367,20 +381,23 @@ hipError_t launch_global_energy(const ax_params &p, const void *state, size_t pi
                                 hipStream_t st) {
   const R *b = (const R *)state;
   const int cur = n % 2, nw = 1 - cur;   /* the pre-step field of TimeStep n and its result */
-  const GlobalGeom g = geom_of(p, pitch);
-  const GlobalConsts<R> k = consts_of<R>(p);
-  const dim3 grid(8 * g.eper), block(256);   /* part holds 3 doubles each (diag_part_blocks) */
-#define AX_GE(P2, W)                                                                                              \
-  hipLaunchKernelGGL((global_energy_kernel<R, P2, W>), grid, block, 0, st, g, k, b + (size_t)cur * pitch,          \
+  GlobalPlan q = plan_of(p, pitch);
+  q.g.per = q.eper;
+  GlobalLap<R> l;
+  R t[3];
+  const bool p2 = consts_of<R>(p, l, t);
+  const GlobalEnergy<R> w = {t[0], t[1], t[2], p.dt, p.dx * p.dy * p.dz, q.eruns};
+  const dim3 grid(8 * q.eper), block(256);   /* part holds 3 doubles each (diag_part_blocks) */
+#define AX_GE(P2, W)                                                                                               \
+  hipLaunchKernelGGL((global_energy_kernel<R, P2, W>), grid, block, 0, st, q.g, l, w, b + (size_t)cur * pitch,      \
                      b + (size_t)(2 + cur) * pitch, b + (size_t)nw * pitch, b + (size_t)(2 + nw) * pitch, b + 4 * pitch, \
                      b + 5 * pitch, part.p)
-  const bool p2 = pow2_of(k);
-  if (p2 && g.wide) AX_GE(true, 2);
+  if (p2 && q.wide) AX_GE(true, 2);
   else if (p2) AX_GE(true, 1);
-  else if (g.wide) AX_GE(false, 2);
+  else if (q.wide) AX_GE(false, 2);
   else AX_GE(false, 1);
 #undef AX_GE
-  part.n = (int)(8 * g.eper);
+  part.n = (int)(8 * q.eper);
   return hipGetLastError();
 }
 
