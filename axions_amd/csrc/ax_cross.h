@@ -17,7 +17,10 @@
 namespace ax {
 
 /* How many roots face_roots finds on the face with corners v.. of Re phi
- * and Im phi: 0, 1 or 2, or 3 if FP32 cannot tell.
+ * and Im phi: 0, 1 or 2, or 3 if FP32 cannot tell, or 4: none if the corners
+ * of Re phi or of Im phi, zero in FP32, are zero, else 3.  (With four zeros
+ * every coefficient is 0 or not a number, and with a NaN a and disc are NaN:
+ * face_roots finds no root.)
  *
  * In coordinates p, q in [0, 1] of the face, phi_c = A + B p + C q + D p q;
  * the roots have a q^2 + b q + c = 0 with a = D1 C0 - D0 C1, b = D1 A0 - D0 A1
@@ -69,7 +72,12 @@ __device__ __forceinline__ int face_class(float r00, float r10, float r01, float
   /* not finite makes disc + F NaN or infinite and the tests below fail */
   const bool sane = m0 > 1e-6f && m1 > 1e-6f && m0 < 1e6f && m1 < 1e6f && fabsf(disc) < 1e30f && k < 1;
   if (sane && disc < -F) return 0;
-  if (!(sane && disc > 2 * F && fabsf(a) > 16 * E)) return 3;
+  if (!(sane && disc > 2 * F && fabsf(a) > 16 * E)) {
+    if (sane) return 3;
+    const bool nan = __builtin_isunordered(r00, r10) || __builtin_isunordered(r01, r11) ||
+                     __builtin_isunordered(i00, i10) || __builtin_isunordered(i01, i11);
+    return nan ? 0 : m0 == 0 || m1 == 0 ? 4 : 3;
+  }
   const float root = __builtin_amdgcn_sqrtf(disc), inv = __builtin_amdgcn_rcpf(2 * a);
   const float eq = (3 * E + F * __builtin_amdgcn_rcpf(root)) * fabsf(2 * inv) * 1.01f + 1e-5f;
   const float en = m0 * (2 * k + 2 * eq), ed = 2 * en;

@@ -293,7 +293,10 @@ __global__ void __launch_bounds__(256) winding_kernel(int nx, int ny, int nz, co
  * 2.67 -> 1.56 ms, scan 0.92 -> 0.15, points 6.96 -> 2.94 (3.9 GB written);
  * FP32 2.63 -> 1.45, 0.92 -> 0.15, 6.29 -> 2.72; with the faces handed on as
  * masks the whole call 4.65 -> 3.88, FP32 4.15 -> 3.27 (301^3 FP64 0.98 ->
- * 0.81, 101^3 78 -> 69 us).  Bound by instructions. */
+ * 0.81, 101^3 78 -> 69 us).  Faces of zeros and NaNs, which the equations leave
+ * at once, are not queued either (a field of zeros, 128^3 FP64: 114 us a call
+ * when they were, 53 now, 57 for the equations alone); that check costs other
+ * fields 1 to 2 %.  Bound by instructions. */
 
 struct CrossGeom {
   int nx, ny, nz, ex, ez, x0, y0, z0;
@@ -370,6 +373,19 @@ __global__ void __launch_bounds__(64) cross_kernel(CrossGeom g, const T *__restr
     head += n;
   };
 
+  /* Re phi or Im phi zero on the corners of a face of site s.  (s opaque: its
+   * addresses are formed again rather than held in registers for this.) */
+  auto zero_face = [&](uint32_t s, int f) {
+    asm("" : "+v"(s));
+    const uint32_t r = quotient(s, g.by_nz), i = quotient(r, g.by_ny);
+    const int k = (int)(s - r * nz), j = (int)(r - i * ny);
+    const int ia = f == 2 ? (int)i : wrapp((int)i, nx), ja = f == 2 ? wrapp(j, ny) : j;
+    const int jb = f == 0 ? wrapp(j, ny) : j, kb = f == 0 ? k : wrapp(k, nz);
+    const uint32_t at[4] = {s, id(ia, ja, k), id((int)i, jb, kb), id(ia, f == 1 ? j : wrapp(j, ny), kb)};
+    auto zero = [&](const T *p) { return p[at[0]] == 0 && p[at[1]] == 0 && p[at[2]] == 0 && p[at[3]] == 0; };
+    return zero(fr) || zero(fi);
+  };
+
   for (uint32_t c = 0; c < g.sites; c += 64) {
     if (base + c >= g.V) break;
     uint64_t mask[3];   /* lanes whose xy, xz, yz face goes to the queue */
@@ -400,6 +416,7 @@ __global__ void __launch_bounds__(64) cross_kernel(CrossGeom g, const T *__restr
         const bool open = bulk && !one_sign(re[0], re[a], re[b], re[ab], g.k);
         if (__builtin_amdgcn_ballot_w64(open) && open)
           n = face_class(re[0], re[a], re[b], re[ab], im[0], im[a], im[b], im[ab], g.k);
+        if (n == 4) n = zero_face(base + c + lane, f) ? 0 : 3;   /* zero in FP32: exactly zero? */
         if (!WRITE) own += n == 3 ? 0 : n;
         some[f] = __builtin_amdgcn_ballot_w64(n != 0);
         mask[f] = WRITE ? some[f] : __builtin_amdgcn_ballot_w64(n == 3);

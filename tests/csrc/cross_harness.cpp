@@ -75,6 +75,17 @@ static Face draw(std::mt19937_64 &g, int kind) {
       f.i[c] = n(g);
     }
     f.r[(int)(4 * w(g)) & 3] = s * pow(10, -7 * w(g)) * (w(g) < 0.3 ? -1 : 1);
+  } else if (kind == 7) {                // zeros, NaNs, infinities, values FP32 does not hold
+    const double odd[6] = {0, -0.0, NAN, INFINITY, 1e-200, 1e200};
+    for (int c = 0; c < 4; ++c) {
+      f.r[c] = n(g);
+      f.i[c] = n(g);
+    }
+    const int every = (int)(g() % 3);    // one corner; all of Re phi; all of Im phi
+    const double v = odd[g() % 6], s = w(g) < 0.5 ? 1 : 1 + w(g);
+    if (every == 0) (g() & 1 ? f.r : f.i)[g() & 3] = v;
+    else
+      for (int c = 0; c < 4; ++c) (every == 1 ? f.r : f.i)[c] = v * (c & 1 ? s : 1);
   } else {                               // q's equation nearly linear
     const double t = pow(10, -1 - 12 * w(g));
     double B0 = n(g), C0 = n(g), D0 = n(g), k = n(g), p = w(g), q = w(g);
@@ -112,6 +123,8 @@ void check_faces(int kind, long long n, unsigned seed, int nx, int ny, int nz, d
       ++out[2];
     } else {
       got = ax::face_class(r[0], r[1], r[2], r[3], (float)f.i[0], (float)f.i[1], (float)f.i[2], (float)f.i[3], k);
+      auto zero = [](const double *v) { return v[0] == 0 && v[1] == 0 && v[2] == 0 && v[3] == 0; };
+      if (got == 4) got = zero(f.r) || zero(f.i) ? 0 : 3;
     }
     if (got == 3) {
       ++out[0];
