@@ -47,6 +47,7 @@ struct GlobalGeom {
   int nx, ny, nz;
   int periodic;          /* 1: all sites updated, periodic wrap; 0: Neumann x/y faces */
   uint32_t V, per;       /* sites; blocks per XCD */
+  uint32_t first;        /* first site stepped: Neumann x faces are left out, no XCD's share lies in them */
   FastDiv by_nz, by_ny;
 };
 
@@ -151,7 +152,7 @@ struct GlobalSite {
   int i, j, k;
   bool on;
   __device__ GlobalSite(const GlobalGeom &g, uint32_t run) {
-    const uint32_t at = (run * 256 + threadIdx.x) * W;
+    const uint32_t at = g.first + (run * 256 + threadIdx.x) * W;
     s = min(at, g.V - W);               /* every lane holds loadable sites */
     const uint32_t r = quotient(s, g.by_nz);
     i = (int)quotient(r, g.by_ny);
@@ -325,7 +326,9 @@ static GlobalPlan plan_of(const ax_params &p, size_t pitch) {
   g.periodic = p.boundary == AX_BC_PERIODIC;
   g.V = (uint32_t)p.nx * p.ny * p.nz;
   q.wide = p.nz % 2 == 0 && pitch % 2 == 0;
-  const uint32_t runs = (g.V + 255) / 256 / (q.wide ? 2 : 1) + 1;   /* of 256 threads */
+  g.first = g.periodic ? 0 : (uint32_t)p.ny * p.nz;
+  const uint32_t sites = g.V - 2 * g.first;
+  const uint32_t runs = (sites + 255) / 256 / (q.wide ? 2 : 1) + 1;   /* of 256 threads */
   g.per = (runs + 7) / 8;
   q.eruns = std::min(kEnergyRuns, (runs + 1023) / 1024);
   q.eper = ((runs + q.eruns - 1) / q.eruns + 7) / 8;
