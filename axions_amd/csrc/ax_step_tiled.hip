@@ -180,7 +180,9 @@ hipError_t launch_step_tiled_ah(const StepConsts &k, const Levels<R> &L, int xse
    * rows.  us per step with partial chunks at the row ends / across rows:
    * FP64 101^3 50 / 43, 200^3 290 / 245, 300^3 949 / 781, 201x201x51 90 / 76;
    * FP32 101^3 33 / 24, 200^3 162 / 121, 300^3 582 / 417 (those lattices'
-   * rows now keep to one XCD too) */
+   * rows now keep to one XCD too).  Whole chunks taken across rows lose: with
+   * 64-bit planes, FP64, whole / across 512^3 3.93 / 4.09 ms, 520x512x1024 7.76 /
+   * 8.08 (8 VGPRs spilled) */
   const bool flat = k.nz % 64 != 0;
 #define AX_AHK(P2, PL, BG, PF, FL)                                                                             \
   hipLaunchKernelGGL((ah_tiled_kernel<R, P2, PL, BG, PF, FL>), grid, block, 0, st, m, L, k.nx, k.ny, k.nz, g, k.ex, \
@@ -195,7 +197,8 @@ hipError_t launch_step_tiled_ah(const StepConsts &k, const Levels<R> &L, int xse
   if (pf) {
     if constexpr (sizeof(R) == 8) AX_AHL(false, true, false);
   } else if (big) {
-    AX_AHL(true, false, true);   /* its row offsets in the lane whatever nz: 168 VGPRs, else 199 */
+    if (flat) AX_AHL(true, false, true);
+    else AX_AHL(true, false, false);
   } else {
     if (flat) AX_AHL(false, false, true);
     else AX_AHL(false, false, false);

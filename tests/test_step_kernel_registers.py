@@ -1,9 +1,11 @@
 """The step kernels keep their vector registers (read from the metadata of the
 built library): none of the ensemble pool's, whose FP64 kernel took 1.25x the
 time with 18 of them in scratch memory, and none of the Moore model's, which
-took 1.5x on large planes with 30.  And the FP64 pool steps whole 64-site
+took 1.5x on large planes with 30, and none of the Abelian-Higgs FP64 kernels
+for whole chunks.  And the FP64 pool steps whole 64-site
 chunks and chunks across rows side by side to the bits of single lattices."""
 import os
+import re
 
 import numpy as np
 import pytest
@@ -26,9 +28,14 @@ def kernels():
     return out
 
 
-@pytest.mark.parametrize("kernel,variants", [("pool_step_kernel", 4), ("moore_tiled_kernel", 20)])
+# ah_tiled_kernel<double, ..., FLAT = false>: powers of two or not, plain or
+# not, by 64-bit planes, LDS prefetch or neither
+AH_WHOLE = r"ah_tiled_kernelId(Lb[01]E){4}Lb0EE"
+
+
+@pytest.mark.parametrize("kernel,variants", [("pool_step_kernel", 4), ("moore_tiled_kernel", 20), (AH_WHOLE, 12)])
 def test_step_kernels_do_not_spill(kernel, variants):
-    found = {n: k for n, k in kernels().items() if kernel in n}
+    found = {n: k for n, k in kernels().items() if re.search(kernel, n)}
     assert len(found) == variants, sorted(found)
     for name, k in found.items():
         assert k[".vgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0, name
