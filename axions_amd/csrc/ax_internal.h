@@ -24,12 +24,15 @@ namespace ax {
  * y edges, would sit on different XCDs.  So XCD x gets the x-th eighth of each
  * segment's chunks, a band of consecutive rows (512^3 FP64 reads 15.4 -> 12.9
  * GB per step, FP32 9.0 -> 6.1 GB); where the chunks are no multiple of 8 a
- * few of the workgroups find nothing to do.  Planes of fewer than 16 chunks
- * keep the natural order: their eighths would be one chunk or none, and whole
- * XCDs idle (us per step, eighths / natural: 4000x3x3, one chunk, AH FP64 53.7
- * / 12.2, Moore 88 / 18.6; 1000x10x10, two, 22.5 / 9.5 and 32.6 / 12.9;
- * 400x30x30, 15, 20.7 / 18.3 and 35.5 / 30.7; 50^3, 40, 9.4 / 9.6 and 11.9 /
- * 13.5; 101^3, 160, 41 / 48 and 69 / 74). */
+ * few of the workgroups find nothing to do.  Planes of fewer than 14 chunks
+ * take the natural order once the fullest XCD would get more than 128 waves,
+ * one for each of its SIMDs, while others idle (us per step, eighths / natural:
+ * 4000x3x3, one chunk, AH FP64 53.7 / 12.2, Moore 88 / 18.6; 1000x10x10, two,
+ * 22.5 / 9.5 and 32.6 / 12.9; 600x24x24, nine, 23.0 / 16.2 and 73 / 50;
+ * 150x4x4, one, 6.9 / 5.9 and 11.4 / 9.1).  With fewer waves one XCD's L2 counts
+ * for more (100x4x4 5.8 / 6.1 and 7.5 / 8.0; 43x28x29, 13 chunks, 7.0 / 7.6),
+ * and so it does on wider planes (43x43x22, 15, 6.9 / 7.5 and 8.3 / 9.7; 50^3,
+ * 40, 9.4 / 9.6 and 11.9 / 13.5; 101^3, 160, 41 / 48 and 69 / 74). */
 struct TileGrid {
   int nc;      /* chunks of a plane */
   int xseg;    /* x planes marched by one wave */
@@ -44,9 +47,10 @@ inline TileGrid make_tile_grid(int nx, int ny, int nz, int xseg) {
   g.xseg = (xseg <= 0 || xseg > nx) ? nx : xseg;
   g.nc = tile_chunks(ny, nz);
   const char *o = getenv("AX_TILE_ORDER");        /* "natural" for measurements */
-  const bool natural = (o && o[0] == 'n') || g.nc < 16;
-  g.per = natural ? 0 : (g.nc + 7) / 8;
-  g.work = (natural ? g.nc : 8 * g.per) * ((nx + g.xseg - 1) / g.xseg);
+  const int nseg = (nx + g.xseg - 1) / g.xseg, per = (g.nc + 7) / 8;
+  const bool natural = (o && o[0] == 'n') || (g.nc < 14 && (long long)per * nseg > 128);
+  g.per = natural ? 0 : per;
+  g.work = (natural ? g.nc : 8 * per) * nseg;
   return g;
 }
 

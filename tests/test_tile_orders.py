@@ -40,15 +40,20 @@ def test_partial_buffers_hold_either_order(shape, model, monkeypatch):
             assert items(nx, ny, nz, xs) <= room, (shape, made, launched)
 
 
-@pytest.mark.parametrize("shape", [(4000, 3, 3), (1000, 10, 10), (200, 20, 20), (400, 30, 30)])
-def test_narrow_planes_have_no_empty_workgroups(shape, monkeypatch):
-    """Planes of a few chunks: as many workgroups as chunks and segments, not
-    eight XCD shares of which most are empty."""
+@pytest.mark.parametrize("shape", [(4000, 3, 3), (1000, 10, 10), (200, 20, 20), (43, 28, 29), (600, 28, 29), (43, 43, 22)])
+def test_narrow_planes_keep_the_xcds_busy(shape, monkeypatch):
+    """No XCD gets more waves than its 128 SIMDs while others have far fewer,
+    and below that the chunks of a plane stay together, eighths to an XCD."""
     order(monkeypatch, "")
     nx, ny, nz = shape
     chunks = -(-ny * nz // 64)
-    for xs in (1, 4, 32):
-        assert lib._ZN2ax16fused_work_itemsEiiii(nx, ny, nz, xs) == chunks * -(-nx // xs)
+    for xs in (1, 2, 4, 32):
+        segments = -(-nx // xs)
+        work = lib._ZN2ax16fused_work_itemsEiiii(nx, ny, nz, xs)
+        fullest = -(-work // 8)    # workgroup w goes to XCD w mod 8
+        assert fullest <= max(128, 1.15 * chunks * segments / 8 + 1), (shape, xs)
+        if -(-chunks // 8) * segments <= 128:
+            assert work == 8 * -(-chunks // 8) * segments
 
 
 @pytest.mark.gpu
